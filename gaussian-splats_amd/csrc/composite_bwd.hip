@@ -33,6 +33,7 @@ struct CompositeBwdArgs {
   const float* pinv;
   const float* pcolor;
   const float* popacity;
+  const GsRecord* records;  // RECORDS kernels: gathered instead of the four above
   uint32_t max_id;  // last valid Gaussian index: every gathered id is clamped to it
   const int32_t* ids;
   const int64_t* ranges;
@@ -75,7 +76,10 @@ struct CompositeBwdArgs {
 // entry j of the batch), last batch first; each lane tests its entry's reach
 // of every band's active pixels.  MASKS: only the entries the forward's masks
 // mark (those that reached its active pixels) are gathered and tested.
-template <int TILE, bool ABS, int PIX, bool MASKS>
+// RECORDS: the projection's 48-byte records are gathered (three 16-byte loads
+// of one or two lines, as the forward does) instead of the op's four projected
+// outputs.
+template <int TILE, bool ABS, int PIX, bool MASKS, bool RECORDS>
 __device__ __forceinline__ void composite_bwd_tile(const CompositeBwdArgs& a, float4 (*chunk)[3],
                                                    int lane, int tile, int band0, int seg) {
   constexpr int NPIX = TILE * TILE;
@@ -223,7 +227,9 @@ __device__ __forceinline__ void composite_bwd_tile(const CompositeBwdArgs& a, fl
     uint32_t bands = 0;  // bit k: the Gaussian can reach an active pixel of band k
     if (valid && live_bands && ((walk >> lane) & 1u)) {
       gid = int(min(next_id, a.max_id));
-      const GsRecord rec = load_projected(a.pmean, a.pinv, a.pcolor, a.popacity, gid);
+      const GsRecord rec = RECORDS
+                               ? load_record(a.records, gid)
+                               : load_projected(a.pmean, a.pinv, a.pcolor, a.popacity, gid);
 #pragma unroll
       for (int k = 0; k < PIX; ++k) {
         if (((live_bands >> k) & 1u) && touches_rect(rec, bx0[k], bx1[k], by0[k], by1[k]))
@@ -348,7 +354,7 @@ __device__ __forceinline__ void composite_bwd_tile(const CompositeBwdArgs& a, fl
 // composites the whole tile and the others have no work.  Each kernel thus
 // composites every pixel of any plan exactly once, with one instance of the
 // walk (two would share one register allocation).
-template <int TILE, bool ABS, bool QUARTERS, bool MASKS>
+template <int TILE, bool ABS, bool QUARTERS, bool MASKS, bool RECORDS>
 __global__ __launch_bounds__(kCompositeWaves * 64) void composite_bwd_kernel(CompositeBwdArgs a) {
   constexpr int NPIX = TILE * TILE;
   constexpr int PIX_TILE = NPIX >= 64 ? NPIX / 64 : 1;
@@ -368,24 +374,33 @@ __global__ __launch_bounds__(kCompositeWaves * 64) void composite_bwd_kernel(Com
     static_assert(PIX_TILE >= kCompositeWaves, "quarters of 64-pixel bands");
     constexpr int QPIX = PIX_TILE / kCompositeWaves;
     if (kind == kItemQuarter) {
-      composite_bwd_tile<TILE, ABS, QPIX, MASKS>(a, chunk[wid], lane, tile, index * QPIX, -1);
+      composite_bwd_tile<TILE, ABS, QPIX, MASKS, RECORDS>(a, chunk[wid], lane, tile, index * QPIX, -1);
     } else if (kind == kItemTile || index == 0) {  // a segmented tile whole, by its first item
       for (int q = 0; q < kCompositeWaves; ++q)
-        composite_bwd_tile<TILE, ABS, QPIX, MASKS>(a, chunk[wid], lane, tile, q * QPIX, -1);
+        composite_bwd_tile<TILE, ABS, QPIX, MASKS, RECORDS>(a, chunk[wid], lane, tile, q * QPIX, -1);
     }
   } else {
     if (kind == kItemQuarter && index != 0) return;  // the tile whole, by its first quarter
-    composite_bwd_tile<TILE, ABS, PIX_TILE, MASKS>(a, chunk[wid], lane, tile, 0,
-                                                   kind == kItemSegment ? index : -1);
+    composite_bwd_tile<TILE, ABS, PIX_TILE, MASKS, RECORDS>(a, chunk[wid], lane, tile, 0,
+                                                            kind == kItemSegment ? index : -1);
   }
 }
 
 template <int TILE, bool QUARTERS, bool MASKS>
 void launch_masks(const CompositeBwdArgs& a, unsigned blocks, hipStream_t s) {
+  if constexpr (MASKS && TILE >= 16) {  // image calls (gs_composite_bwd_image)
+    if (a.records) {
+      launch_timed(composite_bwd_kernel<TILE, false, QUARTERS, true, true>, blocks,
+                   kCompositeWaves * 64, 0, s, a);
+      return;
+    }
+  }
   if (a.grad_abs)
-    launch_timed(composite_bwd_kernel<TILE, true, QUARTERS, MASKS>, blocks, kCompositeWaves * 64, 0, s, a);
+    launch_timed(composite_bwd_kernel<TILE, true, QUARTERS, MASKS, false>, blocks,
+                 kCompositeWaves * 64, 0, s, a);
   else
-    launch_timed(composite_bwd_kernel<TILE, false, QUARTERS, MASKS>, blocks, kCompositeWaves * 64, 0, s, a);
+    launch_timed(composite_bwd_kernel<TILE, false, QUARTERS, MASKS, false>, blocks,
+                 kCompositeWaves * 64, 0, s, a);
 }
 
 template <int TILE, bool QUARTERS>
@@ -412,18 +427,19 @@ void launch(const CompositeBwdArgs& a, hipStream_t s) {
 
 using namespace gs;
 
-extern "C" GS_API int gs_composite_bwd(const float* projected_mean,
-                                       const float* inverse_covariance,
-                                       const float* projected_color,
-                                       const float* projected_opacity, int64_t n,
-                                       const int32_t* gaussian_ids, const int64_t* ranges,
-                                       const float* grad_image, const float* final_transmittance,
-                                       const int32_t* n_contributors, const int32_t* tile_order,
-                                       gs_view view, float* grad_projected, float* grad_absolute,
-                                       const void* checkpoints, size_t checkpoint_bytes,
-                                       int64_t num_intersections, const uint64_t* hit_masks,
-                                       size_t hit_mask_bytes, void* stream) {
-  clear_error();
+namespace {
+
+// The compositing backward from the op's projected outputs or, with
+// `records`, from the projection's records (then the four outputs are null).
+int composite_bwd(const float* projected_mean, const float* inverse_covariance,
+                  const float* projected_color, const float* projected_opacity,
+                  const GsRecord* records, int64_t n, const int32_t* gaussian_ids,
+                  const int64_t* ranges, const float* grad_image,
+                  const float* final_transmittance, const int32_t* n_contributors,
+                  const int32_t* tile_order, gs_view view, float* grad_projected,
+                  float* grad_absolute, const void* checkpoints, size_t checkpoint_bytes,
+                  int64_t num_intersections, const uint64_t* hit_masks, size_t hit_mask_bytes,
+                  void* stream) {
   GS_TRY(check_view(view, true));
   GS_REQUIRE(view.rendering_mode == GS_MODE_GAUSSIAN, GS_ERR_UNSUPPORTED,
              "Backward gradients are only supported for Gaussian rendering.");
@@ -431,10 +447,12 @@ extern "C" GS_API int gs_composite_bwd(const float* projected_mean,
              GS_ERR_INVALID_ARGUMENT, "null pointer argument");
   GS_REQUIRE((reinterpret_cast<uintptr_t>(inverse_covariance) & 15u) == 0,
              GS_ERR_INVALID_ARGUMENT, "inverse_covariance must be 16-byte aligned");
+  GS_REQUIRE((reinterpret_cast<uintptr_t>(records) & 15u) == 0, GS_ERR_INVALID_ARGUMENT,
+             "records must be 16-byte aligned");
   GS_REQUIRE(n >= 0 && n <= (int64_t(1) << 31), GS_ERR_INVALID_ARGUMENT,
              "invalid Gaussian count %lld", (long long)n);
-  GS_REQUIRE(n == 0 || (projected_mean && inverse_covariance && projected_color &&
-                        projected_opacity),
+  GS_REQUIRE(n == 0 || records ||
+                 (projected_mean && inverse_covariance && projected_color && projected_opacity),
              GS_ERR_INVALID_ARGUMENT, "null pointer argument");
   CompositeBwdArgs a;
   a.max_id = uint32_t(n > 0 ? n - 1 : 0);
@@ -442,6 +460,7 @@ extern "C" GS_API int gs_composite_bwd(const float* projected_mean,
   a.pinv = inverse_covariance;
   a.pcolor = projected_color;
   a.popacity = projected_opacity;
+  a.records = records;
   a.ids = gaussian_ids;
   a.ranges = ranges;
   a.grad_image = grad_image;
@@ -504,4 +523,42 @@ extern "C" GS_API int gs_composite_bwd(const float* projected_mean,
     default: launch<32>(a, s); break;
   }
   return check_launch("composite_bwd");
+}
+
+}  // namespace
+
+extern "C" GS_API int gs_composite_bwd(const float* projected_mean,
+                                       const float* inverse_covariance,
+                                       const float* projected_color,
+                                       const float* projected_opacity, int64_t n,
+                                       const int32_t* gaussian_ids, const int64_t* ranges,
+                                       const float* grad_image, const float* final_transmittance,
+                                       const int32_t* n_contributors, const int32_t* tile_order,
+                                       gs_view view, float* grad_projected, float* grad_absolute,
+                                       const void* checkpoints, size_t checkpoint_bytes,
+                                       int64_t num_intersections, const uint64_t* hit_masks,
+                                       size_t hit_mask_bytes, void* stream) {
+  clear_error();
+  return composite_bwd(projected_mean, inverse_covariance, projected_color, projected_opacity,
+                       nullptr, n, gaussian_ids, ranges, grad_image, final_transmittance,
+                       n_contributors, tile_order, view, grad_projected, grad_absolute,
+                       checkpoints, checkpoint_bytes, num_intersections, hit_masks,
+                       hit_mask_bytes, stream);
+}
+
+extern "C" GS_API int gs_composite_bwd_image(
+    const void* records, int64_t n, const int32_t* gaussian_ids, const int64_t* ranges,
+    const float* grad_image, const float* final_transmittance, const int32_t* n_contributors,
+    const int32_t* tile_order, gs_view view, float* grad_projected, const void* checkpoints,
+    size_t checkpoint_bytes, int64_t num_intersections, const uint64_t* hit_masks,
+    size_t hit_mask_bytes, void* stream) {
+  clear_error();
+  GS_REQUIRE(view.tile_size >= 16, GS_ERR_UNSUPPORTED,
+             "image calls composite tiles of 16 or 32 pixels (got %d)", view.tile_size);
+  GS_REQUIRE(records && hit_masks, GS_ERR_INVALID_ARGUMENT, "null pointer argument");
+  return composite_bwd(nullptr, nullptr, nullptr, nullptr,
+                       static_cast<const GsRecord*>(records), n, gaussian_ids, ranges, grad_image,
+                       final_transmittance, n_contributors, tile_order, view, grad_projected,
+                       nullptr, checkpoints, checkpoint_bytes, num_intersections, hit_masks,
+                       hit_mask_bytes, stream);
 }

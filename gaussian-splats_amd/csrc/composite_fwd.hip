@@ -33,6 +33,7 @@ struct CompositeArgs {
   const int32_t* items;  // dispatch plan (gs_tile_order), or nullptr: tiles in index order
   int num_items;
   bool split_all;        // without a plan: every tile split into quarters
+  bool long_walk;        // the CKPT kernel (tiles of at most 16 pixels)
   int width, height, tile;  // per view
   int tiles_w, num_tiles;    // of the whole mosaic
   int view_tw, view_th, cols, views;  // tiles per view, mosaic layout (one view: cols = views = 1)
@@ -40,7 +41,7 @@ struct CompositeArgs {
   // A pixel stays active while (1 - T) < threshold, i.e. T > 1 - threshold.
   float t_active;
   float* image;
-  float* final_t;
+  float* final_t;      // both null when the caller wants the image alone
   int32_t* n_contrib;
   // Checkpoints of whole-tile walks for the backward (CheckpointLayout), or
   // null counter: none.
@@ -332,8 +333,10 @@ __device__ __forceinline__ void composite_tile(const CompositeArgs& a, float4 (*
       a.image[pix * 3 + 0] = cr[k];
       a.image[pix * 3 + 1] = cg[k];
       a.image[pix * 3 + 2] = cb[k];
-      a.final_t[pix] = T[k];
-      a.n_contrib[pix] = ncon[k];
+      if (a.final_t) {
+        a.final_t[pix] = T[k];
+        a.n_contrib[pix] = ncon[k];
+      }
     }
   }
   if (write_key) {
@@ -393,7 +396,8 @@ __global__ __launch_bounds__(kCompositeWaves * 64) void composite_fwd_kernel(Com
     }
   } else {
     composite_tile<TILE, ELLIPSOID, PIX_TILE, HITS, CKPT>(a, chunk[wid], chunk2[wid],
-                                                          ck_slots[wid], lane, tile, 0, CKPT, true);
+                                                          ck_slots[wid], lane, tile, 0,
+                                                          CKPT && a.ckpt_counter, true);
   }
 }
 
@@ -422,7 +426,7 @@ void launch(const CompositeArgs& a, bool ellipsoid, hipStream_t s) {
     if (a.split_all) return launch_items<TILE, true, false>(a, ellipsoid, s);
   }
   if constexpr (TILE <= 16) {
-    if (a.ckpt_counter) return launch_items<TILE, false, true>(a, ellipsoid, s);
+    if (a.long_walk) return launch_items<TILE, false, true>(a, ellipsoid, s);
   }
   launch_items<TILE, false, false>(a, ellipsoid, s);
 }
@@ -459,18 +463,17 @@ extern "C" GS_API size_t gs_composite_hit_mask_bytes(gs_view view, int64_t num_i
   return size_t(hit_mask_words(num_intersections, m.num_tiles(), view.tile_size)) * 8;
 }
 
-extern "C" GS_API int gs_composite(const void* records, int64_t num_records,
-                                   const int32_t* gaussian_ids, int64_t num_intersections,
-                                   const int64_t* ranges, const int32_t* tile_order, gs_view view,
-                                   float* image, float* final_transmittance,
-                                   int32_t* n_contributors, void* checkpoints,
-                                   size_t checkpoint_bytes, uint64_t* hit_masks,
-                                   size_t hit_mask_bytes, uint32_t* tile_keys,
-                                   size_t tile_keys_bytes, void* stream) {
-  clear_error();
+namespace {
+
+// `longest_list` (0: unknown) selects the long-list walk for a call without
+// checkpoints; with them it is selected anyway.
+int composite(const void* records, int64_t num_records, const int32_t* gaussian_ids,
+              int64_t num_intersections, int64_t longest_list, const int64_t* ranges,
+              const int32_t* tile_order, gs_view view, float* image, float* final_transmittance, int32_t* n_contributors,
+              void* checkpoints, size_t checkpoint_bytes, uint64_t* hit_masks,
+              size_t hit_mask_bytes, uint32_t* tile_keys, size_t tile_keys_bytes, void* stream) {
   GS_TRY(check_view(view, true));
-  GS_REQUIRE(ranges && image && final_transmittance && n_contributors, GS_ERR_INVALID_ARGUMENT,
-             "null pointer argument");
+  GS_REQUIRE(ranges && image, GS_ERR_INVALID_ARGUMENT, "null pointer argument");
   GS_REQUIRE(num_records >= 0 && num_records <= (int64_t(1) << 31), GS_ERR_INVALID_ARGUMENT,
              "invalid record count %lld", (long long)num_records);
   GS_REQUIRE(num_records == 0 || records, GS_ERR_INVALID_ARGUMENT, "null records");
@@ -549,6 +552,7 @@ extern "C" GS_API int gs_composite(const void* records, int64_t num_records,
     GS_TRY(check_launch("composite checkpoints"));
   }
   const bool ellipsoid = view.rendering_mode == GS_MODE_ELLIPSOID;
+  a.long_walk = a.ckpt_counter || (longest_list > kCheckpointMinList && num_records > 0);
   switch (view.tile_size) {
     case 4: launch<4>(a, ellipsoid, s); break;
     case 8: launch<8>(a, ellipsoid, s); break;
@@ -556,4 +560,36 @@ extern "C" GS_API int gs_composite(const void* records, int64_t num_records,
     default: launch<32>(a, ellipsoid, s); break;
   }
   return check_launch("composite");
+}
+
+}  // namespace
+
+extern "C" GS_API int gs_composite(const void* records, int64_t num_records,
+                                   const int32_t* gaussian_ids, int64_t num_intersections,
+                                   const int64_t* ranges, const int32_t* tile_order, gs_view view,
+                                   float* image, float* final_transmittance,
+                                   int32_t* n_contributors, void* checkpoints,
+                                   size_t checkpoint_bytes, uint64_t* hit_masks,
+                                   size_t hit_mask_bytes, uint32_t* tile_keys,
+                                   size_t tile_keys_bytes, void* stream) {
+  clear_error();
+  GS_TRY(check_view(view, true));
+  GS_REQUIRE(final_transmittance && n_contributors, GS_ERR_INVALID_ARGUMENT,
+             "null pointer argument");
+  return composite(records, num_records, gaussian_ids, num_intersections, 0, ranges, tile_order,
+                   view, image, final_transmittance, n_contributors, checkpoints,
+                   checkpoint_bytes, hit_masks, hit_mask_bytes, tile_keys, tile_keys_bytes,
+                   stream);
+}
+
+extern "C" GS_API int gs_composite_image(const void* records, int64_t num_records,
+                                         const int32_t* gaussian_ids, int64_t num_intersections,
+                                         int64_t longest_list, const int64_t* ranges,
+                                         const int32_t* tile_order, gs_view view, float* image,
+                                         void* stream) {
+  clear_error();
+  GS_REQUIRE(longest_list >= 0, GS_ERR_INVALID_ARGUMENT, "negative list length");
+  return composite(records, num_records, gaussian_ids, num_intersections, longest_list, ranges,
+                   tile_order, view, image, nullptr, nullptr, nullptr, 0, nullptr, 0, nullptr, 0,
+                   stream);
 }

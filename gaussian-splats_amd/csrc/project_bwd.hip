@@ -40,7 +40,10 @@ struct ProjectBwdArgs {
   int64_t view_stride;   // Gaussians between consecutive views' inputs (n for one view)
   bool accumulate;       // add to the gradient buffers instead of overwriting them
   const float* grad_in;  // [views, N, 9]
-  const int32_t* counts;  // [views, N]
+  // [views, N]: a view without intersections for a Gaussian holds `none`
+  // (0 in the op's counts, kNoRect in an image call's packed rectangles).
+  const int32_t* counts;
+  int32_t none;
   int64_t n;
   float eps;
   float* g_mean;
@@ -286,8 +289,8 @@ __global__ __launch_bounds__(kBlock) void project_bwd_kernel(ProjectBwdArgs a) {
   float gcoef[F];
 #pragma unroll
   for (int i = 0; i < F; ++i) gcoef[i] = 0.0f;
-  bool any = have && count0 != 0;
-  for (int v = 1; have && v < views; ++v) any |= a.counts[v * a.view_stride + gi] != 0;
+  bool any = have && count0 != a.none;
+  for (int v = 1; have && v < views; ++v) any |= a.counts[v * a.view_stride + gi] != a.none;
   double q[4] = {0.0, 0.0, 0.0, 0.0};
   double qnorm = 0.0;
   if (any) {
@@ -304,13 +307,13 @@ __global__ __launch_bounds__(kBlock) void project_bwd_kernel(ProjectBwdArgs a) {
     q[2] = qr.z / qn;
     q[3] = qr.w / qn;
     const double sd[3] = {exp(double(ls0)), exp(double(ls1)), exp(double(ls2))};
-    if (!MULTI) {  // count0 != 0 here
+    if (!MULTI) {  // the view has intersections here
       view_gradients<K>(a, a.cam[0], gi, gi, mx, myy, mz, q, sd, alpha0, coef, gmx, gmy, gmz, h,
                         gs3, gop, gcoef, gin0);
     } else {
       for (int v = 0; v < views; ++v) {
         const int64_t vi = v * a.view_stride + gi;
-        if (a.counts[vi] == 0) continue;  // zero gradient from this view (project_bwd.py:324-334)
+        if (a.counts[vi] == a.none) continue;  // zero gradient from this view (project_bwd.py:324-334)
         float gin[9];
 #pragma unroll
         for (int i = 0; i < 9; ++i) gin[i] = a.grad_in[vi * 9 + i];
@@ -383,8 +386,9 @@ int project_bwd_views(const float* mean, const float* rotation, const float* sca
                       const float* camera_rotations, const float* camera_translations,
                       const float* intrinsics, int views, gs_view view,
                       const float* /*inverse_covariance*/, const float* grad_projected,
-                      const int32_t* counts, float* grad_mean, float* grad_rotation,
-                      float* grad_scale, float* grad_opacity, float* grad_color, void* stream) {
+                      const int32_t* counts, int32_t none, float* grad_mean,
+                      float* grad_rotation, float* grad_scale, float* grad_opacity,
+                      float* grad_color, void* stream) {
   GS_REQUIRE(n >= 0, GS_ERR_INVALID_ARGUMENT, "negative Gaussian count");
   GS_REQUIRE(num_sh == 1 || num_sh == 4 || num_sh == 9 || num_sh == 16, GS_ERR_UNSUPPORTED,
              "SH degrees above 3 are not implemented (got %d coefficients)", num_sh);
@@ -432,6 +436,7 @@ int project_bwd_views(const float* mean, const float* rotation, const float* sca
     const int64_t off = int64_t(first) * n;
     a.grad_in = grad_projected + off * 9;
     a.counts = counts + off;
+    a.none = none;
     a.accumulate = first > 0;
     if (views == 1) {
       switch (num_sh) {
@@ -466,7 +471,7 @@ extern "C" GS_API int gs_project_bwd(const float* mean, const float* rotation, c
   clear_error();
   return project_bwd_views(mean, rotation, scale, opacity, color, n, num_sh, camera_rotation,
                            camera_translation, nullptr, 1, view, inverse_covariance,
-                           grad_projected, counts, grad_mean, grad_rotation, grad_scale,
+                           grad_projected, counts, 0, grad_mean, grad_rotation, grad_scale,
                            grad_opacity, grad_color, stream);
 }
 
@@ -480,6 +485,21 @@ extern "C" GS_API int gs_project_bwd_views(
   clear_error();
   return project_bwd_views(mean, rotation, scale, opacity, color, n, num_sh, camera_rotations,
                            camera_translations, intrinsics, mosaic_of(view).views, view,
-                           inverse_covariance, grad_projected, counts, grad_mean, grad_rotation,
-                           grad_scale, grad_opacity, grad_color, stream);
+                           inverse_covariance, grad_projected, counts, 0, grad_mean,
+                           grad_rotation, grad_scale, grad_opacity, grad_color, stream);
+}
+
+extern "C" GS_API int gs_project_bwd_image(
+    const float* mean, const float* rotation, const float* scale, const float* opacity,
+    const float* color, int64_t n, int32_t num_sh, const float* camera_rotations,
+    const float* camera_translations, const float* intrinsics, gs_view view,
+    const uint32_t* tile_rects, const float* grad_projected, float* grad_mean,
+    float* grad_rotation, float* grad_scale, float* grad_opacity, float* grad_color,
+    void* stream) {
+  clear_error();
+  return project_bwd_views(mean, rotation, scale, opacity, color, n, num_sh, camera_rotations,
+                           camera_translations, intrinsics, mosaic_of(view).views, view, nullptr,
+                           grad_projected, reinterpret_cast<const int32_t*>(tile_rects),
+                           int32_t(kNoRect), grad_mean, grad_rotation, grad_scale, grad_opacity,
+                           grad_color, stream);
 }

@@ -46,16 +46,38 @@ struct ProjectArgs {
   int ellipsoid;
   float ellipsoid_extent;  // sqrt(-2 log1p(-confidence))
   float ellipsoid_cutoff;  // -2 log1p(-confidence)
-  float* pmean;
-  float* pinv;
+  bool tight;            // rectangles of the visible ellipse only (tight_extent)
+  float* pmean;          // the op's outputs; null for an image call, which keeps
+  float* pinv;           //   them in the records only
   float* pcolor;
   float* popacity;
   int* bounds;           // optional with tile_rects
-  int* counts;
+  int* counts;           // null for an image call
   GsRecord* records;     // optional
   uint32_t* depth_keys;  // optional
   uint32_t* tile_rects;  // optional: packed rectangles (pack_rect) in mosaic tiles
 };
+
+// Half-width of the Gaussian along one axis, for calls that return only the
+// image (ProjectArgs::tight): `wide` is the reference's extent, 2 sqrt(ln 255
+// alpha) sigma in Gaussian mode, whose square is twice the largest quadratic
+// form `cut` at which alpha reaches 1/255, so every axis is sqrt(2) too long
+// and the rectangles hold about twice the tiles the Gaussian can change.  Here
+// the bounding box of {D <= reach}, half-width sqrt(reach var), never more than
+// `wide`.  It must hold every pixel whose D, as the compositing kernels
+// evaluate it in float32, stays within `cut`: at a point of true value D each
+// term of the form is at most D cond (cond = 1 / (1 - rho^2) = inv00 Sigma00),
+// so some five roundings of 2^-24 per term move the sum of the four by less
+// than 1.2e-6 cond D; reach adds 2e-6 cond, beside the margin touches_rect
+// uses.  Above cond = 1e5 (a bound of 0.2) the reference's extent is kept.
+// 1M Gaussians at 1080p: 21.7M -> 12.6M (tile, Gaussian) entries, the training
+// step 705 -> 663 us; 4M in a small cube: 3.58 -> 2.87 ms (both with the image
+// call's records-only outputs).
+__device__ __forceinline__ float tight_extent(float wide, float cut, float cond, float var) {
+  if (!(cond <= 1.0e5f)) return wide;
+  const float reach = (cut * (1.0f + 1e-3f) + 1e-3f) * (1.0f + 2e-6f * cond);
+  return fminf(wide, sqrtf(reach * var));
+}
 
 // The colour block of kProjectBlock Gaussians is staged through LDS with
 // coalesced 16-byte loads (sh::stage_block), then each thread reads its own
@@ -201,29 +223,39 @@ __global__ __launch_bounds__(kProjectBlock) void project_fwd_kernel(ProjectArgs 
     }
 
     // Rectangle of tiles touched by the extent ellipse (torch.py:233-252).
-    const float rx = extent * sqrtf(float(c00));
-    const float ry = extent * sqrtf(float(c11));
+    float rx = extent * sqrtf(float(c00));
+    float ry = extent * sqrtf(float(c11));
+    if (a.tight) {
+      const float cond = float(c00 * c11 * rdet);
+      rx = tight_extent(rx, cut, cond, float(c00));
+      ry = tight_extent(ry, cut, cond, float(c11));
+    }
     // fmaxf/fminf map a NaN extent (alpha0 < 1/255) to the empty rectangle [0, 0).
     const float bx0 = fminf(fmaxf(floorf((u - rx) / a.tile), 0.0f), a.tiles_w);
     const float bx1 = fminf(fmaxf(floorf((u + rx) / a.tile) + 1.0f, 0.0f), a.tiles_w);
     const float by0 = fminf(fmaxf(floorf((v - ry) / a.tile), 0.0f), a.tiles_h);
     const float by1 = fminf(fmaxf(floorf((v + ry) / a.tile) + 1.0f, 0.0f), a.tiles_h);
     const int x0 = int(bx0), x1 = int(bx1), y0 = int(by0), y1 = int(by1);
-    const bool visible = dc > a.near_plane && dc < a.far_plane;
+    // A Gaussian that reaches alpha 1/255 nowhere (cut < 0) is left out of an
+    // image call's lists; the op's lists keep the reference's rectangle.
+    const bool visible =
+        dc > a.near_plane && dc < a.far_plane && (!a.tight || cut >= 0.0f);
     const int count = visible ? (x1 - x0) * (y1 - y0) : 0;
 
-    a.pmean[vi * 3 + 0] = u;
-    a.pmean[vi * 3 + 1] = v;
-    a.pmean[vi * 3 + 2] = dc;
-    reinterpret_cast<float4*>(a.pinv)[vi] = make_float4(i00, i01, i01, i11);
-    a.pcolor[vi * 3 + 0] = rgb[0];
-    a.pcolor[vi * 3 + 1] = rgb[1];
-    a.pcolor[vi * 3 + 2] = rgb[2];
-    a.popacity[vi] = alpha0;
+    if (a.pmean) {
+      a.pmean[vi * 3 + 0] = u;
+      a.pmean[vi * 3 + 1] = v;
+      a.pmean[vi * 3 + 2] = dc;
+      reinterpret_cast<float4*>(a.pinv)[vi] = make_float4(i00, i01, i01, i11);
+      a.pcolor[vi * 3 + 0] = rgb[0];
+      a.pcolor[vi * 3 + 1] = rgb[1];
+      a.pcolor[vi * 3 + 2] = rgb[2];
+      a.popacity[vi] = alpha0;
+    }
     if (a.bounds)
       reinterpret_cast<int4*>(a.bounds)[vi] =
           make_int4(x0 + cam.tile_x, x1 + cam.tile_x, y0 + cam.tile_y, y1 + cam.tile_y);
-    a.counts[vi] = count;
+    if (a.counts) a.counts[vi] = count;
     if (a.tile_rects)
       a.tile_rects[vi] =
           count > 0 ? pack_rect(x0 + cam.tile_x, x1 - x0, y0 + cam.tile_y, y1 - y0) : kNoRect;
@@ -274,7 +306,7 @@ namespace {
 int project_views(const float* mean, const float* rotation, const float* scale,
                   const float* opacity, const float* color, int64_t n, int32_t num_sh,
                   const float* camera_rotations, const float* camera_translations,
-                  const float* intrinsics, int views, gs_view view, bool mosaic,
+                  const float* intrinsics, int views, gs_view view, bool mosaic, bool image_only,
                   float* projected_mean, float* inverse_covariance, float* projected_color,
                   float* projected_opacity, int32_t* bounds, int32_t* counts, void* records,
                   uint32_t* depth_keys, uint32_t* tile_rects, void* stream) {
@@ -284,10 +316,13 @@ int project_views(const float* mean, const float* rotation, const float* scale,
              "SH degrees above 3 are not implemented (got %d coefficients)", num_sh);
   if (n == 0) return GS_OK;
   GS_REQUIRE(mean && rotation && scale && opacity && color && camera_rotations &&
-                 camera_translations && projected_mean && inverse_covariance &&
-                 projected_color && projected_opacity && (bounds || tile_rects) && counts,
+                 camera_translations &&
+                 (image_only ? records && depth_keys && tile_rects
+                             : projected_mean && inverse_covariance && projected_color &&
+                                   projected_opacity && (bounds || tile_rects) && counts),
              GS_ERR_INVALID_ARGUMENT, "null pointer argument");
-  GS_REQUIRE(aligned16(rotation) && aligned16(color) && aligned16(inverse_covariance) &&
+  GS_REQUIRE(aligned16(rotation) && aligned16(color) &&
+                 (image_only || aligned16(inverse_covariance)) &&
                  (!bounds || aligned16(bounds)) && (!records || aligned16(records)),
              GS_ERR_INVALID_ARGUMENT,
              "rotation, color, inverse_covariance, bounds and records must be 16-byte aligned");
@@ -308,6 +343,7 @@ int project_views(const float* mean, const float* rotation, const float* scale,
   a.far_plane = view.far_plane;
   a.eps = view.covariance_epsilon;
   a.ellipsoid = view.rendering_mode == GS_MODE_ELLIPSOID;
+  a.tight = image_only;
   const double cutoff = -2.0 * std::log1p(-double(view.confidence));
   a.ellipsoid_cutoff = float(cutoff);
   a.ellipsoid_extent = float(std::sqrt(cutoff));
@@ -338,12 +374,12 @@ int project_views(const float* mean, const float* rotation, const float* scale,
       c.tile_y = mosaic ? (vw / m.cols) * m.th : 0;
     }
     const int64_t off = int64_t(first) * n;  // first output slot of this launch
-    a.pmean = projected_mean + off * 3;
-    a.pinv = inverse_covariance + off * 4;
-    a.pcolor = projected_color + off * 3;
-    a.popacity = projected_opacity + off;
+    a.pmean = image_only ? nullptr : projected_mean + off * 3;
+    a.pinv = image_only ? nullptr : inverse_covariance + off * 4;
+    a.pcolor = image_only ? nullptr : projected_color + off * 3;
+    a.popacity = image_only ? nullptr : projected_opacity + off;
     a.bounds = bounds ? bounds + off * 4 : nullptr;
-    a.counts = counts + off;
+    a.counts = counts ? counts + off : nullptr;
     a.tile_rects = tile_rects ? tile_rects + off : nullptr;
     a.records = records ? static_cast<GsRecord*>(records) + off : nullptr;
     a.depth_keys = depth_keys ? depth_keys + off : nullptr;
@@ -369,7 +405,7 @@ extern "C" GS_API int gs_project_and_count(
     void* stream) {
   clear_error();
   return project_views(mean, rotation, scale, opacity, color, n, num_sh, camera_rotation,
-                       camera_translation, nullptr, 1, view, false, projected_mean,
+                       camera_translation, nullptr, 1, view, false, false, projected_mean,
                        inverse_covariance, projected_color, projected_opacity, bounds, counts,
                        records, depth_keys, tile_rects, stream);
 }
@@ -383,9 +419,21 @@ extern "C" GS_API int gs_project_views(
     uint32_t* depth_keys, uint32_t* tile_rects, void* stream) {
   clear_error();
   return project_views(mean, rotation, scale, opacity, color, n, num_sh, camera_rotations,
-                       camera_translations, intrinsics, mosaic_of(view).views, view, true,
+                       camera_translations, intrinsics, mosaic_of(view).views, view, true, false,
                        projected_mean, inverse_covariance, projected_color, projected_opacity,
                        bounds, counts, records, depth_keys, tile_rects, stream);
+}
+
+extern "C" GS_API int gs_project_image(
+    const float* mean, const float* rotation, const float* scale, const float* opacity,
+    const float* color, int64_t n, int32_t num_sh, const float* camera_rotations,
+    const float* camera_translations, const float* intrinsics, gs_view view, void* records,
+    uint32_t* depth_keys, uint32_t* tile_rects, void* stream) {
+  clear_error();
+  return project_views(mean, rotation, scale, opacity, color, n, num_sh, camera_rotations,
+                       camera_translations, intrinsics, mosaic_of(view).views, view, true, true,
+                       nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, records, depth_keys,
+                       tile_rects, stream);
 }
 
 extern "C" GS_API int gs_pack_records(const float* projected_mean,

@@ -15,7 +15,7 @@ from pathlib import Path
 import torch
 
 LIB_PATH = Path(__file__).resolve().parents[2] / "_lib" / "libgs_raster.so"
-ABI_VERSION = 17
+ABI_VERSION = 18
 
 GS_OK = 0
 GS_ERR_INVALID_ARGUMENT = 1
@@ -231,6 +231,10 @@ _SIGNATURES = {
         c_int,
         [c_void_p] * 5 + [c_int64, c_int32, c_void_p, c_void_p, c_void_p, GsView] + [c_void_p] * 10,
     ),
+    "gs_project_image": (
+        c_int,
+        [c_void_p] * 5 + [c_int64, c_int32, c_void_p, c_void_p, c_void_p, GsView] + [c_void_p] * 4,
+    ),
     "gs_pack_records": (c_int, [c_void_p] * 4 + [c_int64, GsView, c_void_p, c_void_p]),
     "gs_scan_workspace_bytes": (c_size_t, [c_int64]),
     "gs_scan_counts": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_size_t, c_void_p]),
@@ -289,6 +293,16 @@ _SIGNATURES = {
         [c_void_p] * 4 + [c_int64] + [c_void_p] * 6
         + [GsView, c_void_p, c_void_p, c_void_p, c_size_t, c_int64, c_void_p, c_size_t, c_void_p],
     ),
+    "gs_composite_image": (
+        c_int,
+        [c_void_p, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_void_p, GsView, c_void_p,
+         c_void_p],
+    ),
+    "gs_composite_bwd_image": (
+        c_int,
+        [c_void_p, c_int64] + [c_void_p] * 6
+        + [GsView, c_void_p, c_void_p, c_size_t, c_int64, c_void_p, c_size_t, c_void_p],
+    ),
     "gs_device_errors": (c_int, [c_void_p, c_int32, c_void_p]),
     "gs_project_bwd": (
         c_int,
@@ -297,6 +311,10 @@ _SIGNATURES = {
     "gs_project_bwd_views": (
         c_int,
         [c_void_p] * 5 + [c_int64, c_int32, c_void_p, c_void_p, c_void_p, GsView] + [c_void_p] * 9,
+    ),
+    "gs_project_bwd_image": (
+        c_int,
+        [c_void_p] * 5 + [c_int64, c_int32, c_void_p, c_void_p, c_void_p, GsView] + [c_void_p] * 8,
     ),
     "gs_l1_loss_workspace_bytes": (c_size_t, [c_int64]),
     "gs_l1_loss_fwd": (

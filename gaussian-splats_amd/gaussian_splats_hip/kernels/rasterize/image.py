@@ -1,0 +1,256 @@
+"""Rendering calls that return only the image.
+
+``rasterize`` and ``rasterize_views`` return images; the op behind them
+(``torch.ops.gaussian_splats_hip.rasterize``) also returns the reference's
+projected Gaussians and sorted tile lists for the caller's tile size
+(src/gaussian_splats/kernels/rasterize/interface.py:17-244).  An eager call of
+the two functions does not go through the op: nothing but the pixels leaves it,
+so it is free in what it lists and in which tiles:
+
+* each Gaussian is listed for the tiles it can change (``gs_project_image``),
+  about half of the reference's rectangle;
+* the tiles are those the kernels do best at (``image_tile``), whatever tile
+  size the caller names;
+* the projection writes the compositing records alone, and both compositing
+  directions read them.
+
+A pixel's entries that blend are the same, in the same order, so images are
+those of the op (``tests/test_gpu_image.py``); gradients differ in the order of
+their sums.  Traced calls (``torch.compile``) use the registered op.
+"""
+
+from __future__ import annotations
+
+from ctypes import c_void_p
+
+import torch
+
+from . import _native as nat
+from .intersections import MAX_BUCKET_GAUSSIANS, MAX_BUCKET_TILES, bin_tiles, depth_key_range
+
+
+def mosaic_columns(views: int, tiles_w: int, tiles_h: int) -> int:
+    """Views per mosaic row: the most nearly square layout whose tile grid fits
+    ``MAX_BUCKET_TILES`` per axis (row/column bucketing), else the most nearly
+    square one."""
+    if views <= 1:
+        return 1
+    best, best_key = 1, None
+    for cols in range(1, views + 1):
+        rows = -(-views // cols)
+        w, h = cols * tiles_w, rows * tiles_h
+        fits = w <= MAX_BUCKET_TILES and h <= MAX_BUCKET_TILES
+        # Fitting layouts first, then the squarest, then the fewest empty slots.
+        key = (not fits, max(w, h), rows * cols - views)
+        if best_key is None or key < best_key:
+            best, best_key = cols, key
+    return best
+
+
+#: Tile sizes the op takes; any other goes to it, which refuses it.
+OP_TILES = (4, 8, 16, 32)
+
+
+def image_tile(asked: int, width: int, height: int, n: int, views: int = 1) -> int | None:
+    """Tile size of an image call for which the caller ``asked`` one the op
+    takes, or None when the op itself has to run: it refuses the size, or
+    row/column bucketing takes neither grid (the op's other binning then runs,
+    with the caller's tile size).  16 pixels: smaller tiles leave lanes of the compositing waves idle
+    and list a Gaussian many times over (200k Gaussians at 1080p, forward and
+    backward: 3.77 ms with the default tile size 4, 0.55 ms with 16); 32 where
+    the grid of 16-pixel tiles is larger than bucketing takes."""
+    if asked not in OP_TILES or width <= 0 or height <= 0 or views * n >= MAX_BUCKET_GAUSSIANS:
+        return None
+    for tile in (16, 32):
+        tw, th = nat.tiles(width, height, tile)
+        cols = mosaic_columns(views, tw, th)
+        if cols * tw <= MAX_BUCKET_TILES and -(-views // cols) * th <= MAX_BUCKET_TILES:
+            return tile
+    return None
+
+
+class ImageRequest:
+    """Everything but the Gaussians of an image call: the cameras in host
+    memory ([V, 9], [V, 3], [V, 4]), the view and the scalars."""
+
+    __slots__ = ("rotations", "translations", "intrinsics", "view", "views", "tiles", "near",
+                 "far", "gaussian")
+
+    def __init__(self, rotations, translations, intrinsics, width, height, tile, threshold, near,
+                 far, rendering_mode, confidence):
+        self.views = rotations.shape[0]
+        self.rotations = nat.host_floats(rotations, 9 * self.views, "camera_rotations")
+        self.translations = nat.host_floats(translations, 3 * self.views, "camera_translations")
+        self.intrinsics = nat.host_floats(intrinsics, 4 * self.views, "intrinsics")
+        tw, th = nat.tiles(width, height, tile)
+        cols = mosaic_columns(self.views, tw, th)
+        self.tiles = (cols * tw, -(-self.views // cols) * th)
+        self.near, self.far = near, far
+        self.gaussian = rendering_mode == "gaussian"
+        self.view = nat.make_view(
+            1.0, 1.0, 0.0, 0.0, width, height, tile, near, far, rendering_mode, confidence,
+            opacity_threshold=threshold, views=self.views, mosaic_cols=cols,
+        )
+
+    def cameras(self):
+        return (c_void_p(self.rotations.data_ptr()), c_void_p(self.translations.data_ptr()),
+                c_void_p(self.intrinsics.data_ptr()))
+
+
+class _Walk:
+    """What the forward keeps for its backward beside the saved tensors."""
+
+    __slots__ = ("view", "accumulator", "checkpoints", "hits", "order")
+
+
+def forward_image(params, request: ImageRequest, keep: bool, timer=None):
+    """Projects, bins and composites; returns ``(image [V, H, W, 3], saved,
+    walk)``, the last two None unless ``keep`` (a backward will follow)."""
+    mark = timer or (lambda name: None)
+    device = nat.require_gpu(*params)
+    mean, rotation, scale, opacity, color = (nat.prepare(t) for t in params)
+    if color.shape[1] > 16:
+        raise NotImplementedError(
+            f"SH degrees above 3 are not implemented. Got {color.shape[1]} coefficients."
+        )
+    lib, stream, ptr = nat.library(), nat.stream(device), nat.ptr
+    n, views = mean.shape[0], request.views
+    vn = views * n
+    view = nat.GsView.from_buffer_copy(request.view)  # active_tiles is set below
+    width, height = view.image_width, view.image_height
+    tiles_w, tiles_h = request.tiles
+
+    records = torch.empty((vn, 12), dtype=torch.float32, device=device)
+    depth_keys = torch.empty(vn, dtype=torch.int32, device=device)
+    tile_rects = torch.empty(vn, dtype=torch.int32, device=device)
+    mark("start")
+    nat.check(
+        nat.launch("project", lambda: lib.gs_project_image(
+            ptr(mean), ptr(rotation), ptr(scale), ptr(opacity), ptr(color), n, color.shape[1],
+            *request.cameras(), view, ptr(records), ptr(depth_keys), ptr(tile_rects), stream,
+        )),
+        "project_image",
+    )
+    mark("project")
+    backward = keep and request.gaussian
+    # The backward's [V N, 9] gradient accumulator, zeroed beside the depth sort.
+    accumulator = (torch.empty((vn, 9), dtype=torch.float32, device=device) if backward else None)
+    ids, ranges = bin_tiles(
+        depth_keys, None, None, tiles_w, tiles_h, timer=mark, tile_rects=tile_rects,
+        clear=accumulator, key_range=depth_key_range(request.near, request.far),
+    )
+    mark("sort")
+    view.active_tiles = nat.active_tiles(ranges)
+    longest = nat.longest_list(ranges)
+    num_tiles, total = tiles_w * tiles_h, ids.numel()
+    image = torch.empty((views, height, width, 3), dtype=torch.float32, device=device)
+    checkpoints = nat.checkpoint_buffer(view, total, longest, device)
+    # With long lists the longest walks start first (as composite does).
+    plan = (nat.dispatch_plan(view, num_tiles, device, ranges=ranges)
+            if checkpoints is not None else None)
+    if not backward:
+        nat.check(
+            nat.launch("composite", lambda: lib.gs_composite_image(
+                ptr(records), vn, ptr(ids), total, longest, ptr(ranges), ptr(plan), view,
+                ptr(image), stream,
+            )),
+            "composite_image",
+        )
+        mark("composite")
+        return image, None, None
+    final_transmittance = torch.empty((views, height, width), dtype=torch.float32, device=device)
+    n_contributors = torch.empty((views, height, width), dtype=torch.int32, device=device)
+    hits = nat.hit_mask_buffer(view, total, device)
+    keys = nat.workspace(lib.gs_tile_order_workspace_bytes(num_tiles), device)
+    nat.check(
+        nat.launch("composite", lambda: lib.gs_composite(
+            ptr(records), vn, ptr(ids), total, ptr(ranges), ptr(plan), view, ptr(image),
+            ptr(final_transmittance), ptr(n_contributors), ptr(checkpoints),
+            nat.buffer_bytes(checkpoints), ptr(hits), nat.buffer_bytes(hits), ptr(keys),
+            keys.numel(), stream,
+        )),
+        "composite",
+    )
+    mark("composite")
+    # The backward's dispatch plan, behind the forward on the stream.
+    walk = _Walk()
+    walk.order = torch.empty(lib.gs_tile_order_items(view, 1), dtype=torch.int32, device=device)
+    nat.check(
+        lib.gs_tile_order(ptr(ranges), ptr(n_contributors), view, ptr(walk.order), ptr(keys),
+                          keys.numel(), 1, stream),
+        "tile_order",
+    )
+    walk.view, walk.accumulator, walk.checkpoints, walk.hits = view, accumulator, checkpoints, hits
+    return image, (records, tile_rects, ids, ranges, final_transmittance, n_contributors), walk
+
+
+def _aligned(t: torch.Tensor) -> torch.Tensor:
+    return t if t.is_contiguous() and t.data_ptr() % 16 == 0 else t.clone(
+        memory_format=torch.contiguous_format)
+
+
+def backward_image(params, saved, walk: _Walk, request: ImageRequest, grad_image):
+    """Gradients of the five parameter tensors for the image gradient."""
+    params = tuple(_aligned(t) for t in params)
+    mean, color = params[0], params[4]
+    records, tile_rects, ids, ranges, final_transmittance, n_contributors = (
+        _aligned(t) for t in saved)
+    n, device = mean.shape[0], mean.device
+    if grad_image is None:
+        return tuple(torch.zeros_like(t) for t in params)
+    grad_image = _aligned(grad_image.float())
+    accumulator, walk.accumulator = walk.accumulator, None
+    if accumulator is None:  # a second backward through the same graph
+        accumulator = torch.zeros((records.shape[0], 9), dtype=torch.float32, device=device)
+    grads = tuple(torch.empty_like(t) for t in params)
+    if n == 0:
+        return grads
+    lib, stream, ptr = nat.library(), nat.stream(device), nat.ptr
+    nat.check(
+        nat.launch("composite_bwd", lambda: lib.gs_composite_bwd_image(
+            ptr(records), records.shape[0], ptr(ids), ptr(ranges), ptr(grad_image),
+            ptr(final_transmittance), ptr(n_contributors), ptr(walk.order), walk.view,
+            ptr(accumulator), ptr(walk.checkpoints), nat.buffer_bytes(walk.checkpoints),
+            ids.numel(), ptr(walk.hits), nat.buffer_bytes(walk.hits), stream,
+        )),
+        "composite_bwd_image",
+    )
+    nat.check(
+        nat.launch("project_bwd", lambda: lib.gs_project_bwd_image(
+            *(ptr(t) for t in params), n, color.shape[1], *request.cameras(), walk.view,
+            ptr(tile_rects), ptr(accumulator), *(ptr(g) for g in grads), stream,
+        )),
+        "project_bwd_image",
+    )
+    return grads
+
+
+class _RenderImage(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, mean, rotation, scale, opacity, color, request, timer):
+        params = (mean, rotation, scale, opacity, color)
+        image, saved, walk = forward_image(params, request, True, timer)
+        ctx.set_materialize_grads(False)
+        ctx.request, ctx.walk = request, walk
+        if saved is not None:
+            ctx.save_for_backward(*params, *saved)
+        return image
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, grad_image):
+        if ctx.walk is None:
+            raise AssertionError(
+                "Backward gradients are only supported for Gaussian rendering."
+            )
+        saved = ctx.saved_tensors
+        grads = backward_image(saved[:5], saved[5:], ctx.walk, ctx.request, grad_image)
+        return (*grads, None, None)
+
+
+def render_image(params, request: ImageRequest, timer=None) -> torch.Tensor:
+    """The [V, H, W, 3] images of ``request``'s cameras, differentiable with
+    respect to the five parameter tensors in Gaussian mode."""
+    if torch.is_grad_enabled() and any(t.requires_grad for t in params):
+        return _RenderImage.apply(*params, request, timer)
+    return forward_image(params, request, False, timer)[0]

@@ -16,6 +16,7 @@ import torch
 from ...timing import stage_timer
 from . import _native as nat
 from .composite import composite
+from .image import ImageRequest, image_tile, render_image
 from .intersections import (
     bin_gaussians,
     bin_tiles,
@@ -410,6 +411,17 @@ def rasterize(
     from ...splats.camera import host_extrinsics  # the splat API imports this module
 
     camera_rotation, camera_translation = host_extrinsics(camera)
+    if not torch.compiler.is_compiling():
+        tile = image_tile(tile_size, int(image_width), int(image_height), mean.shape[0])
+        if tile is not None:
+            request = ImageRequest(
+                camera_rotation[None], camera_translation[None],
+                torch.tensor([[float(fx), float(fy), float(cx), float(cy)]]), int(image_width),
+                int(image_height), tile, float(opacity_threshold), float(near), float(far),
+                rendering_mode, float(confidence),
+            )
+            return render_image((mean, rotation, scale, opacity, color), request,
+                                stage_timer())[0]
     return rasterize_outputs(
         mean,
         rotation,

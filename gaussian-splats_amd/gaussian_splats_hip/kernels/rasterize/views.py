@@ -31,7 +31,6 @@ import torch
 from ...timing import stage_timer
 from . import _native as nat
 from .intersections import (
-    MAX_BUCKET_TILES,
     bin_gaussians,
     bin_tiles,
     bucketing_fits,
@@ -39,30 +38,13 @@ from .intersections import (
     emit_tiles,
     sort_tiles,
 )
+from .image import ImageRequest, image_tile, mosaic_columns, render_image
 from .interface import _contiguous
 from .project import _check_tile
 
 if TYPE_CHECKING:
     from ...splats.camera import Camera
     from ...splats.splats import GaussianSplat
-
-
-def mosaic_columns(views: int, tiles_w: int, tiles_h: int) -> int:
-    """Views per mosaic row: the most nearly square layout whose tile grid fits
-    ``MAX_BUCKET_TILES`` per axis (row/column bucketing), else the most nearly
-    square one."""
-    if views <= 1:
-        return 1
-    best, best_key = 1, None
-    for cols in range(1, views + 1):
-        rows = -(-views // cols)
-        w, h = cols * tiles_w, rows * tiles_h
-        fits = w <= MAX_BUCKET_TILES and h <= MAX_BUCKET_TILES
-        # Fitting layouts first, then the squarest, then the fewest empty slots.
-        key = (not fits, max(w, h), rows * cols - views)
-        if best_key is None or key < best_key:
-            best, best_key = cols, key
-    return best
 
 
 def _mosaic_view(
@@ -516,6 +498,15 @@ def rasterize_views(
     params = (splats.mean, splats.rotation, splats.scale, splats.opacity, splats.color)
     if indices is not None:
         params = tuple(p[indices] for p in params)
+    if not torch.compiler.is_compiling():
+        tile = image_tile(tile_size, width, height, params[0].shape[0], len(cameras))
+        if tile is not None:
+            request = ImageRequest(
+                rotations, translations, intrinsics, width, height, tile,
+                float(opacity_threshold), float(near), float(far), rendering_mode,
+                float(confidence),
+            )
+            return render_image(params, request, stage_timer())
     return rasterize_views_outputs(
         *params,
         rotations,

@@ -42,7 +42,7 @@ extern "C" {
 
 #define GS_API __attribute__((visibility("default")))
 
-#define GS_ABI_VERSION 17
+#define GS_ABI_VERSION 18
 
 typedef enum gs_status {
   GS_OK = 0,
@@ -97,8 +97,8 @@ GS_API const char* gs_last_error(void);
  * kernel's duration per launch.  gs_arm_launch_events arms two hipEvent_t
  * (created beforehand; either may be null) for the calling thread's next
  * timed kernel: the main kernel of gs_project_and_count, gs_project_views,
- * gs_project_bwd, gs_project_bwd_views, gs_composite, gs_composite_bwd,
- * gs_ply_pack or gs_ply_unpack (the first one launched, for calls that
+ * gs_project_bwd, gs_project_bwd_views, gs_composite, gs_composite_bwd, their
+ * _image variants, gs_ply_pack or gs_ply_unpack (the first one launched, for calls that
  * launch several).
  * That launch carries the events (hipExtLaunchKernel), so they take the
  * kernel's own start and end timestamps; hipEventElapsedTime of the pair is
@@ -166,6 +166,20 @@ GS_API int gs_project_views(
     float* projected_mean, float* inverse_covariance, float* projected_color,
     float* projected_opacity, int32_t* bounds, int32_t* counts,
     void* records, uint32_t* depth_keys, uint32_t* tile_rects, void* stream);
+
+/* Projection of a call that returns only the image (no counterpart in the
+ * reference, whose op returns the lists too): records, depth_keys and
+ * tile_rects of gs_project_views (one camera: view.views 0 or 1), without the
+ * op's per-Gaussian outputs, and with each rectangle cut down to the bounding
+ * box of the pixels the Gaussian can change (alpha >= 1/255), about half the
+ * tiles of the reference's extent.  Gaussians that can change no pixel get
+ * 0xFFFFFFFF. */
+GS_API int gs_project_image(
+    const float* mean, const float* rotation, const float* scale,
+    const float* opacity, const float* color, int64_t n, int32_t num_sh,
+    const float* camera_rotations, const float* camera_translations,
+    const float* intrinsics, gs_view view, void* records, uint32_t* depth_keys,
+    uint32_t* tile_rects, void* stream);
 
 /* Packs the per-Gaussian compositing record from the op's projected outputs
  * (used when compositing is called stage-wise, as composite.py:110 is).
@@ -389,6 +403,16 @@ GS_API int gs_composite(
     size_t checkpoint_bytes, uint64_t* hit_masks, size_t hit_mask_bytes, uint32_t* tile_keys,
     size_t tile_keys_bytes, void* stream);
 
+/* gs_composite for a caller that wants the image alone: no transmittance,
+ * contributor counts or state for a backward.  longest_list: the longest of
+ * the lists (totals[3] of gs_bin_tiles_plan), or 0 when unknown; long lists
+ * take the walk of two batches per step that records checkpoints for
+ * gs_composite's caller. */
+GS_API int gs_composite_image(
+    const void* records, int64_t num_records, const int32_t* gaussian_ids,
+    int64_t num_intersections, int64_t longest_list, const int64_t* ranges,
+    const int32_t* tile_order, gs_view view, float* image, void* stream);
+
 /* Back-to-front compositing gradient, accumulated with atomics into
  * grad_projected[N,9] (zeroed by the caller), from the op's projected outputs
  * of n Gaussians (list ids clamped to [0, n), as in gs_composite).
@@ -416,6 +440,16 @@ GS_API int gs_composite_bwd(
     const float* grad_image, const float* final_transmittance,
     const int32_t* n_contributors, const int32_t* tile_order, gs_view view,
     float* grad_projected, float* grad_absolute, const void* checkpoints,
+    size_t checkpoint_bytes, int64_t num_intersections, const uint64_t* hit_masks,
+    size_t hit_mask_bytes, void* stream);
+
+/* gs_composite_bwd from the records of gs_project_image (n of them) instead
+ * of the op's projected outputs, for tiles of 16 and 32 pixels and with the
+ * forward's hit masks (both required). */
+GS_API int gs_composite_bwd_image(
+    const void* records, int64_t n, const int32_t* gaussian_ids, const int64_t* ranges,
+    const float* grad_image, const float* final_transmittance, const int32_t* n_contributors,
+    const int32_t* tile_order, gs_view view, float* grad_projected, const void* checkpoints,
     size_t checkpoint_bytes, int64_t num_intersections, const uint64_t* hit_masks,
     size_t hit_mask_bytes, void* stream);
 
@@ -448,6 +482,17 @@ GS_API int gs_project_bwd_views(
     const float* grad_projected, const int32_t* counts,
     float* grad_mean, float* grad_rotation, float* grad_scale,
     float* grad_opacity, float* grad_color, void* stream);
+
+/* gs_project_bwd_views for gs_project_image (one camera: view.views 0 or 1):
+ * the views without intersections of a Gaussian are those whose tile_rects
+ * [V, N] hold 0xFFFFFFFF, instead of a zero count. */
+GS_API int gs_project_bwd_image(
+    const float* mean, const float* rotation, const float* scale,
+    const float* opacity, const float* color, int64_t n, int32_t num_sh,
+    const float* camera_rotations, const float* camera_translations,
+    const float* intrinsics, gs_view view, const uint32_t* tile_rects,
+    const float* grad_projected, float* grad_mean, float* grad_rotation,
+    float* grad_scale, float* grad_opacity, float* grad_color, void* stream);
 
 /* Photometric L1 loss of the training step that consumes the image
  * (src/gaussian_splats/training/train.py:137-138, the torch expression

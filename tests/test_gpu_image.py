@@ -1,0 +1,181 @@
+"""Image calls (``rasterize`` / ``rasterize_views``, eager) against the op they
+no longer go through: the same pixels from tight rectangles and 16-pixel tiles,
+gradients equal up to the order of their sums."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from gaussian_splats_hip import scenes
+from gaussian_splats_hip.kernels.rasterize.image import image_tile
+from gaussian_splats_hip.kernels.rasterize.interface import rasterize_outputs
+from gaussian_splats_hip.kernels.rasterize.views import camera_tensors, rasterize_views_outputs
+from gaussian_splats_hip.splats import GaussianSplat, rasterize, rasterize_views
+from gaussian_splats_hip.splats.camera import host_extrinsics
+
+pytestmark = pytest.mark.gpu
+
+PARAMS = ("mean", "rotation", "scale", "opacity", "color")
+
+
+def _needles(n, size):
+    """Gaussians from 2 to ~e^7 times longer than wide, in every direction
+    (conditions of the 2-D covariance up to ~1e6, on both sides of the line
+    above which the reference's extent is kept)."""
+    scene = scenes.edge_case_scene(n=n, sh_degree=1, image_size=size, seed=5)
+    g = torch.Generator().manual_seed(9)
+    scene.scale[:, 1:] = scene.scale[:, :1] - 7 * torch.rand(n, 1, generator=g)
+    scene.scale[: n // 4, 0] += 3
+    return scene
+
+
+def _op(scene, params, cam, tile, mode):
+    r, t = host_extrinsics(cam)
+    (fx, fy), (cx, cy), (w, h) = cam.focal_length, cam.principal_point, cam.image_size
+    return rasterize_outputs(*params, r, t, float(fx), float(fy), float(cx), float(cy), w, h, tile,
+                             0.999, scene.near, scene.far, mode, 0.95)[0]
+
+
+def _same_gradients(a, b):
+    """Two sums of the same float32 terms in other orders: two runs of one path
+    (atomic adds) differ by up to 1e-5 of a gradient's norm; one entry missing
+    at one tile would show as 1e-3 or more in scenes of this size."""
+    for name, x, y in zip(PARAMS, a, b):
+        assert (x - y).norm() <= 1e-4 * y.norm(), name
+
+
+@pytest.mark.parametrize("mode", ["gaussian", "ellipsoid"])
+@pytest.mark.parametrize("tile", [4, 8, 16, 32])
+@pytest.mark.parametrize("kind,size", [("edge", (96, 80)), ("edge", (17, 1)), ("needle", (333, 207)),
+                                       ("cloud", (1111, 1043))])
+def test_image_equals_op(kind, size, tile, mode, device):
+    if kind == "needle":
+        scene = _needles(3000, size)
+    elif kind == "cloud":  # above 4096 tiles of 16 pixels: whole tiles per wave
+        scene = scenes.edge_case_scene(n=20000, sh_degree=0, image_size=size, seed=6)
+    else:
+        scene = scenes.edge_case_scene(n=1000, image_size=size)
+    scene = scene.to(device)
+    cam = scene.cameras[0]
+    splats = GaussianSplat.from_tensors(*scene.params())
+    leaves = [p.detach().clone().requires_grad_(True) for p in scene.params()]
+    image = rasterize(splats, cam, tile, near=scene.near, far=scene.far, rendering_mode=mode)
+    expected = _op(scene, leaves, cam, tile, mode)
+    if mode == "ellipsoid":
+        # A pixel within rounding of the ellipse's edge may lie outside the
+        # reference's rectangle for one tile size and inside for another.
+        same = (image == expected).all(-1).float().mean()
+        assert same > 0.9995
+        with pytest.raises(AssertionError):
+            image.sum().backward()
+        return
+    with torch.no_grad():
+        assert torch.equal(image, rasterize(splats, cam, tile, near=scene.near, far=scene.far))
+    if kind == "needle" and tile != 16:
+        # The walk's own overlap test evaluates a needle's form at the edges of
+        # a tile's rectangle, whose rounding depends on the tile: an entry of
+        # alpha at the cut, 1/255, may be skipped with one tile size and blended
+        # with another, in the op as here.  (Colours are below 2.)
+        differs = (image != expected).any(-1)
+        assert differs.float().mean() < 1e-3
+        assert (image - expected).abs().max() < 4 / 255
+        expected = _op(scene, leaves, cam, 16, mode)
+    assert torch.equal(image, expected)
+    weight = torch.linspace(-1, 1, image.numel(), device=device).reshape(image.shape)
+    (image * weight).sum().backward()
+    (expected * weight).sum().backward()
+    grads = [getattr(splats, n).grad for n in PARAMS]
+    if kind != "needle":
+        _same_gradients(grads, [p.grad for p in leaves])
+        return
+    # A needle's chain back through its covariance amplifies the rounding of
+    # the sums over pixels by the condition number: the differences are held to
+    # those between two of the op's own orders of the sums (tiles of 4 and 32
+    # pixels), whose largest may lie up to 8 times either way.
+    orders = []
+    for other in (4, 32):
+        again = [p.detach().clone().requires_grad_(True) for p in scene.params()]
+        (_op(scene, again, cam, other, mode) * weight).sum().backward()
+        orders.append([p.grad for p in again])
+    for name, x, y, a, b in zip(PARAMS, grads, (p.grad for p in leaves), *orders):
+        assert (x - y).norm() <= 8 * (a - b).norm() + 1e-6 * y.norm(), name
+
+
+def test_image_long_lists(device):
+    """Lists above 8192 entries: checkpointed walk with a backward, the same
+    walk without checkpoints for the image alone; a second backward through
+    one graph re-zeroes its accumulator."""
+    scene = scenes.config4(n=60000)
+    scene = scene.to(device)
+    cam = scene.cameras[0]
+    splats = GaussianSplat.from_tensors(*scene.params())
+    leaves = [p.detach().clone().requires_grad_(True) for p in scene.params()]
+    image = rasterize(splats, cam, 16)
+    expected = _op(scene, leaves, cam, 16, "gaussian")
+    # Checkpoints cut a pixel's colour into partial sums at list positions, and
+    # the lists differ: up to 64 roundings of a sum below 4.
+    assert (image - expected).abs().max() < 64 * 4 * 2.0 ** -24
+    with torch.no_grad():
+        assert (image - rasterize(splats, cam, 16)).abs().max() < 64 * 4 * 2.0 ** -24
+    loss = (image - scene.target).square().mean()
+    first = torch.autograd.grad(loss, [getattr(splats, n) for n in PARAMS], retain_graph=True)
+    second = torch.autograd.grad(loss, [getattr(splats, n) for n in PARAMS])
+    want = torch.autograd.grad((expected - scene.target).square().mean(), leaves)
+    _same_gradients(first, want)
+    _same_gradients(second, want)
+
+
+def test_views_image_equals_op(device):
+    scene = scenes.config5(seed=2, n=4000, views=5, size=90, focal=110).to(device)
+    splats = GaussianSplat.from_tensors(*scene.params())
+    leaves = [p.detach().clone().requires_grad_(True) for p in scene.params()]
+    images = rasterize_views(splats, scene.cameras, tile_size=8)
+    r, t, k, w, h = camera_tensors(scene.cameras)
+    expected = rasterize_views_outputs(*leaves, r, t, k, w, h, 8, 0.999, 0.2, 100.0, "gaussian",
+                                       0.95)[0]
+    assert torch.equal(images, expected)
+    (images - scene.target).abs().mean().backward()
+    (expected - scene.target).abs().mean().backward()
+    _same_gradients([getattr(splats, n).grad for n in PARAMS], [p.grad for p in leaves])
+
+
+def test_no_gaussians_and_nothing_visible(device):
+    scene = scenes.edge_case_scene(n=40, image_size=(50, 30)).to(device)
+    cam = scene.cameras[0]
+    for params in (tuple(p[:0] for p in scene.params()),
+                   (scene.mean * torch.tensor([1.0, 1.0, -1.0], device=device), *scene.params()[1:])):
+        splats = GaussianSplat.from_tensors(*params)
+        image = rasterize(splats, cam, near=scene.near, far=scene.far)
+        assert image.shape == (30, 50, 3) and not image.any()
+        image.sum().backward()
+        assert all(not getattr(splats, n).grad.any() for n in PARAMS)
+
+
+def test_saved_tensor_hooks(device):
+    """The forward's tensors go through saved-tensor hooks (here to the host
+    and back) like any autograd function's."""
+    scene = scenes.edge_case_scene(n=500, image_size=(64, 48)).to(device)
+    cam = scene.cameras[0]
+    grads = []
+    for hooked in (False, True):
+        splats = GaussianSplat.from_tensors(*(p.clone() for p in scene.params()))
+        if hooked:
+            with torch.autograd.graph.save_on_cpu():
+                image = rasterize(splats, cam, near=scene.near, far=scene.far)
+        else:
+            image = rasterize(splats, cam, near=scene.near, far=scene.far)
+        image.square().sum().backward()
+        grads.append([getattr(splats, n).grad for n in PARAMS])
+    _same_gradients(*grads)
+
+
+def test_image_tile_rule():
+    assert image_tile(4, 1920, 1080, 10) == 16
+    assert image_tile(32, 4096, 4096, 10) == 16
+    assert image_tile(4, 4097, 16, 10) == 32
+    assert image_tile(4, 8193, 16, 10) is None
+    assert image_tile(64, 640, 480, 10) is None
+    assert image_tile(8, 800, 800, 10, views=16) == 16
+    assert image_tile(8, 1000, 1000, 10, views=25) == 32
+    assert image_tile(16, 640, 480, 1 << 26) is None
