@@ -14,14 +14,14 @@
 // g . S_{i-1} = alpha_i (g . c_i) + (1 - alpha_i) g . S_i.
 //
 // Per Gaussian, each lane sums over its pixels (which share one column, so one
-// dx) q = dL/dalpha * G, q dy, q dy^2 and g T alpha, folds them into the nine
+// dx) q = o dL/dalpha * G, q dy, q dy^2 and g T alpha, folds them into the nine
 // per-lane partial gradients
-//   (u, v, inv00, inv01, inv11, r, g, b, opacity) += (-2 k (a Sx + b Sy),
-//   -2 k (b Sx + c Sy), k Sxx, k Sxy, k Syy, Sr, Sg, Sb, Sq),  k = -o / 2,
+//   (u, v, inv00, inv01, inv11, r, g, b, opacity) += (a Sx + b Sy, b Sx + c Sy,
+//   k Sxx, k Sxy, k Syy, Sr, Sg, Sb, Sq / o),  k = -1/2,
 // and the wave sums them with a transposing permlane/DPP reduction that leaves
-// them in four rows of three registers; two fp32 atomic adds (four and five
-// lanes) write them, once per (tile, Gaussian).  Replaces composite_bwd.py:47-204 and the
-// index_add_ scatter of composite_bwd.py:268-273.
+// them in one register, written by one nine-lane fp32 atomic add per (tile,
+// Gaussian).  Replaces composite_bwd.py:47-204 and the index_add_ scatter of
+// composite_bwd.py:268-273.
 #include "common.h"
 #include "raster_math.h"
 
@@ -168,12 +168,13 @@ __device__ __forceinline__ void composite_bwd_tile(const CompositeBwdArgs& a, fl
     if (lo >= hi) return;
   }
 
-  // Gradient fields written by this lane's two atomics: lane 16 r writes the
-  // row-r fields of t0 and t1 of the nine-way sum, lane 1 the opacity total t2.
-  const int field = sum9_field(lane >> 4);
-  const bool row_writer = (lane & 15) == 0;
-  const bool second_writer = row_writer || lane == 1;
-  const int second_field = row_writer ? 4 + field : 8;
+  // Gradient field written by this lane's atomic (wave_sum9's layout): lanes
+  // 0 and 8 of row r write its two fields, lane 4 the opacity's.  The lane's
+  // total is scaled to the gradient's units on the way (see `fold`).
+  const int column = lane & 15;
+  const bool writer = column == 0 || column == 8 || lane == 4;
+  const int field = lane == 4 ? 8 : (column == 8 ? 4 : 0) + sum9_field(lane >> 4);
+  const float unit = field < 2 ? 1.0f / kNegHalfLog2e : field < 5 ? -0.5f : 1.0f;
 
   // Each batch's ids are requested one batch ahead, once the current batch
   // is in LDS, so a batch waits on one dependent load (the gather), not two.
@@ -225,6 +226,7 @@ __device__ __forceinline__ void composite_bwd_tile(const CompositeBwdArgs& a, fl
     LaneSplat mine;
     int gid = 0;
     uint32_t bands = 0;  // bit k: the Gaussian can reach an active pixel of band k
+    float inverse_opacity = 0.0f;
     if (valid && live_bands && ((walk >> lane) & 1u)) {
       gid = int(min(next_id, a.max_id));
       const GsRecord rec = RECORDS
@@ -236,10 +238,11 @@ __device__ __forceinline__ void composite_bwd_tile(const CompositeBwdArgs& a, fl
           bands |= 1u << k;
       }
       mine = lane_splat(rec);
+      inverse_opacity = 1.0f / rec.opacity;
     }
     chunk[lane][0] = make_float4(mine.u, mine.v, mine.o, mine.pa);
     chunk[lane][1] = make_float4(mine.pb, mine.pc, mine.r, mine.g);
-    chunk[lane][2] = make_float4(mine.b, mine.oa, mine.ob, mine.oc);
+    chunk[lane][2] = make_float4(mine.b, 0.5f * mine.pb, inverse_opacity, 0.0f);
     next_id = bt - 1 >= b_lo ? uint32_t(a.ids[start + (bt - 1) * 64 + lane]) : 0u;
     if constexpr (MASKS) load_masks(bt - 1);
     uint64_t mask = __ballot(bands != 0);
@@ -259,85 +262,88 @@ __device__ __forceinline__ void composite_bwd_tile(const CompositeBwdArgs& a, fl
       s.r = f1.z;
       s.g = f1.w;
       s.bl = f2.x;
+      const float half_pb = f2.y;
       const int pos = pos0 + j;
       const ColumnTerms c = column_terms(s, pxf);
       // Per-lane sums over the lane's pixels; -0 is the identity of +, so the
       // first term needs no add.
-      float s0 = -0.0f, s1 = -0.0f, s2 = -0.0f;  // sum q, q dy, q dy^2
+      float s0 = -0.0f, s1 = -0.0f, s2 = -0.0f;  // sum o q, o q dy, o q dy^2
       float sr = -0.0f, sg = -0.0f, sb = -0.0f;
-      float ax = -0.0f, ay = -0.0f;  // ABS: sum |q (oa dx + ob dy)|, |q (ob dx + oc dy)|
-      const float oa = f2.y, ob = f2.z, oc = f2.w;
-      const float oadx = oa * c.dx, obdx = ob * c.dx;
-      bool touched = false;
+      float ax = -0.0f, ay = -0.0f;  // ABS: sums of |mean gradient terms| / |kNegHalfLog2e|
+      const float padx = s.pa * c.dx, hbdx = half_pb * c.dx;
+      uint64_t touched = 0;
       // Branch-free: an entry a pixel did not process while active, or whose
       // alpha is cut to 0, runs with alpha = 0, which leaves T, g.S and every
-      // sum unchanged.
+      // sum unchanged.  29 VALU instructions per band.
 #pragma unroll
       for (int k = 0; k < PIX; ++k) {
-        // A band of 64 pixels that the Gaussian cannot reach, or none of
-        // which processed this entry, is skipped.
-        if (!((band_mask >> k) & 1u) || __ballot(pos < ncon[k]) == 0) continue;
+        // A band of 64 pixels that the Gaussian cannot reach, or none of which
+        // processed this entry, is skipped.
+        const uint64_t active = ballot_of(pos < ncon[k]);
+        if (!((band_mask >> k) & 1u) || active == 0) continue;
         const float dy = pyf[k] - s.v;
-        float prob;
-        const float raw = raw_alpha<false>(s, c, dy, prob);
-        const float clamped = fminf(raw, kMaxAlpha);
-        const bool hit = pos < ncon[k] && clamped >= kMinAlpha;
-        const float alpha = hit ? clamped : 0.0f;
+        float raw;
+        const float a0 = entry_alpha<false>(s, c, dy, raw);
+        const uint64_t hit = ballot_of(a0 >= kMinAlpha) & active;
+        const float alpha = in_mask(hit) ? a0 : 0.0f;
         touched |= hit;
-        // T before the entry = T after it / (1 - alpha), with 1 / (1 - alpha)
-        // formed as 1 + alpha / (1 - alpha): v_rcp_f32's error (up to an ulp,
-        // of one sign) then enters scaled by alpha, so walking back through
-        // thousands of small-alpha entries does not accumulate it (with the
-        // plain reciprocal: ~2e-4 relative after 1600 entries).  alpha = 0
-        // gives exactly 1.
-        const float t_before = T[k] * fmaf(alpha, __builtin_amdgcn_rcpf(1.0f - alpha), 1.0f);
-        const float w = t_before * alpha;
+        // T before the entry = T after it / (1 - alpha) = T + w with
+        // w = T alpha / (1 - alpha): v_rcp_f32's error (up to an ulp, of one
+        // sign) then enters scaled by alpha, so walking back through thousands
+        // of small-alpha entries does not accumulate it (with the plain
+        // reciprocal: ~2e-4 relative after 1600 entries).  alpha = 0 gives
+        // exactly T.
+        const float w = T[k] * (alpha * __builtin_amdgcn_rcpf(1.0f - alpha));
+        T[k] += w;
         sr += gr[k] * w;
         sg += gg[k] * w;
         sb += gb[k] * w;
         const float gc = gr[k] * s.r + gg[k] * s.g + gb[k] * s.bl;
         const float diff = gc - gs_[k];
         gs_[k] += alpha * diff;
-        T[k] = t_before;
-        // dL/dalpha * G where alpha is neither cut nor clamped (alpha == raw
-        // holds exactly then, and never for a cut or clamped alpha with G > 0).
-        const float q = alpha == raw ? t_before * diff * prob : 0.0f;
+        // o times dL/dalpha * G = w diff where alpha is not clamped (a cut
+        // alpha has w = 0).
+        const float q = raw <= kMaxAlpha ? w * diff : 0.0f;
         const float qy = q * dy;
         s0 += q;
         s1 += qy;
         s2 += qy * dy;
         if constexpr (ABS) {
-          ax += fabsf(q * fmaf(ob, dy, oadx));
-          ay += fabsf(q * fmaf(oc, dy, obdx));
+          ax += fabsf(q * fmaf(half_pb, dy, padx));
+          ay += fabsf(q * fmaf(s.pc, dy, hbdx));
         }
       }
-      if (__ballot(touched) == 0) continue;
-      // d alpha / d(u, v, conic) folded per lane before the reduction
-      // (k = -o/2, -2k = o):  u: o (a Sx + b Sy),  v: o (b Sx + c Sy),
-      // inv00: k Sxx,  inv01: k Sxy,  inv11: k Syy,  Sx = dx s0, Sxx = dx^2 s0,
-      // Sxy = dx s1, Sy = s1, Syy = s2.
+      if (touched == 0) continue;
+      // d alpha / d(u, v, conic, opacity) folded per lane before the reduction,
+      // up to the lanes' `unit` (and 1 / o for the opacity), with the sums
+      // already holding o:  u: a Sx + b Sy,  v: b Sx + c Sy,  inv00: -Sxx / 2,
+      // inv01: -Sxy / 2,  inv11: -Syy / 2,  Sx = dx s0, Sxx = dx^2 s0,
+      // Sxy = dx s1, Sy = s1, Syy = s2, and (a, b, c) = (pa, pb / 2, pc) unit.
       const float sx = c.dx * s0;
-      const float kdx = (-0.5f * s.o) * c.dx;
       float v[9];
-      v[0] = oa * sx + ob * s1;
-      v[1] = ob * sx + oc * s1;
-      v[2] = kdx * sx;
-      v[3] = kdx * s1;
-      v[4] = (-0.5f * s.o) * s2;
+      v[0] = s.pa * sx + half_pb * s1;
+      v[1] = half_pb * sx + s.pc * s1;
+      v[2] = c.dx * sx;
+      v[3] = c.dx * s1;
+      v[4] = s2;
       v[5] = sr;
       v[6] = sg;
       v[7] = sb;
       v[8] = s0;
-      float t0, t1, t2;
-      wave_sum9(v, t0, t1, t2);
+      const float total = wave_sum9(v) * (lane == 4 ? f2.z : unit);
+      // One instruction for the nine fields: its lanes' 36 bytes leave the L2
+      // as one atomic request (two for a row across a line).  Device-scope
+      // atomics are executed in memory, about 9 requests per ns over the whole
+      // chip, a bound of this kernel beside its VALU issue.  With two
+      // instructions per entry 300k Gaussians at 1237 x 822, whose tiles are
+      // walked in quarters, sent 3.4M requests in 336 us, with one 2.1M in 218.
       float* dst = a.grad + int64_t(__builtin_amdgcn_readlane(gid, j)) * 9;
-      if (row_writer) unsafeAtomicAdd(dst + field, t0);
-      if (second_writer) unsafeAtomicAdd(dst + second_field, row_writer ? t1 : t2);
+      if (writer) unsafeAtomicAdd(dst + field, total);
       if constexpr (ABS) {
         // Lanes 0-31 fold |du| terms, 32-63 |dv| terms; then every lane of
         // rows 0-1 holds the |du| total and of rows 2-3 the |dv| total.
         const float h = fold_halves(ax, ay);
-        const float tabs = row_sum(fold_rows(h, h));
+        const float tabs = row_sum(fold_rows(h, h)) * (-1.0f / kNegHalfLog2e);
         if ((lane & 31) == 0)
           unsafeAtomicAdd(a.grad_abs + int64_t(__builtin_amdgcn_readlane(gid, j)) * 2 + (lane >> 5),
                           tabs);

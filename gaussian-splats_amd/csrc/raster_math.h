@@ -12,17 +12,19 @@ constexpr float kMinAlpha = 1.0f / 255.0f;  // torch.py:350, composite.py:82
 constexpr float kMaxAlpha = 0.99f;          // torch.py:349, composite.py:81
 constexpr float kNegHalfLog2e = -0.72134752044448170f;  // -0.5 / ln 2
 
-// Gaussian broadcast to every lane of a wave (values live in SGPRs).  The
-// conic is pre-scaled so that exp(-D/2) = exp2(pa dx^2 + pb dx dy + pc dy^2)
-// with D the quadratic form a dx^2 + 2 b dx dy + c dy^2 of utils.py:78-87.
+// One list entry as a wave reads it back from LDS (a broadcast).  The conic is
+// scaled so that exp(-D / 2) = exp2(pa dx^2 + pb dx dy + pc dy^2) with D the
+// quadratic form a dx^2 + 2 b dx dy + c dy^2 of utils.py:78-87.  (The opacity
+// stays a factor: as log2 o in the exponent it would save a multiplication,
+// but the exponent, near -8 at the 1/255 cut, then rounds more coarsely and
+// more entries fall on the other side of the cut.)
 struct Splat {
   float u, v, o, pa, pb, pc, cut, r, g, bl;
 };
 
-// Per-lane view of a gathered record with the pre-scaled conic.
+// Per-lane view of a gathered record in those units.
 struct LaneSplat {
   float u, v, o, pa, pb, pc, cut, r, g, b;
-  float oa, ob, oc;  // opacity times the unscaled inverse covariance (mean gradient)
 };
 
 __device__ __forceinline__ LaneSplat lane_splat(const GsRecord& r) {
@@ -37,9 +39,6 @@ __device__ __forceinline__ LaneSplat lane_splat(const GsRecord& r) {
   s.r = r.r;
   s.g = r.g;
   s.b = r.b;
-  s.oa = r.opacity * r.inv00;
-  s.ob = r.opacity * r.inv01;
-  s.oc = r.opacity * r.inv11;
   return s;
 }
 
@@ -61,29 +60,26 @@ __device__ __forceinline__ ColumnTerms column_terms(const Splat& s, float px) {
   return c;
 }
 
-__device__ __forceinline__ float falloff_log2(const ColumnTerms& c, float pc, float dy) {
-  return fmaf(dy, fmaf(pc, dy, c.p1), c.p0);
-}
-
-// Unclamped alpha = opacity * probability (utils.py:90-99); `prob` returns the
-// probability.  Ellipsoid mode compares D = power / (-0.5 log2 e) with the
-// cutoff stored in the record.
+// Alpha of torch.py:349-350 before the 1/255 cut: min(o exp(-D / 2), 0.99), or
+// in ellipsoid mode min(o, 0.99) inside the cutoff and 0 outside.  `raw`
+// returns the value before the ceiling.
 template <bool ELLIPSOID>
-__device__ __forceinline__ float raw_alpha(const Splat& s, const ColumnTerms& c, float dy,
-                                           float& prob) {
-  const float power = falloff_log2(c, s.pc, dy);
-  if constexpr (ELLIPSOID) {
-    prob = power >= kNegHalfLog2e * s.cut ? 1.0f : 0.0f;
-  } else {
-    prob = __builtin_amdgcn_exp2f(power);
-  }
-  return s.o * prob;
+__device__ __forceinline__ float entry_alpha(const Splat& s, const ColumnTerms& c, float dy,
+                                             float& raw) {
+  const float power = fmaf(dy, fmaf(s.pc, dy, c.p1), c.p0);
+  if constexpr (ELLIPSOID)
+    raw = power >= kNegHalfLog2e * s.cut ? s.o : 0.0f;
+  else
+    raw = s.o * __builtin_amdgcn_exp2f(power);
+  return fminf(raw, kMaxAlpha);
 }
 
-// Clamp to 0.99 and drop alphas below 1/255 (torch.py:349-350).
-__device__ __forceinline__ float blend_alpha(float raw) {
-  const float a = fminf(raw, kMaxAlpha);
-  return a >= kMinAlpha ? a : 0.0f;
+// Lane masks in scalar registers: ballot_of gives a predicate's mask (one
+// comparison writes it directly), in_mask turns a mask back into a predicate (a
+// select reads it directly), so that masks combine with scalar instructions.
+__device__ __forceinline__ uint64_t ballot_of(bool p) { return __builtin_amdgcn_ballot_w64(p); }
+__device__ __forceinline__ bool in_mask(uint64_t m) {
+  return __builtin_amdgcn_inverse_ballot_w64(m);
 }
 
 // Smallest value of the quadratic form over the pixel rectangle
@@ -188,27 +184,6 @@ __device__ __forceinline__ GsRecord load_projected(const float* __restrict__ pme
   return r;
 }
 
-__device__ __forceinline__ float bcast(float x, int j) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), j));
-}
-
-// Broadcasts lane j's splat to the whole wave (v_readlane into SGPRs, so the
-// per-pixel math takes the Gaussian's fields as scalar operands).
-__device__ __forceinline__ Splat broadcast(const LaneSplat& l, int j) {
-  Splat s;
-  s.u = bcast(l.u, j);
-  s.v = bcast(l.v, j);
-  s.o = bcast(l.o, j);
-  s.pa = bcast(l.pa, j);
-  s.pb = bcast(l.pb, j);
-  s.pc = bcast(l.pc, j);
-  s.cut = bcast(l.cut, j);
-  s.r = bcast(l.r, j);
-  s.g = bcast(l.g, j);
-  s.bl = bcast(l.b, j);
-  return s;
-}
-
 // DPP read of another lane's value (all rows and banks enabled; a lane whose
 // source is out of range reads 0).  Combined with an add it compiles to a single
 // v_add_f32_dpp.
@@ -245,23 +220,42 @@ __device__ __forceinline__ float fold_rows(float x, float y) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-// Wave totals of nine per-lane values v[0..8] by a transposing reduction:
-// the two swap folds spread the values over the rows of three registers and a
-// row sum finishes each, 30 VALU operations instead of 54 for nine full
-// butterflies.  On return, every lane of row r (lanes 16 r .. 16 r + 15) of
-//   t0 holds the total of v[sum9_field(r)],  t1 that of v[4 + sum9_field(r)],
-// and t2 holds the total of v[8] in every lane.  Needs a full EXEC.
+// Lanes of `a` with those of the row's banks (groups of four lanes) in
+// BANKS taken from `b`.
+template <int BANKS>
+__device__ __forceinline__ float merge_banks(float a, float b) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(a), __float_as_int(b), 0xE4,
+                                                    0xF, BANKS, false));
+}
+
+// Wave totals of nine per-lane values v[0..8] by a transposing reduction: the
+// two swap folds spread the values over the rows of three registers, whose
+// sums along the row then share instructions (each row holds three values in
+// its banks after the merges): 25 VALU operations instead of 54 for nine full
+// butterflies.  On return lane i of row r holds the total of
+//   v[sum9_field(r)] in lanes 0-3, v[8] in lanes 4-7,
+//   v[4 + sum9_field(r)] in lanes 8-15 of the row.  Needs a full EXEC.
 __device__ __forceinline__ int sum9_field(int row) { return ((row & 1) << 1) | (row >> 1); }
 
-__device__ __forceinline__ void wave_sum9(const float (&v)[9], float& t0, float& t1, float& t2) {
+__device__ __forceinline__ float wave_sum9(const float (&v)[9]) {
   const float a0 = fold_halves(v[0], v[1]);
   const float a1 = fold_halves(v[2], v[3]);
   const float a2 = fold_halves(v[4], v[5]);
   const float a3 = fold_halves(v[6], v[7]);
   const float a4 = fold_halves(v[8], v[8]);
-  t0 = row_sum(fold_rows(a0, a1));  // rows: v0, v2, v1, v3
-  t1 = row_sum(fold_rows(a2, a3));  // rows: v4, v6, v5, v7
-  t2 = row_sum(fold_rows(a4, a4));  // every row: v8
+  float t0 = fold_rows(a0, a1);  // rows: v0, v2, v1, v3
+  float t1 = fold_rows(a2, a3);  // rows: v4, v6, v5, v7
+  float t2 = fold_rows(a4, a4);  // every row: v8
+  t0 += dpp0<0x128>(t0);  // row_ror:8
+  t1 += dpp0<0x128>(t1);
+  t2 += dpp0<0x128>(t2);
+  float t = merge_banks<0xC>(t0, t1);
+  t += dpp0<0x141>(t);  // row_half_mirror
+  t2 += dpp0<0x141>(t2);
+  t = merge_banks<0x2>(t, t2);
+  t += dpp0<0xB1>(t);  // quad_perm [1,0,3,2]
+  t += dpp0<0x4E>(t);  // quad_perm [2,3,0,1]
+  return t;
 }
 
 }  // namespace gs
