@@ -275,6 +275,12 @@ _SIGNATURES = {
         [c_int64, c_int32, c_int32, c_void_p, c_int64, c_int64, c_int64,
          c_void_p, c_size_t, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p],
     ),
+    "gs_small_lists_bytes": (c_size_t, [c_int64, c_int32, c_int32]),
+    "gs_small_lists": (
+        c_int,
+        [c_void_p, c_void_p, c_int64, c_int32, c_int32, c_void_p, c_void_p, c_int64, c_void_p,
+         c_size_t, c_void_p, c_int32, c_void_p],
+    ),
     "gs_tile_order_workspace_bytes": (c_size_t, [c_int32]),
     "gs_tile_order_items": (c_int64, [GsView, c_int32]),
     "gs_tile_order": (

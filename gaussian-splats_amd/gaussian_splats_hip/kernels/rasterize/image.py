@@ -103,6 +103,25 @@ class _Walk:
     __slots__ = ("view", "accumulator", "checkpoints", "hits", "order")
 
 
+def small_lists(depth_keys, tile_rects, tiles_w, tiles_h, nbytes, clear=None):
+    """Tile lists of a small scene (gs_small_lists; ``nbytes`` its workspace):
+    ``(gaussian_ids, ranges)`` with n slots per tile, so no total is read back
+    and the call does not wait.  ``clear``: an optional [N, C] tensor to zero."""
+    n, device = tile_rects.shape[0], tile_rects.device
+    ids = torch.empty(n * tiles_w * tiles_h, dtype=torch.int32, device=device)
+    ranges = torch.empty((tiles_w * tiles_h, 2), dtype=torch.int64, device=device)
+    ws = nat.workspace(nbytes, device)
+    nat.check(
+        nat.library().gs_small_lists(
+            nat.ptr(depth_keys), nat.ptr(tile_rects), n, tiles_w, tiles_h, nat.ptr(ranges),
+            nat.ptr(ids), ids.numel(), nat.ptr(ws), ws.numel(), nat.ptr(clear),
+            clear.shape[1] if clear is not None else 0, nat.stream(device),
+        ),
+        "small_lists",
+    )
+    return ids, ranges
+
+
 def forward_image(params, request: ImageRequest, keep: bool, timer=None):
     """Projects, bins and composites; returns ``(image [V, H, W, 3], saved,
     walk)``, the last two None unless ``keep`` (a backward will follow)."""
@@ -135,13 +154,20 @@ def forward_image(params, request: ImageRequest, keep: bool, timer=None):
     backward = keep and request.gaussian
     # The backward's [V N, 9] gradient accumulator, zeroed beside the depth sort.
     accumulator = (torch.empty((vn, 9), dtype=torch.float32, device=device) if backward else None)
-    ids, ranges = bin_tiles(
-        depth_keys, None, None, tiles_w, tiles_h, timer=mark, tile_rects=tile_rects,
-        clear=accumulator, key_range=depth_key_range(request.near, request.far),
-    )
+    small = lib.gs_small_lists_bytes(vn, tiles_w, tiles_h)
+    if small:
+        ids, ranges = small_lists(depth_keys, tile_rects, tiles_w, tiles_h, small, accumulator)
+        longest = 0  # unknown to the host; too few Gaussians or tiles for checkpoints
+        mark("bin")
+        mark("emit")
+    else:
+        ids, ranges = bin_tiles(
+            depth_keys, None, None, tiles_w, tiles_h, timer=mark, tile_rects=tile_rects,
+            clear=accumulator, key_range=depth_key_range(request.near, request.far),
+        )
+        longest = nat.longest_list(ranges)
     mark("sort")
     view.active_tiles = nat.active_tiles(ranges)
-    longest = nat.longest_list(ranges)
     num_tiles, total = tiles_w * tiles_h, ids.numel()
     image = torch.empty((views, height, width, 3), dtype=torch.float32, device=device)
     checkpoints = nat.checkpoint_buffer(view, total, longest, device)

@@ -308,6 +308,20 @@ GS_API int gs_bin_tiles_emit(
     void* plan, size_t plan_bytes, const int64_t* ranges, int32_t* sorted_ids,
     void* workspace, size_t workspace_bytes, void* stream);
 
+/* Tile lists of a small scene (no counterpart in the reference, which sorts
+ * its intersections): the lists of gs_bin_tiles_plan and gs_bin_tiles_emit from
+ * the same depth_keys (not consumed) and tile_rects, without totals for the
+ * host to read.  ranges[t] lies in [t n, (t + 1) n): gaussian_ids holds n slots
+ * per tile (num_ids >= n * tiles).  clear (optional): n * clear_per_gaussian
+ * floats to zero.  gs_small_lists_bytes: the workspace, or 0 when the scene is
+ * not small (GS_ERR_UNSUPPORTED): above 24576 Gaussians, 2^24 slots or 256
+ * tiles per axis. */
+GS_API size_t gs_small_lists_bytes(int64_t n, int32_t tiles_w, int32_t tiles_h);
+GS_API int gs_small_lists(
+    const uint32_t* depth_keys, const uint32_t* tile_rects, int64_t n, int32_t tiles_w,
+    int32_t tiles_h, int64_t* ranges, int32_t* gaussian_ids, int64_t num_ids, void* workspace,
+    size_t workspace_bytes, float* clear, int32_t clear_per_gaussian, void* stream);
+
 /* Dispatch plan of the compositing kernels (no counterpart in the reference,
  * whose launches take tiles in index order): writes
  * gs_tile_order_items(view, n_contributors != NULL) int32 work items to

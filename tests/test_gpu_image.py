@@ -179,3 +179,50 @@ def test_image_tile_rule():
     assert image_tile(8, 800, 800, 10, views=16) == 16
     assert image_tile(8, 1000, 1000, 10, views=25) == 32
     assert image_tile(16, 640, 480, 1 << 26) is None
+
+
+@pytest.mark.parametrize("n,tw,th", [(1, 1, 1), (63, 5, 3), (64, 4, 1), (65, 3, 7), (1000, 256, 2),
+                                     (1025, 17, 256), (5000, 30, 41), (24576, 26, 26)])
+def test_small_lists_equal_bucketing(n, tw, th, device):
+    """gs_small_lists against the row/column bucketing: the same lists (ties
+    by index, Gaussians without a rectangle nowhere), and the clear buffer."""
+    from gaussian_splats_hip.kernels.rasterize import _native as nat
+    from gaussian_splats_hip.kernels.rasterize.image import small_lists
+    from gaussian_splats_hip.kernels.rasterize.intersections import bin_tiles
+
+    g = torch.Generator().manual_seed(n + tw)
+    x0, y0 = torch.randint(tw, (n,), generator=g), torch.randint(th, (n,), generator=g)
+    w = (torch.rand(n, generator=g).pow(3) * (tw - x0)).long() + 1
+    h = (torch.rand(n, generator=g).pow(3) * (th - y0)).long() + 1
+    rects = x0 | (w - 1) << 8 | y0 << 16 | (h - 1) << 24
+    # Few distinct depths, so ties are common.
+    keys = torch.randint(1 << 30, (max(1, n // 3),), generator=g)[
+        torch.randint(max(1, n // 3), (n,), generator=g)]
+    culled = torch.rand(n, generator=g) < 0.2
+    rects[culled], keys[culled] = 0xFFFFFFFF, 0xFFFFFFFF
+
+    def int32(t):
+        return torch.where(t >= 1 << 31, t - (1 << 32), t).to(torch.int32).to(device)
+
+    rects, keys = int32(rects), int32(keys)
+    nbytes = nat.library().gs_small_lists_bytes(n, tw, th)
+    assert nbytes
+    clear = torch.full((n, 9), 7.0, device=device)
+    ids, ranges = small_lists(keys, rects, tw, th, nbytes, clear)
+    assert not clear.any()
+    starts = torch.arange(tw * th, device=device) * n
+    assert torch.equal(ranges[:, 0], starts)
+    want_ids, want = bin_tiles(keys.clone(), None, None, tw, th, tile_rects=rects)
+    lengths = want[:, 1] - want[:, 0]
+    assert torch.equal(ranges[:, 1] - starts, lengths)
+    tile = torch.repeat_interleave(torch.arange(tw * th, device=device), lengths)
+    at = torch.arange(len(want_ids), device=device) - want[tile, 0] + starts[tile]
+    assert torch.equal(ids[at], want_ids)
+
+
+def test_small_lists_limits(device):
+    from gaussian_splats_hip.kernels.rasterize import _native as nat
+
+    size = nat.library().gs_small_lists_bytes
+    assert size(24576, 26, 26) and not size(24577, 1, 1) and not size(0, 4, 4)
+    assert size(256, 256, 256) and not size(257, 256, 256) and not size(10, 257, 1)
