@@ -216,6 +216,29 @@ inline CheckpointLayout checkpoint_layout(void* base, int tile_size, int64_t tot
   return c;
 }
 
+// Walk records (image calls whose forward splits every tile into quarters):
+// the walk back of a 16-pixel tile is cut at fixed walk positions, so that a
+// tile runs on up to kWalkSegments waves that each take all of its pixels.
+// Whenever a quarter's forward wave starts the batch at walk_bound(j), it
+// records per pixel (T, colour since its previous record), and at the end of
+// the walk turns the colours into the colour composited after the record (a
+// suffix sum, as with the checkpoints above).  Record j of a tile exists for the pixels still
+// active there, the only ones a backward segment starts from it.  Short bounds
+// first: segments are waves that take as long as they are, and twice as many
+// waves of half the length leave less of the chip idle at the end (300k
+// Gaussians at 1237 x 822, backward: 158 us, 190 with bounds twice as far).
+constexpr int kWalkSegments = 8;
+__host__ __device__ inline int walk_bound(int j) {  // 0 <= j < kWalkSegments
+  const int b[kWalkSegments] = {0, 64, 128, 192, 256, 384, 640, 1280};
+  return b[j];
+}
+constexpr int kWalkPixels = 256;  // per record
+inline size_t walk_record_bytes(int num_tiles) {
+  return size_t(num_tiles) * (kWalkSegments - 1) * kWalkPixels * 16;
+}
+// The forward's waves also leave each quarter's largest contributor count:
+// keys[4 tile + quarter].
+
 // Dispatch plan of the compositing kernels (gs_tile_order).  Each of the 8
 // XCD regions of tiles (a contiguous range of tile indices) owns the same
 // number of item slots; an item is one wave's work, tile << 7 | code:
@@ -388,6 +411,19 @@ __device__ __forceinline__ int xcd_swizzle(int b, int nb) {
   const int q = nb >> 3, r = nb & 7;
   const int x = b & 7;
   return x * q + min(x, r) + (b >> 3);
+}
+
+// Like xcd_swizzle, but XCD x takes every eighth chunk of 2^shift consecutive
+// work items instead of one contiguous range: neighbours still share an XCD's
+// L2, and a dense band of the image is spread over all of them.  The grid is
+// deal_grid(items) workgroups; indices past the last item have no work.
+__device__ __forceinline__ int xcd_deal(int b, int shift) {
+  const int i = b >> 3;
+  return ((((i >> shift) << 3) | (b & 7)) << shift) | (i & ((1 << shift) - 1));
+}
+inline int64_t deal_grid(int64_t items, int shift) {
+  const int64_t round = int64_t(8) << shift;
+  return (items + round - 1) / round * round;
 }
 
 __device__ __forceinline__ uint64_t lanemask_lt() {

@@ -22,6 +22,8 @@
 // them in one register, written by one nine-lane fp32 atomic add per (tile,
 // Gaussian).  Replaces composite_bwd.py:47-204 and the index_add_ scatter of
 // composite_bwd.py:268-273.
+#include <climits>
+
 #include "common.h"
 #include "raster_math.h"
 
@@ -58,6 +60,9 @@ struct CompositeBwdArgs {
   // The forward's hit masks (hit_mask_slot), read by the MASKS kernels.
   const uint64_t* hit_masks;
   int64_t hit_capacity;  // words
+  // WALK kernels: the forward's walk records and quarters' contributor counts.
+  const float4* walk_records;
+  const int32_t* quarter_keys;
 };
 
 // One wave takes PIX pixels per lane of `tile`: the 64-pixel bands band0 ..
@@ -79,7 +84,15 @@ struct CompositeBwdArgs {
 // RECORDS: the projection's 48-byte records are gathered (three 16-byte loads
 // of one or two lines, as the forward does) instead of the op's four projected
 // outputs.
-template <int TILE, bool ABS, int PIX, bool MASKS, bool RECORDS>
+// WALK: segment `seg` between the forward's walk bounds instead, started from
+// its walk records (a pixel no longer active at the segment's end starts from
+// its final T, with nothing composited after it).  On few tiles a wave per tile
+// leaves SIMDs idle behind the longest walk, and a wave per quarter of the
+// tile's bands repeats each entry's fold, reduction and atomic up to four times:
+// quarters -> segments 218 -> 158 us (300k Gaussians, 1237 x 822), 112 -> 81
+// (400k, 640 x 480), 59 -> 47 (20k, 403 x 307), 434 -> 303 (4M in a small cube);
+// the records cost the forward 3 to 15 us.
+template <int TILE, bool ABS, int PIX, bool MASKS, bool RECORDS, bool WALK>
 __device__ __forceinline__ void composite_bwd_tile(const CompositeBwdArgs& a, float4 (*chunk)[3],
                                                    int lane, int tile, int band0, int seg) {
   constexpr int NPIX = TILE * TILE;
@@ -91,6 +104,13 @@ __device__ __forceinline__ void composite_bwd_tile(const CompositeBwdArgs& a, fl
   const int vx = tx / a.view_tw, vy = ty / a.view_th;
   const int view = vy * a.cols + vx;
   if (view >= a.views) return;  // an empty slot of the mosaic's last row
+  // WALK: nothing to do for a segment past the tile's largest contributor count.
+  const int walk_lo = WALK ? walk_bound(seg) : 0;
+  const int walk_hi = WALK && seg + 1 < kWalkSegments ? walk_bound(seg + 1) : INT_MAX;
+  if constexpr (WALK) {
+    const int4 n4 = reinterpret_cast<const int4*>(a.quarter_keys)[tile];
+    if (max(max(n4.x, n4.y), max(n4.z, n4.w)) <= walk_lo) return;
+  }
   const int ox = (tx - vx * a.view_tw) * TILE, oy = (ty - vy * a.view_th) * TILE;
   const int64_t view_base = int64_t(view) * a.width * a.height;  // first pixel of the view
   const int64_t start = a.ranges[2 * tile];
@@ -137,7 +157,24 @@ __device__ __forceinline__ void composite_bwd_tile(const CompositeBwdArgs& a, fl
     max_n = __builtin_amdgcn_readfirstlane(max_n);
   }
   int lo = 0, hi = max_n;  // positions walked
-  if (seg >= 0) {
+  if constexpr (WALK) {
+    lo = walk_lo;
+    hi = min(max_n, walk_hi);
+    if (hi == walk_hi) {  // the walk goes on past this segment
+      const float4* rec = a.walk_records +
+                          (int64_t(tile) * (kWalkSegments - 1) + seg) * kWalkPixels + lane;
+#pragma unroll
+      for (int p = 0; p < PIX; ++p) {
+        if (ncon[p] > hi) {
+          const float4 v = rec[64 * p];
+          T[p] = v.x;
+          const float dot = gr[p] * v.y + gg[p] * v.z + gb[p] * v.w;
+          gs_[p] = v.x > 0.0f ? dot / v.x : 0.0f;
+        }
+      }
+    }
+    if (lo >= hi) return;
+  } else if (seg >= 0) {
     // Recorded checkpoints: a prefix of the tile's crossings (lane j reads
     // the table slot of crossing j + 1).
     const bool table =
@@ -352,6 +389,10 @@ __device__ __forceinline__ void composite_bwd_tile(const CompositeBwdArgs& a, fl
   }
 }
 
+// Tiles of the WALK kernel dealt to an XCD at a time (2^shift).
+constexpr int kWalkDealShift = 3;
+static_assert(kWalkSegments == 2 * kCompositeWaves, "two workgroups per tile");
+
 // kCompositeWaves waves per workgroup, one work item each (composite_item);
 // workgroups are mapped onto XCDs so that each XCD takes one region of the
 // plan (xcd_swizzle).  QUARTERS: the launch's items are quarters (every tile
@@ -360,7 +401,7 @@ __device__ __forceinline__ void composite_bwd_tile(const CompositeBwdArgs& a, fl
 // composites the whole tile and the others have no work.  Each kernel thus
 // composites every pixel of any plan exactly once, with one instance of the
 // walk (two would share one register allocation).
-template <int TILE, bool ABS, bool QUARTERS, bool MASKS, bool RECORDS>
+template <int TILE, bool ABS, bool QUARTERS, bool MASKS, bool RECORDS, bool WALK = false>
 __global__ __launch_bounds__(kCompositeWaves * 64) void composite_bwd_kernel(CompositeBwdArgs a) {
   constexpr int NPIX = TILE * TILE;
   constexpr int PIX_TILE = NPIX >= 64 ? NPIX / 64 : 1;
@@ -372,6 +413,21 @@ __global__ __launch_bounds__(kCompositeWaves * 64) void composite_bwd_kernel(Com
   // (pb, pc, r, g), (b, oa, ob, oc): written once per lane, then read as LDS
   // broadcasts per entry instead of twelve v_readlane.
   __shared__ float4 chunk[kCompositeWaves][64][3];
+  if constexpr (WALK) {
+    // A workgroup takes half of a tile's segments: all tiles' later halves
+    // first (few exist, but they are the long ones), then the earlier ones.
+    // Interleaved, every second workgroup would have no work, and those with
+    // work go to the same half of the shader engines (300k Gaussians at 1237 x
+    // 822: 303 us).
+    const int half_grid = gridDim.x >> 1;
+    const bool later = int(blockIdx.x) < half_grid;
+    const int tile = xcd_deal(later ? blockIdx.x : blockIdx.x - half_grid, kWalkDealShift);
+    const int seg = (later ? kCompositeWaves : 0) + ((wid + tile) & (kCompositeWaves - 1));
+    if (tile < a.num_tiles)
+      composite_bwd_tile<TILE, ABS, PIX_TILE, MASKS, RECORDS, true>(a, chunk[wid], lane, tile, 0,
+                                                                    seg);
+    return;
+  }
   const int slot = xcd_swizzle(blockIdx.x, gridDim.x) * kCompositeWaves + wid;
   int tile, kind, index;
   if (!composite_item(a.items, a.num_items, a.num_tiles, a.split_all, slot, tile, kind, index))
@@ -380,21 +436,29 @@ __global__ __launch_bounds__(kCompositeWaves * 64) void composite_bwd_kernel(Com
     static_assert(PIX_TILE >= kCompositeWaves, "quarters of 64-pixel bands");
     constexpr int QPIX = PIX_TILE / kCompositeWaves;
     if (kind == kItemQuarter) {
-      composite_bwd_tile<TILE, ABS, QPIX, MASKS, RECORDS>(a, chunk[wid], lane, tile, index * QPIX, -1);
+      composite_bwd_tile<TILE, ABS, QPIX, MASKS, RECORDS, false>(a, chunk[wid], lane, tile, index * QPIX, -1);
     } else if (kind == kItemTile || index == 0) {  // a segmented tile whole, by its first item
       for (int q = 0; q < kCompositeWaves; ++q)
-        composite_bwd_tile<TILE, ABS, QPIX, MASKS, RECORDS>(a, chunk[wid], lane, tile, q * QPIX, -1);
+        composite_bwd_tile<TILE, ABS, QPIX, MASKS, RECORDS, false>(a, chunk[wid], lane, tile, q * QPIX, -1);
     }
   } else {
     if (kind == kItemQuarter && index != 0) return;  // the tile whole, by its first quarter
-    composite_bwd_tile<TILE, ABS, PIX_TILE, MASKS, RECORDS>(a, chunk[wid], lane, tile, 0,
-                                                            kind == kItemSegment ? index : -1);
+    composite_bwd_tile<TILE, ABS, PIX_TILE, MASKS, RECORDS, false>(
+        a, chunk[wid], lane, tile, 0, kind == kItemSegment ? index : -1);
   }
 }
 
 template <int TILE, bool QUARTERS, bool MASKS>
 void launch_masks(const CompositeBwdArgs& a, unsigned blocks, hipStream_t s) {
   if constexpr (MASKS && TILE >= 16) {  // image calls (gs_composite_bwd_image)
+    if constexpr (TILE == 16 && QUARTERS) {
+      if (a.walk_records) {
+        launch_timed(composite_bwd_kernel<16, false, false, true, true, true>,
+                     unsigned(2 * deal_grid(a.num_tiles, kWalkDealShift)), kCompositeWaves * 64, 0,
+                     s, a);
+        return;
+      }
+    }
     if (a.records) {
       launch_timed(composite_bwd_kernel<TILE, false, QUARTERS, true, true>, blocks,
                    kCompositeWaves * 64, 0, s, a);
@@ -445,7 +509,7 @@ int composite_bwd(const float* projected_mean, const float* inverse_covariance,
                   const int32_t* tile_order, gs_view view, float* grad_projected,
                   float* grad_absolute, const void* checkpoints, size_t checkpoint_bytes,
                   int64_t num_intersections, const uint64_t* hit_masks, size_t hit_mask_bytes,
-                  void* stream) {
+                  const void* walk, size_t walk_bytes, void* stream) {
   GS_TRY(check_view(view, true));
   GS_REQUIRE(view.rendering_mode == GS_MODE_GAUSSIAN, GS_ERR_UNSUPPORTED,
              "Backward gradients are only supported for Gaussian rendering.");
@@ -502,6 +566,16 @@ int composite_bwd(const float* projected_mean, const float* inverse_covariance,
                "hit masks must be 8-byte aligned");
     a.hit_capacity = words;
   }
+  a.walk_records = nullptr;
+  a.quarter_keys = nullptr;
+  if (walk) {
+    const size_t need = gs_composite_walk_bytes(view);
+    GS_REQUIRE(need > 0 && walk_bytes >= need, GS_ERR_WORKSPACE,
+               "walk buffer too small (%zu bytes, need %zu)", walk_bytes, need);
+    a.walk_records = static_cast<const float4*>(walk);
+    a.quarter_keys = reinterpret_cast<const int32_t*>(static_cast<const char*>(walk) +
+                                                      walk_record_bytes(a.num_tiles));
+  }
   a.ckpt_stamp = nullptr;
   a.ckpt_table_len = 0;
   // The forward records checkpoints under these conditions only
@@ -549,7 +623,7 @@ extern "C" GS_API int gs_composite_bwd(const float* projected_mean,
                        nullptr, n, gaussian_ids, ranges, grad_image, final_transmittance,
                        n_contributors, tile_order, view, grad_projected, grad_absolute,
                        checkpoints, checkpoint_bytes, num_intersections, hit_masks,
-                       hit_mask_bytes, stream);
+                       hit_mask_bytes, nullptr, 0, stream);
 }
 
 extern "C" GS_API int gs_composite_bwd_image(
@@ -557,7 +631,7 @@ extern "C" GS_API int gs_composite_bwd_image(
     const float* grad_image, const float* final_transmittance, const int32_t* n_contributors,
     const int32_t* tile_order, gs_view view, float* grad_projected, const void* checkpoints,
     size_t checkpoint_bytes, int64_t num_intersections, const uint64_t* hit_masks,
-    size_t hit_mask_bytes, void* stream) {
+    size_t hit_mask_bytes, const void* walk, size_t walk_bytes, void* stream) {
   clear_error();
   GS_REQUIRE(view.tile_size >= 16, GS_ERR_UNSUPPORTED,
              "image calls composite tiles of 16 or 32 pixels (got %d)", view.tile_size);
@@ -566,5 +640,5 @@ extern "C" GS_API int gs_composite_bwd_image(
                        static_cast<const GsRecord*>(records), n, gaussian_ids, ranges, grad_image,
                        final_transmittance, n_contributors, tile_order, view, grad_projected,
                        nullptr, checkpoints, checkpoint_bytes, num_intersections, hit_masks,
-                       hit_mask_bytes, stream);
+                       hit_mask_bytes, walk, walk_bytes, stream);
 }

@@ -57,6 +57,11 @@ struct CompositeArgs {
   // checkpoints a backward walk crosses), written by whole-tile walks; or
   // null: none.
   uint32_t* tile_keys;
+  // Walk records of quarter waves (walk_bound) and, per quarter, the largest
+  // contributor count; or null: none.
+  float4* walk_records;
+  int32_t* quarter_keys;
+  int deal_shift;  // without a plan: chunk of workgroups dealt to an XCD (negative: contiguous)
 };
 
 // One wave composites PIX pixels per lane of `tile`: the 64-pixel bands
@@ -157,6 +162,27 @@ __device__ __forceinline__ void composite_tile(const CompositeArgs& a, float4 (*
     ++ck_count;
     ck_next = ck_count < kMaxCheckpoints ? checkpoint_batch(start, ck_count + 1) : -1;
   };
+  // Quarter waves with walk records: at each bound of the walk (a batch start)
+  // the pixels' T and the colour since the previous record, summed beside the
+  // image's own sum (pr, pg, pb; the first record's is the image's), so that
+  // the image does not depend on the records.
+  constexpr bool kRecords = HITS && TILE == 16 && PIX == 1;
+  int walk_count = 0, walk_next = -1;
+  float pr = 0.0f, pg = 0.0f, pb = 0.0f;
+  if constexpr (kRecords) walk_next = a.walk_records ? walk_bound(1) : -1;
+  float4* const walk = kRecords ? a.walk_records + int64_t(tile) * (kWalkSegments - 1) * kWalkPixels +
+                                      64 * band0 + lane
+                                : nullptr;
+  auto record_at = [&](int bpos) {
+    if constexpr (kRecords) {
+      if (bpos != walk_next) return;
+      walk[walk_count * kWalkPixels] =
+          walk_count == 0 ? make_float4(T[0], cr[0], cg[0], cb[0]) : make_float4(T[0], pr, pg, pb);
+      pr = pg = pb = 0.0f;
+      ++walk_count;
+      walk_next = walk_count + 1 < kWalkSegments ? walk_bound(walk_count + 1) : -1;
+    }
+  };
   // The overlap test's rectangle: the columns and rows of the pixels still
   // active (a set that only shrinks along the walk; the walk is running, so it
   // is not empty).
@@ -228,6 +254,11 @@ __device__ __forceinline__ void composite_tile(const CompositeArgs& a, float4 (*
         cr[k] += w * s.r;
         cg[k] += w * s.g;
         cb[k] += w * s.bl;
+        if (kRecords && walk_count > 0) {
+          pr += w * s.r;
+          pg += w * s.g;
+          pb += w * s.bl;
+        }
         T[k] = T[k] - w;
         const uint64_t done = ballot_of(!(T[k] > a.t_active)) & hit;
         ncon[k] = in_mask(done) ? pos + 1 : ncon[k];
@@ -292,6 +323,7 @@ __device__ __forceinline__ void composite_tile(const CompositeArgs& a, float4 (*
     // walked and each batch waits on one dependent load (the record gather).
     for (int64_t base = start; running && base < end; base += 64) {
       checkpoint_at(int(base - start));
+      record_at(int(base - start));
       float rx0, rx1, ry0, ry1;
       active_rect(rx0, rx1, ry0, ry1);
       const int64_t e = base + lane;
@@ -324,6 +356,22 @@ __device__ __forceinline__ void composite_tile(const CompositeArgs& a, float4 (*
     }
   }
 
+  if constexpr (kRecords) {
+    for (int j = walk_count - 1; j >= 0; --j) {
+      const float4 v = walk[j * kWalkPixels];
+      walk[j * kWalkPixels] = make_float4(v.x, pr, pg, pb);
+      pr += v.y;
+      pg += v.z;
+      pb += v.w;
+    }
+    if (a.walk_records) {
+      int m = ncon[0];
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o, 64));
+      if (lane == 0) a.quarter_keys[tile * 4 + band0] = m;
+    }
+  }
+
 #pragma unroll
   for (int k = 0; k < PIX; ++k) {
     const int q = lane + 64 * (band0 + k);
@@ -353,9 +401,19 @@ __device__ __forceinline__ void composite_tile(const CompositeArgs& a, float4 (*
   }
 }
 
+// Tiles up to which a launch without a plan deals chunks of 8 workgroups to the
+// XCDs.  A tile list follows the scene, dense in the middle of most images, and
+// with one contiguous range per XCD the middle ones finished last (200k
+// Gaussians at 1080p 122 -> 111 us, 100k at 640 x 480 62 -> 51; 1M at 1080p 97
+// either way).  More tiles are several rounds of the resident waves: ranges
+// then cost nothing and keep neighbours in one L2 (16 views of 2500 tiles: 1434
+// us, dealt 1500).
+constexpr int kDealTiles = 16384;
+constexpr int kDealShift = 3;
+
 // kCompositeWaves waves per workgroup, one work item each (composite_item);
 // workgroups are mapped onto XCDs so that each XCD takes one region of the
-// plan (xcd_swizzle).  QUARTERS: the launch's items are quarters (every tile
+// plan (xcd_swizzle) or, without a plan, chunks of neighbours (kDealTiles).  QUARTERS: the launch's items are quarters (every tile
 // split); a whole-tile item is then composited as its four quarters in turn.
 // Otherwise items are whole tiles; of a tile split into several items the
 // first composites the whole tile and the others have no work.  Each kernel
@@ -376,7 +434,9 @@ __global__ __launch_bounds__(kCompositeWaves * 64) void composite_fwd_kernel(Com
   // The second batch of a two-batch step (checkpoint kernel only).
   __shared__ float4 chunk2[kCompositeWaves][CKPT ? 64 : 1][3];
   __shared__ int ck_slots[kCompositeWaves][CKPT ? kMaxCheckpoints : 1];  // a wave's records
-  const int slot = xcd_swizzle(blockIdx.x, gridDim.x) * kCompositeWaves + wid;
+  const int group = a.items || a.deal_shift < 0 ? xcd_swizzle(blockIdx.x, gridDim.x)
+                                                : xcd_deal(blockIdx.x, a.deal_shift);
+  const int slot = group * kCompositeWaves + wid;
   int tile, kind, index;
   if (!composite_item(a.items, a.num_items, a.num_tiles, a.split_all, slot, tile, kind, index))
     return;
@@ -403,9 +463,10 @@ __global__ __launch_bounds__(kCompositeWaves * 64) void composite_fwd_kernel(Com
 
 template <int TILE, bool QUARTERS, bool CKPT>
 void launch_items(const CompositeArgs& a, bool ellipsoid, hipStream_t s) {
-  const unsigned blocks = unsigned(
-      a.items ? a.num_items / kCompositeWaves
-              : (a.split_all ? a.num_tiles : ceil_div(a.num_tiles, kCompositeWaves)));
+  const int64_t groups = a.split_all ? a.num_tiles : ceil_div(a.num_tiles, kCompositeWaves);
+  const unsigned blocks = unsigned(a.items             ? a.num_items / kCompositeWaves
+                                   : a.deal_shift < 0 ? groups
+                                                      : deal_grid(groups, a.deal_shift));
   if (ellipsoid)
     launch_timed(composite_fwd_kernel<TILE, true, QUARTERS, CKPT, false>, blocks, kCompositeWaves * 64, 0,
                  s, a);
@@ -471,7 +532,8 @@ int composite(const void* records, int64_t num_records, const int32_t* gaussian_
               int64_t num_intersections, int64_t longest_list, const int64_t* ranges,
               const int32_t* tile_order, gs_view view, float* image, float* final_transmittance, int32_t* n_contributors,
               void* checkpoints, size_t checkpoint_bytes, uint64_t* hit_masks,
-              size_t hit_mask_bytes, uint32_t* tile_keys, size_t tile_keys_bytes, void* stream) {
+              size_t hit_mask_bytes, uint32_t* tile_keys, size_t tile_keys_bytes,
+              void* walk_records, int32_t* quarter_keys, void* stream) {
   GS_TRY(check_view(view, true));
   GS_REQUIRE(ranges && image, GS_ERR_INVALID_ARGUMENT, "null pointer argument");
   GS_REQUIRE(num_records >= 0 && num_records <= (int64_t(1) << 31), GS_ERR_INVALID_ARGUMENT,
@@ -516,6 +578,9 @@ int composite(const void* records, int64_t num_records, const int32_t* gaussian_
   // Keys come from whole-tile walks; with every tile split into quarters the
   // backward's plan computes them itself.
   a.tile_keys = plan.split_all ? nullptr : tile_keys;
+  a.walk_records = plan.split_all ? static_cast<float4*>(walk_records) : nullptr;
+  a.quarter_keys = quarter_keys;
+  a.deal_shift = a.num_tiles <= kDealTiles ? kDealShift : -1;
   if (hit_masks) {
     GS_REQUIRE(view.rendering_mode == GS_MODE_GAUSSIAN, GS_ERR_UNSUPPORTED,
                "hit masks are recorded for Gaussian rendering only (its backward reads them)");
@@ -579,7 +644,7 @@ extern "C" GS_API int gs_composite(const void* records, int64_t num_records,
   return composite(records, num_records, gaussian_ids, num_intersections, 0, ranges, tile_order,
                    view, image, final_transmittance, n_contributors, checkpoints,
                    checkpoint_bytes, hit_masks, hit_mask_bytes, tile_keys, tile_keys_bytes,
-                   stream);
+                   nullptr, nullptr, stream);
 }
 
 extern "C" GS_API int gs_composite_image(const void* records, int64_t num_records,
@@ -591,5 +656,34 @@ extern "C" GS_API int gs_composite_image(const void* records, int64_t num_record
   GS_REQUIRE(longest_list >= 0, GS_ERR_INVALID_ARGUMENT, "negative list length");
   return composite(records, num_records, gaussian_ids, num_intersections, longest_list, ranges,
                    tile_order, view, image, nullptr, nullptr, nullptr, 0, nullptr, 0, nullptr, 0,
-                   stream);
+                   nullptr, nullptr, stream);
+}
+
+extern "C" GS_API size_t gs_composite_walk_bytes(gs_view view) {
+  if (check_view(view, true) != GS_OK || view.tile_size != 16) return 0;
+  const Mosaic m = mosaic_of(view);
+  if (!dispatch_plan(m.num_tiles(), 16, view.active_tiles, false).split_all) return 0;
+  return walk_record_bytes(m.num_tiles()) + align_up(size_t(m.num_tiles()) * 16);
+}
+
+extern "C" GS_API int gs_composite_walk(
+    const void* records, int64_t num_records, const int32_t* gaussian_ids,
+    int64_t num_intersections, const int64_t* ranges, gs_view view, float* image,
+    float* final_transmittance, int32_t* n_contributors, uint64_t* hit_masks,
+    size_t hit_mask_bytes, void* walk, size_t walk_bytes, void* stream) {
+  clear_error();
+  const size_t need = gs_composite_walk_bytes(view);
+  GS_REQUIRE(need > 0 && view.rendering_mode == GS_MODE_GAUSSIAN, GS_ERR_UNSUPPORTED,
+             "walk records are for Gaussian rendering on few tiles of 16 pixels");
+  GS_REQUIRE(final_transmittance && n_contributors && hit_masks && walk, GS_ERR_INVALID_ARGUMENT,
+             "null pointer argument");
+  GS_REQUIRE(walk_bytes >= need, GS_ERR_WORKSPACE,
+             "walk buffer too small (%zu bytes, need %zu)", walk_bytes, need);
+  GS_REQUIRE((reinterpret_cast<uintptr_t>(walk) & 15u) == 0, GS_ERR_INVALID_ARGUMENT,
+             "the walk buffer must be 16-byte aligned");
+  int32_t* keys = reinterpret_cast<int32_t*>(static_cast<char*>(walk) +
+                                             walk_record_bytes(mosaic_of(view).num_tiles()));
+  return composite(records, num_records, gaussian_ids, num_intersections, 0, ranges, nullptr, view,
+                   image, final_transmittance, n_contributors, nullptr, 0, hit_masks,
+                   hit_mask_bytes, nullptr, 0, walk, keys, stream);
 }

@@ -100,7 +100,7 @@ class ImageRequest:
 class _Walk:
     """What the forward keeps for its backward beside the saved tensors."""
 
-    __slots__ = ("view", "accumulator", "checkpoints", "hits", "order")
+    __slots__ = ("view", "accumulator", "checkpoints", "hits", "order", "records")
 
 
 def small_lists(depth_keys, tile_rects, tiles_w, tiles_h, nbytes, clear=None):
@@ -187,25 +187,42 @@ def forward_image(params, request: ImageRequest, keep: bool, timer=None):
     final_transmittance = torch.empty((views, height, width), dtype=torch.float32, device=device)
     n_contributors = torch.empty((views, height, width), dtype=torch.int32, device=device)
     hits = nat.hit_mask_buffer(view, total, device)
-    keys = nat.workspace(lib.gs_tile_order_workspace_bytes(num_tiles), device)
-    nat.check(
-        nat.launch("composite", lambda: lib.gs_composite(
-            ptr(records), vn, ptr(ids), total, ptr(ranges), ptr(plan), view, ptr(image),
-            ptr(final_transmittance), ptr(n_contributors), ptr(checkpoints),
-            nat.buffer_bytes(checkpoints), ptr(hits), nat.buffer_bytes(hits), ptr(keys),
-            keys.numel(), stream,
-        )),
-        "composite",
-    )
-    mark("composite")
-    # The backward's dispatch plan, behind the forward on the stream.
     walk = _Walk()
-    walk.order = torch.empty(lib.gs_tile_order_items(view, 1), dtype=torch.int32, device=device)
-    nat.check(
-        lib.gs_tile_order(ptr(ranges), ptr(n_contributors), view, ptr(walk.order), ptr(keys),
-                          keys.numel(), 1, stream),
-        "tile_order",
-    )
+    walk.order = walk.records = None
+    walk_bytes = lib.gs_composite_walk_bytes(view)
+    if walk_bytes:
+        # Few tiles: the walk's state at fixed positions, for a backward in
+        # segments (no plan: the segments are dealt in tile order).
+        walk.records = nat.workspace(walk_bytes, device)
+        nat.check(
+            nat.launch("composite", lambda: lib.gs_composite_walk(
+                ptr(records), vn, ptr(ids), total, ptr(ranges), view, ptr(image),
+                ptr(final_transmittance), ptr(n_contributors), ptr(hits), nat.buffer_bytes(hits),
+                ptr(walk.records), walk_bytes, stream,
+            )),
+            "composite_walk",
+        )
+        mark("composite")
+    else:
+        keys = nat.workspace(lib.gs_tile_order_workspace_bytes(num_tiles), device)
+        nat.check(
+            nat.launch("composite", lambda: lib.gs_composite(
+                ptr(records), vn, ptr(ids), total, ptr(ranges), ptr(plan), view, ptr(image),
+                ptr(final_transmittance), ptr(n_contributors), ptr(checkpoints),
+                nat.buffer_bytes(checkpoints), ptr(hits), nat.buffer_bytes(hits), ptr(keys),
+                keys.numel(), stream,
+            )),
+            "composite",
+        )
+        mark("composite")
+        # The backward's dispatch plan, behind the forward on the stream.
+        walk.order = torch.empty(lib.gs_tile_order_items(view, 1), dtype=torch.int32,
+                                 device=device)
+        nat.check(
+            lib.gs_tile_order(ptr(ranges), ptr(n_contributors), view, ptr(walk.order), ptr(keys),
+                              keys.numel(), 1, stream),
+            "tile_order",
+        )
     walk.view, walk.accumulator, walk.checkpoints, walk.hits = view, accumulator, checkpoints, hits
     return image, (records, tile_rects, ids, ranges, final_transmittance, n_contributors), walk
 
@@ -237,7 +254,8 @@ def backward_image(params, saved, walk: _Walk, request: ImageRequest, grad_image
             ptr(records), records.shape[0], ptr(ids), ptr(ranges), ptr(grad_image),
             ptr(final_transmittance), ptr(n_contributors), ptr(walk.order), walk.view,
             ptr(accumulator), ptr(walk.checkpoints), nat.buffer_bytes(walk.checkpoints),
-            ids.numel(), ptr(walk.hits), nat.buffer_bytes(walk.hits), stream,
+            ids.numel(), ptr(walk.hits), nat.buffer_bytes(walk.hits), ptr(walk.records),
+            nat.buffer_bytes(walk.records), stream,
         )),
         "composite_bwd_image",
     )

@@ -427,6 +427,19 @@ GS_API int gs_composite_image(
     int64_t num_intersections, int64_t longest_list, const int64_t* ranges,
     const int32_t* tile_order, gs_view view, float* image, void* stream);
 
+/* gs_composite for a Gaussian image call on few tiles (fewer than 4096 tiles
+ * of 16 pixels with work, whose pixel bands are split over four waves each),
+ * which also records the walk's state at fixed positions, so that
+ * gs_composite_bwd_image walks each tile back in segments of all of its
+ * pixels.  gs_composite_walk_bytes: the size of `walk`, or 0 when the view is
+ * not of that kind (GS_ERR_UNSUPPORTED). */
+GS_API size_t gs_composite_walk_bytes(gs_view view);
+GS_API int gs_composite_walk(
+    const void* records, int64_t num_records, const int32_t* gaussian_ids,
+    int64_t num_intersections, const int64_t* ranges, gs_view view, float* image,
+    float* final_transmittance, int32_t* n_contributors, uint64_t* hit_masks,
+    size_t hit_mask_bytes, void* walk, size_t walk_bytes, void* stream);
+
 /* Back-to-front compositing gradient, accumulated with atomics into
  * grad_projected[N,9] (zeroed by the caller), from the op's projected outputs
  * of n Gaussians (list ids clamped to [0, n), as in gs_composite).
@@ -459,13 +472,14 @@ GS_API int gs_composite_bwd(
 
 /* gs_composite_bwd from the records of gs_project_image (n of them) instead
  * of the op's projected outputs, for tiles of 16 and 32 pixels and with the
- * forward's hit masks (both required). */
+ * forward's hit masks (both required).  walk: the buffer gs_composite_walk
+ * filled for the same lists and view (tile_order is then not used), or NULL. */
 GS_API int gs_composite_bwd_image(
     const void* records, int64_t n, const int32_t* gaussian_ids, const int64_t* ranges,
     const float* grad_image, const float* final_transmittance, const int32_t* n_contributors,
     const int32_t* tile_order, gs_view view, float* grad_projected, const void* checkpoints,
     size_t checkpoint_bytes, int64_t num_intersections, const uint64_t* hit_masks,
-    size_t hit_mask_bytes, void* stream);
+    size_t hit_mask_bytes, const void* walk, size_t walk_bytes, void* stream);
 
 /* Chain rule from grad_projected to the parameters.  Replaces project_bwd
  * (src/gaussian_splats/kernels/rasterize/project_bwd.py:8-381); gradients are

@@ -126,6 +126,35 @@ def test_image_long_lists(device):
     _same_gradients(second, want)
 
 
+@pytest.mark.parametrize("size,n", [(48, 4000), (24, 700), (24, 65), (24, 129), (736, 2500)])
+def test_image_walk_segments(size, n, device):
+    """Faint Gaussians that each cover the image: every pixel walks the whole
+    list, through every walk bound, and some pixels saturate on the way."""
+    g = torch.Generator().manual_seed(n)
+    scene = scenes.edge_case_scene(n=n, sh_degree=1, image_size=(size, size), seed=3)
+    scene.mean[:, :2] = torch.randn(n, 2, generator=g) * 0.3
+    scene.mean[:, 2] = -(torch.rand(n, generator=g) + 3)
+    scene.scale[:] = torch.rand(n, 3, generator=g) * 0.5 + 0.5
+    scene.opacity[:] = torch.randn(n, 1, generator=g) * 0.3 - 5
+    scene.opacity[n // 2::97] = 1.0
+    scene.mean[n // 2::97, :2] = torch.tensor([1.0, 0.5])
+    scene.scale[n // 2::97] = -1.0
+    scene = scene.to(device)
+    cam = scene.cameras[0]
+    splats = GaussianSplat.from_tensors(*scene.params())
+    leaves = [p.detach().clone().requires_grad_(True) for p in scene.params()]
+    image = rasterize(splats, cam, near=scene.near, far=scene.far)
+    expected = _op(scene, leaves, cam, 16, "gaussian")
+    assert torch.equal(image, expected)
+    weight = torch.linspace(-1, 1, image.numel(), device=device).reshape(image.shape)
+    loss = (image * weight).sum()
+    first = torch.autograd.grad(loss, [getattr(splats, p) for p in PARAMS], retain_graph=True)
+    second = torch.autograd.grad(loss, [getattr(splats, p) for p in PARAMS])
+    (expected * weight).sum().backward()
+    _same_gradients(first, [p.grad for p in leaves])
+    _same_gradients(second, [p.grad for p in leaves])
+
+
 def test_views_image_equals_op(device):
     scene = scenes.config5(seed=2, n=4000, views=5, size=90, focal=110).to(device)
     splats = GaussianSplat.from_tensors(*scene.params())
