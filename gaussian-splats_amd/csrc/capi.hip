@@ -57,6 +57,8 @@ int check_view(const gs_view& v, bool need_tiles) {
                "tile_size %d not supported (4, 8, 16 or 32)", v.tile_size);
     GS_REQUIRE(v.views >= 0 && v.mosaic_cols >= 0 && v.active_tiles >= 0,
                GS_ERR_INVALID_ARGUMENT, "views, mosaic_cols and active_tiles must be non-negative");
+    GS_REQUIRE(v.list_shift == 0 || (v.list_shift == 1 && v.tile_size == 16),
+               GS_ERR_INVALID_ARGUMENT, "list_shift must be 0, or 1 with tiles of 16 pixels");
     const int views = v.views > 1 ? v.views : 1;
     const int cols = std::min(views, v.mosaic_cols > 1 ? v.mosaic_cols : 1);
     const int64_t rows = (views + cols - 1) / cols;

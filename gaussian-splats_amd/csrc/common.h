@@ -189,13 +189,14 @@ struct CheckpointLayout {
 // buffer must come from the forward over the same lists.
 constexpr uint32_t kCheckpointMagic = 0x70636773u;  // "sgcp"
 constexpr int kCheckpointStampWords = 4;  // magic, tile size, tiles, table length
-inline CheckpointLayout checkpoint_layout(void* base, int tile_size, int64_t total,
+inline CheckpointLayout checkpoint_layout(void* base, int tile_size, int64_t total, int subs,
                                           size_t available = ~size_t(0)) {
   CheckpointLayout c;
   const size_t record = size_t(checkpoint_pixels(tile_size)) * 16;
   // A crossing's position lies below the list end + 64 (its batch starts
   // inside the list): table slots up to (total + 63) / kCheckpointEntries.
-  c.table_len = total / kCheckpointEntries + 2;
+  // With one list for several tiles each tile has slots of its own.
+  c.table_len = (total / kCheckpointEntries + 2) * subs;
   char* p = static_cast<char*>(base);
   size_t off = 0;
   auto take = [&](size_t n) {
@@ -228,9 +229,14 @@ inline CheckpointLayout checkpoint_layout(void* base, int tile_size, int64_t tot
 // waves of half the length leave less of the chip idle at the end (300k
 // Gaussians at 1237 x 822, backward: 158 us, 190 with bounds twice as far).
 constexpr int kWalkSegments = 8;
-__host__ __device__ inline int walk_bound(int j) {  // 0 <= j < kWalkSegments
-  const int b[kWalkSegments] = {0, 64, 128, 192, 256, 384, 640, 1280};
-  return b[j];
+// A list shared by 2 x 2 tiles (shift) holds about twice the entries a tile
+// keeps: the bounds double.  Long lists (above kCheckpointMinList) are those of
+// faint or dense scenes, which walk thousands of entries at places: bounds that
+// reach further.
+__host__ __device__ inline int walk_bound(int j, int shift, bool long_lists) {
+  const int b[2][kWalkSegments] = {{0, 64, 128, 192, 256, 384, 640, 1280},
+                                   {0, 128, 384, 768, 1280, 2048, 3072, 4608}};
+  return long_lists ? b[1][j] : b[0][j] << shift;  // 0 <= j < kWalkSegments
 }
 constexpr int kWalkPixels = 256;  // per record
 inline size_t walk_record_bytes(int num_tiles) {
@@ -346,15 +352,24 @@ __host__ __device__ inline int checkpoint_count(int64_t start, int max_n, int64_
 // start / 64 + t + b (unique for lists that follow each other in tile order,
 // as the binning writes them) times the tile's band count.  The backward
 // walks only the marked entries and bands.
-__host__ __device__ inline int64_t hit_mask_slot(int64_t start, int tile, int64_t batch) {
-  return (start >> 6) + tile + batch;
+// With one list for several tiles (gs_view.list_shift) t is the list, and each
+// of its `subs` tiles (sub) has its own masks.
+__host__ __device__ inline int64_t hit_mask_slot(int64_t start, int list, int64_t batch, int subs,
+                                                 int sub) {
+  return ((start >> 6) + list + batch) * subs + sub;
 }
 __host__ __device__ inline int tile_bands(int tile_size) {
   return tile_size * tile_size >= 64 ? tile_size * tile_size / 64 : 1;
 }
-__host__ __device__ inline int64_t hit_mask_words(int64_t num_intersections, int num_tiles,
-                                                  int tile_size) {
-  return (num_intersections / 64 + num_tiles + 2) * tile_bands(tile_size);
+inline int64_t hit_mask_words(int64_t num_intersections, int num_lists, int subs, int tile_size) {
+  return (num_intersections / 64 + num_lists + 2) * subs * tile_bands(tile_size);
+}
+
+// The list of mosaic tile (tx, ty), and which of the list's tiles it is.
+__host__ __device__ inline int list_of_tile(int tx, int ty, int tiles_w, int shift, int& sub) {
+  const int m = (1 << shift) - 1;
+  sub = ((ty & m) << shift) | (tx & m);
+  return (ty >> shift) * (tiles_w >> shift) + (tx >> shift);
 }
 
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
@@ -373,6 +388,9 @@ int check_view(const gs_view& v, bool need_tiles);
 // tiles; the mosaic is cols x rows views.
 struct Mosaic {
   int views, cols, rows, tw, th;
+  int shift;  // gs_view.list_shift
+  int subs() const { return 1 << (2 * shift); }  // tiles per list
+  int num_lists() const { return num_tiles() >> (2 * shift); }
   int tiles_w() const { return cols * tw; }
   int tiles_h() const { return rows * th; }
   int num_tiles() const { return tiles_w() * tiles_h(); }
@@ -383,8 +401,9 @@ inline Mosaic mosaic_of(const gs_view& v) {
   m.cols = v.mosaic_cols > 1 ? v.mosaic_cols : 1;
   if (m.cols > m.views) m.cols = m.views;
   m.rows = (m.views + m.cols - 1) / m.cols;
-  m.tw = tiles_along(v.image_width, v.tile_size);
-  m.th = tiles_along(v.image_height, v.tile_size);
+  m.shift = v.list_shift;
+  m.tw = tiles_along(v.image_width, v.tile_size << m.shift) << m.shift;
+  m.th = tiles_along(v.image_height, v.tile_size << m.shift) << m.shift;
   return m;
 }
 

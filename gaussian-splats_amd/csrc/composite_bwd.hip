@@ -47,6 +47,7 @@ struct CompositeBwdArgs {
   const int32_t* n_contrib;
   int width, height;       // per view
   int tiles_w, num_tiles;  // of the whole mosaic
+  int list_shift;            // lists of 2 x 2 tiles (gs_view.list_shift)
   int view_tw, view_th, cols, views;  // tiles per view, mosaic layout (one view: cols = views = 1)
   float* grad;      // [N, 9]
   float* grad_abs;  // [N, 2]: sums of |per-pixel mean gradient| (ABS kernels only)
@@ -63,6 +64,7 @@ struct CompositeBwdArgs {
   // WALK kernels: the forward's walk records and quarters' contributor counts.
   const float4* walk_records;
   const int32_t* quarter_keys;
+  bool long_lists;  // walk_bound's
 };
 
 // One wave takes PIX pixels per lane of `tile`: the 64-pixel bands band0 ..
@@ -105,15 +107,18 @@ __device__ __forceinline__ void composite_bwd_tile(const CompositeBwdArgs& a, fl
   const int view = vy * a.cols + vx;
   if (view >= a.views) return;  // an empty slot of the mosaic's last row
   // WALK: nothing to do for a segment past the tile's largest contributor count.
-  const int walk_lo = WALK ? walk_bound(seg) : 0;
-  const int walk_hi = WALK && seg + 1 < kWalkSegments ? walk_bound(seg + 1) : INT_MAX;
+  const int walk_lo = WALK ? walk_bound(seg, a.list_shift, a.long_lists) : 0;
+  const int walk_hi = WALK && seg + 1 < kWalkSegments ? walk_bound(seg + 1, a.list_shift, a.long_lists) : INT_MAX;
   if constexpr (WALK) {
     const int4 n4 = reinterpret_cast<const int4*>(a.quarter_keys)[tile];
     if (max(max(n4.x, n4.y), max(n4.z, n4.w)) <= walk_lo) return;
   }
   const int ox = (tx - vx * a.view_tw) * TILE, oy = (ty - vy * a.view_th) * TILE;
   const int64_t view_base = int64_t(view) * a.width * a.height;  // first pixel of the view
-  const int64_t start = a.ranges[2 * tile];
+  int sub;
+  const int list = list_of_tile(tx, ty, a.tiles_w, a.list_shift, sub);
+  const int subs = 1 << (2 * a.list_shift);
+  const int64_t start = a.ranges[2 * list];
 
   // The lane's pixels share one column (see column_terms).
   const float pxf = float(ox + lane % TILE);
@@ -180,10 +185,9 @@ __device__ __forceinline__ void composite_bwd_tile(const CompositeBwdArgs& a, fl
     const bool table =
         a.ckpt_table && a.ckpt_stamp[0] == kCheckpointMagic && a.ckpt_stamp[1] == uint32_t(TILE) &&
         a.ckpt_stamp[2] == uint32_t(a.num_tiles) && a.ckpt_stamp[3] == a.ckpt_table_len;
-    const int m = table ? checkpoint_count(start, max_n, a.ranges[2 * tile + 1] - start) : 0;
+    const int m = table ? checkpoint_count(start, max_n, a.ranges[2 * list + 1] - start) : 0;
     const int64_t first = checkpoint_first(start);
-    const int slot = lane < m ? a.ckpt_table[(first + int64_t(lane) * kCheckpointEntries) /
-                                             kCheckpointEntries]
+    const int slot = lane < m ? a.ckpt_table[(first / kCheckpointEntries + lane) * subs + sub]
                               : -1;
     // A slot outside the pool (never written by this forward) counts as missing.
     const uint64_t missing = __ballot(lane < m && (slot < 0 || int64_t(slot) >= a.ckpt_capacity));
@@ -229,7 +233,7 @@ __device__ __forceinline__ void composite_bwd_tile(const CompositeBwdArgs& a, fl
   const ConstMasks masks = (ConstMasks)a.hit_masks;
   uint64_t next_walk = ~uint64_t(0);
   auto load_masks = [&](int64_t bt) {
-    const int64_t w0 = hit_mask_slot(start, tile, bt) * kBands + band0;
+    const int64_t w0 = hit_mask_slot(start, list, bt, subs, sub) * kBands + band0;
     next_walk = 0;
 #pragma unroll
     for (int k = 0; k < PIX; ++k)
@@ -509,7 +513,7 @@ int composite_bwd(const float* projected_mean, const float* inverse_covariance,
                   const int32_t* tile_order, gs_view view, float* grad_projected,
                   float* grad_absolute, const void* checkpoints, size_t checkpoint_bytes,
                   int64_t num_intersections, const uint64_t* hit_masks, size_t hit_mask_bytes,
-                  const void* walk, size_t walk_bytes, void* stream) {
+                  const void* walk, size_t walk_bytes, int64_t longest_list, void* stream) {
   GS_TRY(check_view(view, true));
   GS_REQUIRE(view.rendering_mode == GS_MODE_GAUSSIAN, GS_ERR_UNSUPPORTED,
              "Backward gradients are only supported for Gaussian rendering.");
@@ -544,6 +548,7 @@ int composite_bwd(const float* projected_mean, const float* inverse_covariance,
   a.view_tw = m.tw;
   a.view_th = m.th;
   a.cols = m.cols;
+  a.list_shift = m.shift;
   a.views = m.views;
   a.grad = grad_projected;
   a.grad_abs = grad_absolute;
@@ -558,7 +563,8 @@ int composite_bwd(const float* projected_mean, const float* inverse_covariance,
   a.hit_capacity = 0;
   if (hit_masks) {
     GS_REQUIRE(num_intersections >= 0, GS_ERR_INVALID_ARGUMENT, "negative intersection count");
-    const int64_t words = hit_mask_words(num_intersections, a.num_tiles, view.tile_size);
+    const int64_t words =
+        hit_mask_words(num_intersections, m.num_lists(), m.subs(), view.tile_size);
     GS_REQUIRE(hit_mask_bytes >= size_t(words) * 8, GS_ERR_WORKSPACE,
                "hit mask buffer too small (%zu bytes, need %zu)", hit_mask_bytes,
                size_t(words) * 8);
@@ -568,6 +574,7 @@ int composite_bwd(const float* projected_mean, const float* inverse_covariance,
   }
   a.walk_records = nullptr;
   a.quarter_keys = nullptr;
+  a.long_lists = longest_list > kCheckpointMinList;
   if (walk) {
     const size_t need = gs_composite_walk_bytes(view);
     GS_REQUIRE(need > 0 && walk_bytes >= need, GS_ERR_WORKSPACE,
@@ -583,7 +590,7 @@ int composite_bwd(const float* projected_mean, const float* inverse_covariance,
   if (checkpoints && !plan.split_all && view.tile_size <= 16 && n > 0) {
     GS_REQUIRE(num_intersections >= 0, GS_ERR_INVALID_ARGUMENT, "negative intersection count");
     const CheckpointLayout c = checkpoint_layout(const_cast<void*>(checkpoints), view.tile_size,
-                                                 num_intersections, checkpoint_bytes);
+                                                 num_intersections, m.subs(), checkpoint_bytes);
     GS_REQUIRE(checkpoint_bytes >= c.header_bytes, GS_ERR_WORKSPACE,
                "checkpoint buffer too small (%zu bytes, need at least %zu)", checkpoint_bytes,
                c.header_bytes);
@@ -623,7 +630,7 @@ extern "C" GS_API int gs_composite_bwd(const float* projected_mean,
                        nullptr, n, gaussian_ids, ranges, grad_image, final_transmittance,
                        n_contributors, tile_order, view, grad_projected, grad_absolute,
                        checkpoints, checkpoint_bytes, num_intersections, hit_masks,
-                       hit_mask_bytes, nullptr, 0, stream);
+                       hit_mask_bytes, nullptr, 0, 0, stream);
 }
 
 extern "C" GS_API int gs_composite_bwd_image(
@@ -631,7 +638,8 @@ extern "C" GS_API int gs_composite_bwd_image(
     const float* grad_image, const float* final_transmittance, const int32_t* n_contributors,
     const int32_t* tile_order, gs_view view, float* grad_projected, const void* checkpoints,
     size_t checkpoint_bytes, int64_t num_intersections, const uint64_t* hit_masks,
-    size_t hit_mask_bytes, const void* walk, size_t walk_bytes, void* stream) {
+    size_t hit_mask_bytes, const void* walk, size_t walk_bytes, int64_t longest_list,
+    void* stream) {
   clear_error();
   GS_REQUIRE(view.tile_size >= 16, GS_ERR_UNSUPPORTED,
              "image calls composite tiles of 16 or 32 pixels (got %d)", view.tile_size);
@@ -640,5 +648,5 @@ extern "C" GS_API int gs_composite_bwd_image(
                        static_cast<const GsRecord*>(records), n, gaussian_ids, ranges, grad_image,
                        final_transmittance, n_contributors, tile_order, view, grad_projected,
                        nullptr, checkpoints, checkpoint_bytes, num_intersections, hit_masks,
-                       hit_mask_bytes, walk, walk_bytes, stream);
+                       hit_mask_bytes, walk, walk_bytes, longest_list, stream);
 }

@@ -36,6 +36,7 @@ struct CompositeArgs {
   bool long_walk;        // the CKPT kernel (tiles of at most 16 pixels)
   int width, height, tile;  // per view
   int tiles_w, num_tiles;    // of the whole mosaic
+  int list_shift;            // lists of 2 x 2 tiles (gs_view.list_shift)
   int view_tw, view_th, cols, views;  // tiles per view, mosaic layout (one view: cols = views = 1)
   float threshold;
   // A pixel stays active while (1 - T) < threshold, i.e. T > 1 - threshold.
@@ -61,6 +62,7 @@ struct CompositeArgs {
   // contributor count; or null: none.
   float4* walk_records;
   int32_t* quarter_keys;
+  bool long_lists;  // walk_bound's
   int deal_shift;  // without a plan: chunk of workgroups dealt to an XCD (negative: contiguous)
 };
 
@@ -84,8 +86,11 @@ __device__ __forceinline__ void composite_tile(const CompositeArgs& a, float4 (*
   const int ty = tile / a.tiles_w;
   const int vx = tx / a.view_tw, vy = ty / a.view_th;
   const int view = vy * a.cols + vx;
-  const int64_t start = a.ranges[2 * tile];
-  const int64_t end = a.ranges[2 * tile + 1];
+  int sub;
+  const int list = list_of_tile(tx, ty, a.tiles_w, a.list_shift, sub);
+  const int subs = 1 << (2 * a.list_shift);
+  const int64_t start = a.ranges[2 * list];
+  const int64_t end = a.ranges[2 * list + 1];
   const int list_len = int(end - start);
   write_key = write_key && a.tile_keys;
   if (view >= a.views) {  // an empty slot of the mosaic's last row
@@ -148,7 +153,7 @@ __device__ __forceinline__ void composite_tile(const CompositeArgs& a, float4 (*
     slot = uint32_t(__builtin_amdgcn_readfirstlane(int(slot)));
     const bool ok = ck_written == ck_count && int64_t(slot) < a.ckpt_capacity;
     const int64_t pos = checkpoint_first(start) + int64_t(ck_count) * kCheckpointEntries;
-    if (lane == 0) a.ckpt_table[pos / kCheckpointEntries] = ok ? int32_t(slot) : -1;
+    if (lane == 0) a.ckpt_table[pos / kCheckpointEntries * subs + sub] = ok ? int32_t(slot) : -1;
     if (ok) {
       float4* rec = a.ckpt_records + int64_t(slot) * kRecord;
 #pragma unroll
@@ -169,7 +174,7 @@ __device__ __forceinline__ void composite_tile(const CompositeArgs& a, float4 (*
   constexpr bool kRecords = HITS && TILE == 16 && PIX == 1;
   int walk_count = 0, walk_next = -1;
   float pr = 0.0f, pg = 0.0f, pb = 0.0f;
-  if constexpr (kRecords) walk_next = a.walk_records ? walk_bound(1) : -1;
+  if constexpr (kRecords) walk_next = a.walk_records ? walk_bound(1, a.list_shift, a.long_lists) : -1;
   float4* const walk = kRecords ? a.walk_records + int64_t(tile) * (kWalkSegments - 1) * kWalkPixels +
                                       64 * band0 + lane
                                 : nullptr;
@@ -180,7 +185,7 @@ __device__ __forceinline__ void composite_tile(const CompositeArgs& a, float4 (*
           walk_count == 0 ? make_float4(T[0], cr[0], cg[0], cb[0]) : make_float4(T[0], pr, pg, pb);
       pr = pg = pb = 0.0f;
       ++walk_count;
-      walk_next = walk_count + 1 < kWalkSegments ? walk_bound(walk_count + 1) : -1;
+      walk_next = walk_count + 1 < kWalkSegments ? walk_bound(walk_count + 1, a.list_shift, a.long_lists) : -1;
     }
   };
   // The overlap test's rectangle: the columns and rows of the pixels still
@@ -215,7 +220,7 @@ __device__ __forceinline__ void composite_tile(const CompositeArgs& a, float4 (*
   // still active, stored for each of the bands (vector stores).
   auto store_hits = [&](uint64_t mask, int64_t base) {
     if constexpr (HITS) {
-      const int64_t w0 = hit_mask_slot(start, tile, (base - start) >> 6) * kBands + band0;
+      const int64_t w0 = hit_mask_slot(start, list, (base - start) >> 6, subs, sub) * kBands + band0;
       if (lane < PIX && w0 + lane < a.hit_capacity) a.hit_masks[w0 + lane] = mask;
     }
   };
@@ -515,13 +520,13 @@ extern "C" GS_API size_t gs_composite_checkpoint_bytes(gs_view view, int64_t num
   if (view.tile_size > 16) return 0;  // 16 pixels per lane leave no registers for them
   const Mosaic m = mosaic_of(view);
   if (dispatch_plan(m.num_tiles(), view.tile_size, view.active_tiles, false).split_all) return 0;
-  return checkpoint_layout(nullptr, view.tile_size, num_intersections).bytes;
+  return checkpoint_layout(nullptr, view.tile_size, num_intersections, m.subs()).bytes;
 }
 
 extern "C" GS_API size_t gs_composite_hit_mask_bytes(gs_view view, int64_t num_intersections) {
   if (check_view(view, true) != GS_OK || num_intersections < 0) return 0;
   const Mosaic m = mosaic_of(view);
-  return size_t(hit_mask_words(num_intersections, m.num_tiles(), view.tile_size)) * 8;
+  return size_t(hit_mask_words(num_intersections, m.num_lists(), m.subs(), view.tile_size)) * 8;
 }
 
 namespace {
@@ -555,6 +560,7 @@ int composite(const void* records, int64_t num_records, const int32_t* gaussian_
   a.view_tw = m.tw;
   a.view_th = m.th;
   a.cols = m.cols;
+  a.list_shift = m.shift;
   a.views = m.views;
   a.threshold = view.opacity_threshold;
   a.t_active = float(1.0 - double(view.opacity_threshold));
@@ -580,11 +586,13 @@ int composite(const void* records, int64_t num_records, const int32_t* gaussian_
   a.tile_keys = plan.split_all ? nullptr : tile_keys;
   a.walk_records = plan.split_all ? static_cast<float4*>(walk_records) : nullptr;
   a.quarter_keys = quarter_keys;
+  a.long_lists = longest_list > kCheckpointMinList;
   a.deal_shift = a.num_tiles <= kDealTiles ? kDealShift : -1;
   if (hit_masks) {
     GS_REQUIRE(view.rendering_mode == GS_MODE_GAUSSIAN, GS_ERR_UNSUPPORTED,
                "hit masks are recorded for Gaussian rendering only (its backward reads them)");
-    const int64_t words = hit_mask_words(num_intersections, a.num_tiles, view.tile_size);
+    const int64_t words =
+        hit_mask_words(num_intersections, m.num_lists(), m.subs(), view.tile_size);
     GS_REQUIRE(hit_mask_bytes >= size_t(words) * 8, GS_ERR_WORKSPACE,
                "hit mask buffer too small (%zu bytes, need %zu)", hit_mask_bytes,
                size_t(words) * 8);
@@ -595,7 +603,8 @@ int composite(const void* records, int64_t num_records, const int32_t* gaussian_
   hipStream_t s = as_stream(stream);
   if (checkpoints) {
     const CheckpointLayout c =
-        checkpoint_layout(checkpoints, view.tile_size, num_intersections, checkpoint_bytes);
+        checkpoint_layout(checkpoints, view.tile_size, num_intersections, m.subs(),
+                          checkpoint_bytes);
     GS_REQUIRE(checkpoint_bytes >= c.header_bytes, GS_ERR_WORKSPACE,
                "checkpoint buffer too small (%zu bytes, need at least %zu)", checkpoint_bytes,
                c.header_bytes);
@@ -668,8 +677,8 @@ extern "C" GS_API size_t gs_composite_walk_bytes(gs_view view) {
 
 extern "C" GS_API int gs_composite_walk(
     const void* records, int64_t num_records, const int32_t* gaussian_ids,
-    int64_t num_intersections, const int64_t* ranges, gs_view view, float* image,
-    float* final_transmittance, int32_t* n_contributors, uint64_t* hit_masks,
+    int64_t num_intersections, int64_t longest_list, const int64_t* ranges, gs_view view,
+    float* image, float* final_transmittance, int32_t* n_contributors, uint64_t* hit_masks,
     size_t hit_mask_bytes, void* walk, size_t walk_bytes, void* stream) {
   clear_error();
   const size_t need = gs_composite_walk_bytes(view);
@@ -683,7 +692,7 @@ extern "C" GS_API int gs_composite_walk(
              "the walk buffer must be 16-byte aligned");
   int32_t* keys = reinterpret_cast<int32_t*>(static_cast<char*>(walk) +
                                              walk_record_bytes(mosaic_of(view).num_tiles()));
-  return composite(records, num_records, gaussian_ids, num_intersections, 0, ranges, nullptr, view,
-                   image, final_transmittance, n_contributors, nullptr, 0, hit_masks,
+  return composite(records, num_records, gaussian_ids, num_intersections, longest_list, ranges,
+                   nullptr, view, image, final_transmittance, n_contributors, nullptr, 0, hit_masks,
                    hit_mask_bytes, nullptr, 0, walk, keys, stream);
 }

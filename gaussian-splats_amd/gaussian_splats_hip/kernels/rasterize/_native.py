@@ -15,7 +15,7 @@ from pathlib import Path
 import torch
 
 LIB_PATH = Path(__file__).resolve().parents[2] / "_lib" / "libgs_raster.so"
-ABI_VERSION = 18
+ABI_VERSION = 19
 
 GS_OK = 0
 GS_ERR_INVALID_ARGUMENT = 1
@@ -60,6 +60,7 @@ class GsView(ctypes.Structure):
         ("views", c_int32),
         ("mosaic_cols", c_int32),
         ("active_tiles", c_int32),
+        ("list_shift", c_int32),
     ]
 
 
@@ -80,6 +81,7 @@ def make_view(
     views: int = 1,
     mosaic_cols: int = 1,
     active_tiles: int = 0,
+    list_shift: int = 0,
 ) -> GsView:
     if rendering_mode not in MODES:
         raise ValueError(f"Invalid rendering mode: {rendering_mode}")
@@ -87,7 +89,7 @@ def make_view(
         float(fx), float(fy), float(cx), float(cy), int(image_width), int(image_height),
         int(tile_size), float(near), float(far), MODES[rendering_mode], float(confidence),
         float(opacity_threshold), float(covariance_epsilon), int(views), int(mosaic_cols),
-        int(active_tiles),
+        int(active_tiles), int(list_shift),
     )
 
 
@@ -308,12 +310,12 @@ _SIGNATURES = {
         c_int,
         [c_void_p, c_int64] + [c_void_p] * 6
         + [GsView, c_void_p, c_void_p, c_size_t, c_int64, c_void_p, c_size_t, c_void_p, c_size_t,
-           c_void_p],
+           c_int64, c_void_p],
     ),
     "gs_composite_walk_bytes": (c_size_t, [GsView]),
     "gs_composite_walk": (
         c_int,
-        [c_void_p, c_int64, c_void_p, c_int64, c_void_p, GsView] + [c_void_p] * 4
+        [c_void_p, c_int64, c_void_p, c_int64, c_int64, c_void_p, GsView] + [c_void_p] * 4
         + [c_size_t, c_void_p, c_size_t, c_void_p],
     ),
     "gs_device_errors": (c_int, [c_void_p, c_int32, c_void_p]),

@@ -47,6 +47,11 @@ def mosaic_columns(views: int, tiles_w: int, tiles_h: int) -> int:
     return best
 
 
+#: The compositing calls split each tile over four waves below this many tiles
+#: with work (kCompositeSplitTiles), and record checkpoints on lists above this
+#: length (kCheckpointMinList).
+SPLIT_TILES, LONG_LIST = 4096, 8192
+
 #: Tile sizes the op takes; any other goes to it, which refuses it.
 OP_TILES = (4, 8, 16, 32)
 
@@ -70,27 +75,49 @@ def image_tile(asked: int, width: int, height: int, n: int, views: int = 1) -> i
 
 
 class ImageRequest:
-    """Everything but the Gaussians of an image call: the cameras in host
-    memory ([V, 9], [V, 3], [V, 4]), the view and the scalars."""
+    """Everything but the Gaussians of an image call on ``n`` of them: the
+    cameras in host memory ([V, 9], [V, 3], [V, 4]), the views and the scalars.
 
-    __slots__ = ("rotations", "translations", "intrinsics", "view", "views", "tiles", "near",
-                 "far", "gaussian")
+    The lists are those of ``tiles`` = (width, height) list tiles, laid out by
+    ``list_view``; the compositing tiles by ``view``.  ``small``: the bytes of a
+    small scene's lists' workspace, or 0.
 
-    def __init__(self, rotations, translations, intrinsics, width, height, tile, threshold, near,
-                 far, rendering_mode, confidence):
+    In a single view of many tiles 2 x 2 compositing tiles share a list
+    (the views' ``list_shift``).  A walk ends where its pixels are opaque, mostly long before
+    the list does (1M Gaussians at 1080p: after 126 of 1535 entries), so most
+    entries are placed and never read; half of the rows and columns are about
+    half of the entries to place, while a tile tests about twice the entries it
+    walks.  1M at 1080p: 642 -> 613 us a step, 4M in a small cube: 2432 -> 1961,
+    200k at 1080p: 525 -> 513.  With fewer tiles the walks, not the placing, set
+    the time (800k at 800 x 600: +5%, 300k in a small cube at 800 x 800: +86%),
+    and 16 views of 2500 tiles, which walk a quarter of their lists, gained
+    nothing."""
+
+    __slots__ = ("rotations", "translations", "intrinsics", "view", "list_view", "views", "tiles",
+                 "near", "far", "gaussian", "small")
+
+    def __init__(self, n, rotations, translations, intrinsics, width, height, tile, threshold,
+                 near, far, rendering_mode, confidence):
         self.views = rotations.shape[0]
         self.rotations = nat.host_floats(rotations, 9 * self.views, "camera_rotations")
         self.translations = nat.host_floats(translations, 3 * self.views, "camera_translations")
         self.intrinsics = nat.host_floats(intrinsics, 4 * self.views, "intrinsics")
         tw, th = nat.tiles(width, height, tile)
+        shift = int(tile == 16 and self.views == 1 and tw * th >= SPLIT_TILES)
+        tw, th = nat.tiles(width, height, tile << shift)
         cols = mosaic_columns(self.views, tw, th)
         self.tiles = (cols * tw, -(-self.views // cols) * th)
+        self.small = nat.library().gs_small_lists_bytes(n * self.views, *self.tiles)
         self.near, self.far = near, far
         self.gaussian = rendering_mode == "gaussian"
-        self.view = nat.make_view(
-            1.0, 1.0, 0.0, 0.0, width, height, tile, near, far, rendering_mode, confidence,
-            opacity_threshold=threshold, views=self.views, mosaic_cols=cols,
-        )
+
+        def view(tile, shift):
+            return nat.make_view(
+                1.0, 1.0, 0.0, 0.0, width, height, tile, near, far, rendering_mode, confidence,
+                opacity_threshold=threshold, views=self.views, mosaic_cols=cols, list_shift=shift,
+            )
+
+        self.list_view, self.view = view(tile << shift, 0), view(tile, shift)
 
     def cameras(self):
         return (c_void_p(self.rotations.data_ptr()), c_void_p(self.translations.data_ptr()),
@@ -100,7 +127,7 @@ class ImageRequest:
 class _Walk:
     """What the forward keeps for its backward beside the saved tensors."""
 
-    __slots__ = ("view", "accumulator", "checkpoints", "hits", "order", "records")
+    __slots__ = ("view", "accumulator", "checkpoints", "hits", "order", "records", "longest")
 
 
 def small_lists(depth_keys, tile_rects, tiles_w, tiles_h, nbytes, clear=None):
@@ -146,7 +173,8 @@ def forward_image(params, request: ImageRequest, keep: bool, timer=None):
     nat.check(
         nat.launch("project", lambda: lib.gs_project_image(
             ptr(mean), ptr(rotation), ptr(scale), ptr(opacity), ptr(color), n, color.shape[1],
-            *request.cameras(), view, ptr(records), ptr(depth_keys), ptr(tile_rects), stream,
+            *request.cameras(), request.list_view, ptr(records), ptr(depth_keys),
+            ptr(tile_rects), stream,
         )),
         "project_image",
     )
@@ -154,9 +182,9 @@ def forward_image(params, request: ImageRequest, keep: bool, timer=None):
     backward = keep and request.gaussian
     # The backward's [V N, 9] gradient accumulator, zeroed beside the depth sort.
     accumulator = (torch.empty((vn, 9), dtype=torch.float32, device=device) if backward else None)
-    small = lib.gs_small_lists_bytes(vn, tiles_w, tiles_h)
-    if small:
-        ids, ranges = small_lists(depth_keys, tile_rects, tiles_w, tiles_h, small, accumulator)
+    if request.small:
+        ids, ranges = small_lists(depth_keys, tile_rects, tiles_w, tiles_h, request.small,
+                                  accumulator)
         longest = 0  # unknown to the host; too few Gaussians or tiles for checkpoints
         mark("bin")
         mark("emit")
@@ -167,8 +195,14 @@ def forward_image(params, request: ImageRequest, keep: bool, timer=None):
         )
         longest = nat.longest_list(ranges)
     mark("sort")
-    view.active_tiles = nat.active_tiles(ranges)
-    num_tiles, total = tiles_w * tiles_h, ids.numel()
+    subs = 1 << (2 * view.list_shift)  # compositing tiles per list
+    active = nat.active_tiles(ranges) * subs
+    # With long lists the longest walk sets the time of a launch: tiles are
+    # split over four waves however many there are (4M Gaussians in a small cube,
+    # 4264 tiles with work: 355 + 646 us forward and backward with a wave per
+    # tile and checkpoints, 323 + 362 with four).
+    view.active_tiles = min(active, SPLIT_TILES - 1) if longest > LONG_LIST else active
+    num_tiles, total = tiles_w * tiles_h * subs, ids.numel()
     image = torch.empty((views, height, width, 3), dtype=torch.float32, device=device)
     checkpoints = nat.checkpoint_buffer(view, total, longest, device)
     # With long lists the longest walks start first (as composite does).
@@ -189,6 +223,7 @@ def forward_image(params, request: ImageRequest, keep: bool, timer=None):
     hits = nat.hit_mask_buffer(view, total, device)
     walk = _Walk()
     walk.order = walk.records = None
+    walk.longest = longest
     walk_bytes = lib.gs_composite_walk_bytes(view)
     if walk_bytes:
         # Few tiles: the walk's state at fixed positions, for a backward in
@@ -196,7 +231,7 @@ def forward_image(params, request: ImageRequest, keep: bool, timer=None):
         walk.records = nat.workspace(walk_bytes, device)
         nat.check(
             nat.launch("composite", lambda: lib.gs_composite_walk(
-                ptr(records), vn, ptr(ids), total, ptr(ranges), view, ptr(image),
+                ptr(records), vn, ptr(ids), total, longest, ptr(ranges), view, ptr(image),
                 ptr(final_transmittance), ptr(n_contributors), ptr(hits), nat.buffer_bytes(hits),
                 ptr(walk.records), walk_bytes, stream,
             )),
@@ -255,7 +290,7 @@ def backward_image(params, saved, walk: _Walk, request: ImageRequest, grad_image
             ptr(final_transmittance), ptr(n_contributors), ptr(walk.order), walk.view,
             ptr(accumulator), ptr(walk.checkpoints), nat.buffer_bytes(walk.checkpoints),
             ids.numel(), ptr(walk.hits), nat.buffer_bytes(walk.hits), ptr(walk.records),
-            nat.buffer_bytes(walk.records), stream,
+            nat.buffer_bytes(walk.records), walk.longest, stream,
         )),
         "composite_bwd_image",
     )

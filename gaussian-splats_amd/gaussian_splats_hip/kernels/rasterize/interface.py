@@ -415,7 +415,7 @@ def rasterize(
         tile = image_tile(tile_size, int(image_width), int(image_height), mean.shape[0])
         if tile is not None:
             request = ImageRequest(
-                camera_rotation[None], camera_translation[None],
+                mean.shape[0], camera_rotation[None], camera_translation[None],
                 torch.tensor([[float(fx), float(fy), float(cx), float(cy)]]), int(image_width),
                 int(image_height), tile, float(opacity_threshold), float(near), float(far),
                 rendering_mode, float(confidence),

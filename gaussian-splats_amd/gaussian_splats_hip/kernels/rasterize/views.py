@@ -502,7 +502,7 @@ def rasterize_views(
         tile = image_tile(tile_size, width, height, params[0].shape[0], len(cameras))
         if tile is not None:
             request = ImageRequest(
-                rotations, translations, intrinsics, width, height, tile,
+                params[0].shape[0], rotations, translations, intrinsics, width, height, tile,
                 float(opacity_threshold), float(near), float(far), rendering_mode,
                 float(confidence),
             )

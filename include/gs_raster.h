@@ -42,7 +42,7 @@ extern "C" {
 
 #define GS_API __attribute__((visibility("default")))
 
-#define GS_ABI_VERSION 18
+#define GS_ABI_VERSION 19
 
 typedef enum gs_status {
   GS_OK = 0,
@@ -83,6 +83,10 @@ typedef struct gs_view {
    * when fewer than 4096 tiles have work (few or skewed tiles would leave
    * SIMDs idle behind their longest tiles); results do not depend on it. */
   int32_t active_tiles;
+  /* 1: the lists are those of 2 x 2 tiles (compositing calls with tiles of 16
+   * pixels): `ranges` covers the grid of doubled tiles, and each view's tile
+   * grid is rounded up to whole ones.  0: one list per tile. */
+  int32_t list_shift;
 } gs_view;
 
 /* ABI version of the loaded library (GS_ABI_VERSION). No counterpart in the
@@ -431,13 +435,14 @@ GS_API int gs_composite_image(
  * of 16 pixels with work, whose pixel bands are split over four waves each),
  * which also records the walk's state at fixed positions, so that
  * gs_composite_bwd_image walks each tile back in segments of all of its
- * pixels.  gs_composite_walk_bytes: the size of `walk`, or 0 when the view is
+ * pixels.  longest_list (0: unknown) sets how far apart the positions are and
+ * must be the same in both calls.  gs_composite_walk_bytes: the size of `walk`, or 0 when the view is
  * not of that kind (GS_ERR_UNSUPPORTED). */
 GS_API size_t gs_composite_walk_bytes(gs_view view);
 GS_API int gs_composite_walk(
     const void* records, int64_t num_records, const int32_t* gaussian_ids,
-    int64_t num_intersections, const int64_t* ranges, gs_view view, float* image,
-    float* final_transmittance, int32_t* n_contributors, uint64_t* hit_masks,
+    int64_t num_intersections, int64_t longest_list, const int64_t* ranges, gs_view view,
+    float* image, float* final_transmittance, int32_t* n_contributors, uint64_t* hit_masks,
     size_t hit_mask_bytes, void* walk, size_t walk_bytes, void* stream);
 
 /* Back-to-front compositing gradient, accumulated with atomics into
@@ -479,7 +484,8 @@ GS_API int gs_composite_bwd_image(
     const float* grad_image, const float* final_transmittance, const int32_t* n_contributors,
     const int32_t* tile_order, gs_view view, float* grad_projected, const void* checkpoints,
     size_t checkpoint_bytes, int64_t num_intersections, const uint64_t* hit_masks,
-    size_t hit_mask_bytes, const void* walk, size_t walk_bytes, void* stream);
+    size_t hit_mask_bytes, const void* walk, size_t walk_bytes, int64_t longest_list,
+    void* stream);
 
 /* Chain rule from grad_projected to the parameters.  Replaces project_bwd
  * (src/gaussian_splats/kernels/rasterize/project_bwd.py:8-381); gradients are

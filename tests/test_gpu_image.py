@@ -48,7 +48,7 @@ def _same_gradients(a, b):
 @pytest.mark.parametrize("mode", ["gaussian", "ellipsoid"])
 @pytest.mark.parametrize("tile", [4, 8, 16, 32])
 @pytest.mark.parametrize("kind,size", [("edge", (96, 80)), ("edge", (17, 1)), ("needle", (333, 207)),
-                                       ("cloud", (1111, 1043))])
+                                       ("cloud", (1111, 1043)), ("cloud", (1100, 1030))])
 def test_image_equals_op(kind, size, tile, mode, device):
     if kind == "needle":
         scene = _needles(3000, size)
