@@ -175,3 +175,11 @@ def test_ssim_deterministic_and_checks():
         ssim(torch.zeros(10, 30, 3, device=DEV), torch.zeros(10, 30, 3, device=DEV))
     with pytest.raises(ValueError):
         ssim(torch.zeros(30, 30, 4, device=DEV), torch.zeros(30, 30, 4, device=DEV))
+
+
+@pytest.mark.parametrize("shape", [(22, 32), (23, 33), (32, 42), (33, 43), (54, 75), (11, 107)])
+def test_ssim_at_block_edges(shape):
+    """One workgroup covers 32 x 22 outputs of the 10-pixel larger staged
+    block: images of exactly one block, one pixel more, and remainders of
+    columns and of the three-row groups (tolerances as above)."""
+    test_ssim_matches_torch_and_oracle(shape)
