@@ -108,7 +108,9 @@ __device__ __forceinline__ void composite_bwd_tile(const CompositeBwdArgs& a, fl
   if (view >= a.views) return;  // an empty slot of the mosaic's last row
   // WALK: nothing to do for a segment past the tile's largest contributor count.
   const int walk_lo = WALK ? walk_bound(seg, a.list_shift, a.long_lists) : 0;
-  const int walk_hi = WALK && seg + 1 < kWalkSegments ? walk_bound(seg + 1, a.list_shift, a.long_lists) : INT_MAX;
+  const int walk_hi = WALK && seg + 1 < kWalkSegments
+                          ? walk_bound(seg + 1, a.list_shift, a.long_lists)
+                          : INT_MAX;
   if constexpr (WALK) {
     const int4 n4 = reinterpret_cast<const int4*>(a.quarter_keys)[tile];
     if (max(max(n4.x, n4.y), max(n4.z, n4.w)) <= walk_lo) return;
@@ -636,10 +638,9 @@ extern "C" GS_API int gs_composite_bwd(const float* projected_mean,
 extern "C" GS_API int gs_composite_bwd_image(
     const void* records, int64_t n, const int32_t* gaussian_ids, const int64_t* ranges,
     const float* grad_image, const float* final_transmittance, const int32_t* n_contributors,
-    const int32_t* tile_order, gs_view view, float* grad_projected, const void* checkpoints,
-    size_t checkpoint_bytes, int64_t num_intersections, const uint64_t* hit_masks,
-    size_t hit_mask_bytes, const void* walk, size_t walk_bytes, int64_t longest_list,
-    void* stream) {
+    const int32_t* tile_order, gs_view view, float* grad_projected, int64_t num_intersections,
+    const uint64_t* hit_masks, size_t hit_mask_bytes, const void* walk, size_t walk_bytes,
+    int64_t longest_list, void* stream) {
   clear_error();
   GS_REQUIRE(view.tile_size >= 16, GS_ERR_UNSUPPORTED,
              "image calls composite tiles of 16 or 32 pixels (got %d)", view.tile_size);
@@ -647,6 +648,6 @@ extern "C" GS_API int gs_composite_bwd_image(
   return composite_bwd(nullptr, nullptr, nullptr, nullptr,
                        static_cast<const GsRecord*>(records), n, gaussian_ids, ranges, grad_image,
                        final_transmittance, n_contributors, tile_order, view, grad_projected,
-                       nullptr, checkpoints, checkpoint_bytes, num_intersections, hit_masks,
-                       hit_mask_bytes, walk, walk_bytes, longest_list, stream);
+                       nullptr, nullptr, 0, num_intersections, hit_masks, hit_mask_bytes, walk,
+                       walk_bytes, longest_list, stream);
 }

@@ -33,7 +33,6 @@ struct CompositeArgs {
   const int32_t* items;  // dispatch plan (gs_tile_order), or nullptr: tiles in index order
   int num_items;
   bool split_all;        // without a plan: every tile split into quarters
-  bool long_walk;        // the CKPT kernel (tiles of at most 16 pixels)
   int width, height, tile;  // per view
   int tiles_w, num_tiles;    // of the whole mosaic
   int list_shift;            // lists of 2 x 2 tiles (gs_view.list_shift)
@@ -174,10 +173,12 @@ __device__ __forceinline__ void composite_tile(const CompositeArgs& a, float4 (*
   constexpr bool kRecords = HITS && TILE == 16 && PIX == 1;
   int walk_count = 0, walk_next = -1;
   float pr = 0.0f, pg = 0.0f, pb = 0.0f;
-  if constexpr (kRecords) walk_next = a.walk_records ? walk_bound(1, a.list_shift, a.long_lists) : -1;
-  float4* const walk = kRecords ? a.walk_records + int64_t(tile) * (kWalkSegments - 1) * kWalkPixels +
-                                      64 * band0 + lane
-                                : nullptr;
+  if constexpr (kRecords)
+    walk_next = a.walk_records ? walk_bound(1, a.list_shift, a.long_lists) : -1;
+  float4* const walk =
+      kRecords ? a.walk_records + int64_t(tile) * (kWalkSegments - 1) * kWalkPixels + 64 * band0 +
+                     lane
+               : nullptr;
   auto record_at = [&](int bpos) {
     if constexpr (kRecords) {
       if (bpos != walk_next) return;
@@ -185,7 +186,9 @@ __device__ __forceinline__ void composite_tile(const CompositeArgs& a, float4 (*
           walk_count == 0 ? make_float4(T[0], cr[0], cg[0], cb[0]) : make_float4(T[0], pr, pg, pb);
       pr = pg = pb = 0.0f;
       ++walk_count;
-      walk_next = walk_count + 1 < kWalkSegments ? walk_bound(walk_count + 1, a.list_shift, a.long_lists) : -1;
+      walk_next = walk_count + 1 < kWalkSegments
+                      ? walk_bound(walk_count + 1, a.list_shift, a.long_lists)
+                      : -1;
     }
   };
   // The overlap test's rectangle: the columns and rows of the pixels still
@@ -418,9 +421,9 @@ constexpr int kDealShift = 3;
 
 // kCompositeWaves waves per workgroup, one work item each (composite_item);
 // workgroups are mapped onto XCDs so that each XCD takes one region of the
-// plan (xcd_swizzle) or, without a plan, chunks of neighbours (kDealTiles).  QUARTERS: the launch's items are quarters (every tile
-// split); a whole-tile item is then composited as its four quarters in turn.
-// Otherwise items are whole tiles; of a tile split into several items the
+// plan (xcd_swizzle) or, without a plan, chunks of neighbours (kDealTiles).
+// QUARTERS: the launch's items are quarters (every tile split); a whole-tile
+// item is then composited as its four quarters in turn.  Otherwise items are whole tiles; of a tile split into several items the
 // first composites the whole tile and the others have no work.  Each kernel
 // thus composites every pixel of any plan exactly once, with one instance of
 // the walk (two would share one register allocation).
@@ -492,7 +495,7 @@ void launch(const CompositeArgs& a, bool ellipsoid, hipStream_t s) {
     if (a.split_all) return launch_items<TILE, true, false>(a, ellipsoid, s);
   }
   if constexpr (TILE <= 16) {
-    if (a.long_walk) return launch_items<TILE, false, true>(a, ellipsoid, s);
+    if (a.ckpt_counter) return launch_items<TILE, false, true>(a, ellipsoid, s);
   }
   launch_items<TILE, false, false>(a, ellipsoid, s);
 }
@@ -531,11 +534,11 @@ extern "C" GS_API size_t gs_composite_hit_mask_bytes(gs_view view, int64_t num_i
 
 namespace {
 
-// `longest_list` (0: unknown) selects the long-list walk for a call without
-// checkpoints; with them it is selected anyway.
+// `longest_list` (0: unknown) selects the bounds of the walk records.
 int composite(const void* records, int64_t num_records, const int32_t* gaussian_ids,
               int64_t num_intersections, int64_t longest_list, const int64_t* ranges,
-              const int32_t* tile_order, gs_view view, float* image, float* final_transmittance, int32_t* n_contributors,
+              const int32_t* tile_order, gs_view view, float* image,
+              float* final_transmittance, int32_t* n_contributors,
               void* checkpoints, size_t checkpoint_bytes, uint64_t* hit_masks,
               size_t hit_mask_bytes, uint32_t* tile_keys, size_t tile_keys_bytes,
               void* walk_records, int32_t* quarter_keys, void* stream) {
@@ -626,7 +629,6 @@ int composite(const void* records, int64_t num_records, const int32_t* gaussian_
     GS_TRY(check_launch("composite checkpoints"));
   }
   const bool ellipsoid = view.rendering_mode == GS_MODE_ELLIPSOID;
-  a.long_walk = a.ckpt_counter || (longest_list > kCheckpointMinList && num_records > 0);
   switch (view.tile_size) {
     case 4: launch<4>(a, ellipsoid, s); break;
     case 8: launch<8>(a, ellipsoid, s); break;
@@ -658,13 +660,11 @@ extern "C" GS_API int gs_composite(const void* records, int64_t num_records,
 
 extern "C" GS_API int gs_composite_image(const void* records, int64_t num_records,
                                          const int32_t* gaussian_ids, int64_t num_intersections,
-                                         int64_t longest_list, const int64_t* ranges,
-                                         const int32_t* tile_order, gs_view view, float* image,
+                                         const int64_t* ranges, gs_view view, float* image,
                                          void* stream) {
   clear_error();
-  GS_REQUIRE(longest_list >= 0, GS_ERR_INVALID_ARGUMENT, "negative list length");
-  return composite(records, num_records, gaussian_ids, num_intersections, longest_list, ranges,
-                   tile_order, view, image, nullptr, nullptr, nullptr, 0, nullptr, 0, nullptr, 0,
+  return composite(records, num_records, gaussian_ids, num_intersections, 0, ranges, nullptr, view,
+                   image, nullptr, nullptr, nullptr, 0, nullptr, 0, nullptr, 0,
                    nullptr, nullptr, stream);
 }
 

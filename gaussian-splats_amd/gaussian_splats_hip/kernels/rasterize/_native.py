@@ -303,14 +303,12 @@ _SIGNATURES = {
     ),
     "gs_composite_image": (
         c_int,
-        [c_void_p, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_void_p, GsView, c_void_p,
-         c_void_p],
+        [c_void_p, c_int64, c_void_p, c_int64, c_void_p, GsView, c_void_p, c_void_p],
     ),
     "gs_composite_bwd_image": (
         c_int,
         [c_void_p, c_int64] + [c_void_p] * 6
-        + [GsView, c_void_p, c_void_p, c_size_t, c_int64, c_void_p, c_size_t, c_void_p, c_size_t,
-           c_int64, c_void_p],
+        + [GsView, c_void_p, c_int64, c_void_p, c_size_t, c_void_p, c_size_t, c_int64, c_void_p],
     ),
     "gs_composite_walk_bytes": (c_size_t, [GsView]),
     "gs_composite_walk": (

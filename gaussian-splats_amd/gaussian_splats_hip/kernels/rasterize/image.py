@@ -48,8 +48,8 @@ def mosaic_columns(views: int, tiles_w: int, tiles_h: int) -> int:
 
 
 #: The compositing calls split each tile over four waves below this many tiles
-#: with work (kCompositeSplitTiles), and record checkpoints on lists above this
-#: length (kCheckpointMinList).
+#: with work (kCompositeSplitTiles); lists above this length count as long
+#: (kCheckpointMinList: whole-tile walks would record checkpoints on them).
 SPLIT_TILES, LONG_LIST = 4096, 8192
 
 #: Tile sizes the op takes; any other goes to it, which refuses it.
@@ -60,10 +60,11 @@ def image_tile(asked: int, width: int, height: int, n: int, views: int = 1) -> i
     """Tile size of an image call for which the caller ``asked`` one the op
     takes, or None when the op itself has to run: it refuses the size, or
     row/column bucketing takes neither grid (the op's other binning then runs,
-    with the caller's tile size).  16 pixels: smaller tiles leave lanes of the compositing waves idle
-    and list a Gaussian many times over (200k Gaussians at 1080p, forward and
-    backward: 3.77 ms with the default tile size 4, 0.55 ms with 16); 32 where
-    the grid of 16-pixel tiles is larger than bucketing takes."""
+    with the caller's tile size).  16 pixels: smaller tiles leave lanes of the
+    compositing waves idle and list a Gaussian many times over (200k Gaussians
+    at 1080p, forward and backward: 3.65 ms with the default tile size 4, 0.52 ms
+    with 16); 32 where the grid of 16-pixel tiles is larger than bucketing
+    takes."""
     if asked not in OP_TILES or width <= 0 or height <= 0 or views * n >= MAX_BUCKET_GAUSSIANS:
         return None
     for tile in (16, 32):
@@ -82,8 +83,8 @@ class ImageRequest:
     ``list_view``; the compositing tiles by ``view``.  ``small``: the bytes of a
     small scene's lists' workspace, or 0.
 
-    In a single view of many tiles 2 x 2 compositing tiles share a list
-    (the views' ``list_shift``).  A walk ends where its pixels are opaque, mostly long before
+    In a single view of many tiles 2 x 2 compositing tiles share a list (the
+    views' ``list_shift``).  A walk ends where its pixels are opaque, mostly long before
     the list does (1M Gaussians at 1080p: after 126 of 1535 entries), so most
     entries are placed and never read; half of the rows and columns are about
     half of the entries to place, while a tile tests about twice the entries it
@@ -127,7 +128,7 @@ class ImageRequest:
 class _Walk:
     """What the forward keeps for its backward beside the saved tensors."""
 
-    __slots__ = ("view", "accumulator", "checkpoints", "hits", "order", "records", "longest")
+    __slots__ = ("view", "accumulator", "hits", "order", "records", "longest")
 
 
 def small_lists(depth_keys, tile_rects, tiles_w, tiles_h, nbytes, clear=None):
@@ -204,15 +205,10 @@ def forward_image(params, request: ImageRequest, keep: bool, timer=None):
     view.active_tiles = min(active, SPLIT_TILES - 1) if longest > LONG_LIST else active
     num_tiles, total = tiles_w * tiles_h * subs, ids.numel()
     image = torch.empty((views, height, width, 3), dtype=torch.float32, device=device)
-    checkpoints = nat.checkpoint_buffer(view, total, longest, device)
-    # With long lists the longest walks start first (as composite does).
-    plan = (nat.dispatch_plan(view, num_tiles, device, ranges=ranges)
-            if checkpoints is not None else None)
     if not backward:
         nat.check(
             nat.launch("composite", lambda: lib.gs_composite_image(
-                ptr(records), vn, ptr(ids), total, longest, ptr(ranges), ptr(plan), view,
-                ptr(image), stream,
+                ptr(records), vn, ptr(ids), total, ptr(ranges), view, ptr(image), stream,
             )),
             "composite_image",
         )
@@ -242,10 +238,9 @@ def forward_image(params, request: ImageRequest, keep: bool, timer=None):
         keys = nat.workspace(lib.gs_tile_order_workspace_bytes(num_tiles), device)
         nat.check(
             nat.launch("composite", lambda: lib.gs_composite(
-                ptr(records), vn, ptr(ids), total, ptr(ranges), ptr(plan), view, ptr(image),
-                ptr(final_transmittance), ptr(n_contributors), ptr(checkpoints),
-                nat.buffer_bytes(checkpoints), ptr(hits), nat.buffer_bytes(hits), ptr(keys),
-                keys.numel(), stream,
+                ptr(records), vn, ptr(ids), total, ptr(ranges), None, view, ptr(image),
+                ptr(final_transmittance), ptr(n_contributors), None, 0, ptr(hits),
+                nat.buffer_bytes(hits), ptr(keys), keys.numel(), stream,
             )),
             "composite",
         )
@@ -258,7 +253,7 @@ def forward_image(params, request: ImageRequest, keep: bool, timer=None):
                               keys.numel(), 1, stream),
             "tile_order",
         )
-    walk.view, walk.accumulator, walk.checkpoints, walk.hits = view, accumulator, checkpoints, hits
+    walk.view, walk.accumulator, walk.hits = view, accumulator, hits
     return image, (records, tile_rects, ids, ranges, final_transmittance, n_contributors), walk
 
 
@@ -288,8 +283,7 @@ def backward_image(params, saved, walk: _Walk, request: ImageRequest, grad_image
         nat.launch("composite_bwd", lambda: lib.gs_composite_bwd_image(
             ptr(records), records.shape[0], ptr(ids), ptr(ranges), ptr(grad_image),
             ptr(final_transmittance), ptr(n_contributors), ptr(walk.order), walk.view,
-            ptr(accumulator), ptr(walk.checkpoints), nat.buffer_bytes(walk.checkpoints),
-            ids.numel(), ptr(walk.hits), nat.buffer_bytes(walk.hits), ptr(walk.records),
+            ptr(accumulator), ids.numel(), ptr(walk.hits), nat.buffer_bytes(walk.hits), ptr(walk.records),
             nat.buffer_bytes(walk.records), walk.longest, stream,
         )),
         "composite_bwd_image",

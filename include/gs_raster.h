@@ -422,22 +422,19 @@ GS_API int gs_composite(
     size_t tile_keys_bytes, void* stream);
 
 /* gs_composite for a caller that wants the image alone: no transmittance,
- * contributor counts or state for a backward.  longest_list: the longest of
- * the lists (totals[3] of gs_bin_tiles_plan), or 0 when unknown; long lists
- * take the walk of two batches per step that records checkpoints for
- * gs_composite's caller. */
+ * contributor counts or state for a backward. */
 GS_API int gs_composite_image(
     const void* records, int64_t num_records, const int32_t* gaussian_ids,
-    int64_t num_intersections, int64_t longest_list, const int64_t* ranges,
-    const int32_t* tile_order, gs_view view, float* image, void* stream);
+    int64_t num_intersections, const int64_t* ranges, gs_view view, float* image, void* stream);
 
 /* gs_composite for a Gaussian image call on few tiles (fewer than 4096 tiles
  * of 16 pixels with work, whose pixel bands are split over four waves each),
  * which also records the walk's state at fixed positions, so that
  * gs_composite_bwd_image walks each tile back in segments of all of its
- * pixels.  longest_list (0: unknown) sets how far apart the positions are and
- * must be the same in both calls.  gs_composite_walk_bytes: the size of `walk`, or 0 when the view is
- * not of that kind (GS_ERR_UNSUPPORTED). */
+ * pixels.  longest_list (totals[3] of gs_bin_tiles_plan, 0: unknown) sets how
+ * far apart the positions are and must be the same in both calls.
+ * gs_composite_walk_bytes: the size of `walk`, or 0 when the view is not of
+ * that kind (GS_ERR_UNSUPPORTED). */
 GS_API size_t gs_composite_walk_bytes(gs_view view);
 GS_API int gs_composite_walk(
     const void* records, int64_t num_records, const int32_t* gaussian_ids,
@@ -482,10 +479,9 @@ GS_API int gs_composite_bwd(
 GS_API int gs_composite_bwd_image(
     const void* records, int64_t n, const int32_t* gaussian_ids, const int64_t* ranges,
     const float* grad_image, const float* final_transmittance, const int32_t* n_contributors,
-    const int32_t* tile_order, gs_view view, float* grad_projected, const void* checkpoints,
-    size_t checkpoint_bytes, int64_t num_intersections, const uint64_t* hit_masks,
-    size_t hit_mask_bytes, const void* walk, size_t walk_bytes, int64_t longest_list,
-    void* stream);
+    const int32_t* tile_order, gs_view view, float* grad_projected, int64_t num_intersections,
+    const uint64_t* hit_masks, size_t hit_mask_bytes, const void* walk, size_t walk_bytes,
+    int64_t longest_list, void* stream);
 
 /* Chain rule from grad_projected to the parameters.  Replaces project_bwd
  * (src/gaussian_splats/kernels/rasterize/project_bwd.py:8-381); gradients are
