@@ -1,6 +1,7 @@
 // C-ABI bookkeeping: per-thread error text, version, argument validation,
 // the side streams used to overlap independent stages, and the per-device
 // word of device-side check failures.
+#include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <mutex>
@@ -190,6 +191,25 @@ GS_API int gs_device_errors(uint32_t* flags, int32_t clear, void* stream) {
 }
 
 GS_API int gs_abi_version(void) { return GS_ABI_VERSION; }
+
+GS_API int gs_camera_rotation(float w, float x, float y, float z, float* rotation) {
+#pragma clang fp contract(off)
+  gs::clear_error();
+  GS_REQUIRE(rotation, GS_ERR_INVALID_ARGUMENT, "null pointer argument");
+  float norm = std::sqrt(((w * w + x * x) + y * y) + z * z);
+  if (norm < 1e-12f) norm = 1e-12f;  // NaN stays
+  w /= norm;
+  x /= norm;
+  y /= norm;
+  z /= norm;
+  const float xx = x * x, yy = y * y, zz = z * z;
+  const float rows[9] = {
+      1.0f - 2.0f * (yy + zz),       2.0f * (x * y - w * z),        2.0f * (x * z + w * y),
+      2.0f * (x * y + w * z),        1.0f - 2.0f * (xx + zz),       2.0f * (y * z - w * x),
+      2.0f * (x * z - w * y),        2.0f * (y * z + w * x),        1.0f - 2.0f * (xx + yy)};
+  std::copy(rows, rows + 9, rotation);
+  return GS_OK;
+}
 
 GS_API int gs_arm_launch_events(void* start, void* stop) {
   gs::clear_error();

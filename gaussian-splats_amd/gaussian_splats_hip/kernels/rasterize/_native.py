@@ -223,6 +223,7 @@ def buffer_bytes(t: torch.Tensor | None) -> int:
 _SIGNATURES = {
     "gs_abi_version": (c_int, []),
     "gs_last_error": (ctypes.c_char_p, []),
+    "gs_camera_rotation": (c_int, [c_float] * 4 + [c_void_p]),
     "gs_arm_launch_events": (c_int, [c_void_p, c_void_p]),
     "gs_disarm_launch_events": (c_int, []),
     "gs_project_and_count": (
@@ -441,7 +442,11 @@ def ptr(t: torch.Tensor | None) -> c_void_p:
 
 
 def stream(device: torch.device) -> c_void_p:
-    return c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    """The handle of torch's current stream on ``device``, without the Stream
+    object that torch.cuda.current_stream builds (0.2 us instead of 2, several
+    times a call)."""
+    index = device.index if device.index is not None else torch.cuda.current_device()
+    return c_void_p(torch._C._cuda_getCurrentRawStream(index))
 
 
 def require_gpu(*tensors: torch.Tensor) -> torch.device:

@@ -21,7 +21,7 @@ their sums.  Traced calls (``torch.compile``) use the registered op.
 
 from __future__ import annotations
 
-from ctypes import c_void_p
+from ctypes import addressof
 
 import torch
 
@@ -77,7 +77,8 @@ def image_tile(asked: int, width: int, height: int, n: int, views: int = 1) -> i
 
 class ImageRequest:
     """Everything but the Gaussians of an image call on ``n`` of them: the
-    cameras in host memory ([V, 9], [V, 3], [V, 4]), the views and the scalars.
+    ``cameras`` (``camera_floats`` of ``views`` of them), the views and the
+    scalars.
 
     The lists are those of ``tiles`` = (width, height) list tiles, laid out by
     ``list_view``; the compositing tiles by ``view``.  ``small``: the bytes of a
@@ -94,15 +95,12 @@ class ImageRequest:
     and 16 views of 2500 tiles, which walk a quarter of their lists, gained
     nothing."""
 
-    __slots__ = ("rotations", "translations", "intrinsics", "view", "list_view", "views", "tiles",
-                 "near", "far", "gaussian", "small")
+    __slots__ = ("floats", "view", "list_view", "views", "tiles", "near", "far", "gaussian",
+                 "small")
 
-    def __init__(self, n, rotations, translations, intrinsics, width, height, tile, threshold,
-                 near, far, rendering_mode, confidence):
-        self.views = rotations.shape[0]
-        self.rotations = nat.host_floats(rotations, 9 * self.views, "camera_rotations")
-        self.translations = nat.host_floats(translations, 3 * self.views, "camera_translations")
-        self.intrinsics = nat.host_floats(intrinsics, 4 * self.views, "intrinsics")
+    def __init__(self, n, cameras, views, width, height, tile, threshold, near, far,
+                 rendering_mode, confidence):
+        self.views, self.floats = views, cameras
         tw, th = nat.tiles(width, height, tile)
         shift = int(tile == 16 and self.views == 1 and tw * th >= SPLIT_TILES)
         tw, th = nat.tiles(width, height, tile << shift)
@@ -118,11 +116,13 @@ class ImageRequest:
                 opacity_threshold=threshold, views=self.views, mosaic_cols=cols, list_shift=shift,
             )
 
-        self.list_view, self.view = view(tile << shift, 0), view(tile, shift)
+        self.view = view(tile, shift)
+        self.list_view = view(tile << shift, 0) if shift else self.view
 
     def cameras(self):
-        return (c_void_p(self.rotations.data_ptr()), c_void_p(self.translations.data_ptr()),
-                c_void_p(self.intrinsics.data_ptr()))
+        """The three arrays of ``floats``: rotations, translations, intrinsics."""
+        base = addressof(self.floats)
+        return base, base + 36 * self.views, base + 48 * self.views
 
 
 class _Walk:

@@ -408,20 +408,19 @@ def rasterize(
             color[indices],
         )
     # Extrinsics stay in host memory: the kernels take them as arguments.
-    from ...splats.camera import host_extrinsics  # the splat API imports this module
+    from ...splats.camera import camera_floats, host_extrinsics  # they import this module
 
-    camera_rotation, camera_translation = host_extrinsics(camera)
     if not torch.compiler.is_compiling():
         tile = image_tile(tile_size, int(image_width), int(image_height), mean.shape[0])
         if tile is not None:
             request = ImageRequest(
-                mean.shape[0], camera_rotation[None], camera_translation[None],
-                torch.tensor([[float(fx), float(fy), float(cx), float(cy)]]), int(image_width),
-                int(image_height), tile, float(opacity_threshold), float(near), float(far),
-                rendering_mode, float(confidence),
+                mean.shape[0], camera_floats((camera,)), 1, int(image_width), int(image_height),
+                tile, float(opacity_threshold), float(near), float(far), rendering_mode,
+                float(confidence),
             )
             return render_image((mean, rotation, scale, opacity, color), request,
                                 stage_timer())[0]
+    camera_rotation, camera_translation = host_extrinsics(camera)
     return rasterize_outputs(
         mean,
         rotation,

@@ -456,16 +456,21 @@ def rasterize_views_outputs(*inputs) -> tuple[torch.Tensor, ...]:
     return forward_views(*inputs, timer=stage_timer(), record_hits=False)
 
 
-def camera_tensors(cameras: Sequence[Camera]) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, int, int]:
-    """Host-side camera arrays of ``rasterize_views``: rotations [V, 3, 3],
-    translations [V, 3], intrinsics [V, 4] = (fx, fy, cx, cy), and the shared
-    image size."""
+def _shared_size(cameras: Sequence[Camera]) -> tuple[int, int]:
     if not cameras:
         raise ValueError("rasterize_views needs at least one camera")
     sizes = {tuple(int(s) for s in cam.image_size) for cam in cameras}
     if len(sizes) != 1:
         raise ValueError(f"all cameras must share one image size, got {sorted(sizes)}")
-    (width, height), = sizes
+    (size,) = sizes
+    return size
+
+
+def camera_tensors(cameras: Sequence[Camera]) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, int, int]:
+    """Host-side camera arrays of ``rasterize_views``: rotations [V, 3, 3],
+    translations [V, 3], intrinsics [V, 4] = (fx, fy, cx, cy), and the shared
+    image size."""
+    width, height = _shared_size(cameras)
     from ...splats.camera import host_extrinsics  # the splat API imports this module
 
     extrinsics = [host_extrinsics(cam) for cam in cameras]
@@ -494,19 +499,22 @@ def rasterize_views(
     _check_tile(tile_size)
     if rendering_mode not in ("gaussian", "ellipsoid"):
         raise ValueError(f"Invalid rendering mode: {rendering_mode}")
-    rotations, translations, intrinsics, width, height = camera_tensors(cameras)
+    width, height = _shared_size(cameras)
     params = (splats.mean, splats.rotation, splats.scale, splats.opacity, splats.color)
     if indices is not None:
         params = tuple(p[indices] for p in params)
     if not torch.compiler.is_compiling():
         tile = image_tile(tile_size, width, height, params[0].shape[0], len(cameras))
         if tile is not None:
+            from ...splats.camera import camera_floats  # the splat API imports this module
+
             request = ImageRequest(
-                params[0].shape[0], rotations, translations, intrinsics, width, height, tile,
+                params[0].shape[0], camera_floats(cameras), len(cameras), width, height, tile,
                 float(opacity_threshold), float(near), float(far), rendering_mode,
                 float(confidence),
             )
             return render_image(params, request, stage_timer())
+    rotations, translations, intrinsics, width, height = camera_tensors(cameras)
     return rasterize_views_outputs(
         *params,
         rotations,

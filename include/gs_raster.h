@@ -96,6 +96,12 @@ GS_API int gs_abi_version(void);
 /* Message describing the last failure on the calling thread ("" if none). */
 GS_API const char* gs_last_error(void);
 
+/* World-to-camera rotation (row-major [3,3], host memory) of the quaternion
+ * (w, x, y, z), normalised as F.normalize does (the norm clamped at 1e-12):
+ * float32 operations in the order of Camera.rotation_matrix
+ * (src/gaussian_splats/splats/utils.py:8-25), without device work. */
+GS_API int gs_camera_rotation(float w, float x, float y, float z, float* rotation);
+
 /* Kernel timing for benchmarks.  No counterpart in the reference (its
  * benchmark times whole calls on the host); for callers that measure one
  * kernel's duration per launch.  gs_arm_launch_events arms two hipEvent_t

@@ -125,3 +125,37 @@ def test_host_extrinsics_equal_the_torch_rotation_matrix():
                         translation=torch.randn(3, dtype=torch.float64, generator=g))
     r, t = host_extrinsics(cam)
     assert torch.equal(r, cam.rotation_matrix.float()) and t.dtype == torch.float32
+
+
+def test_camera_floats_equal_host_extrinsics():
+    """The image calls' camera array holds host_extrinsics' values bit for bit:
+    any magnitude, zeros, infinities and NaN, float64 translations, parameters
+    that need gradients, and the forms that take the tensor path."""
+    from gaussian_splats_hip.splats.camera import camera_floats, host_extrinsics
+
+    g = torch.Generator().manual_seed(12)
+    inf, nan = float("inf"), float("nan")
+    rotations = [torch.randn(4, generator=g) * 10.0 ** k for k in range(-24, 20)]
+    rotations += [torch.tensor(q) for q in ([0.0] * 4, [1e-30, 0.0, 0.0, -0.0],
+                                            [inf, 1.0, 0.0, 0.0], [nan, 1.0, 0.0, 0.0],
+                                            [1e-13, -1e-13, 0.0, 0.0])]
+    rotations += [torch.randn(1, 4, generator=g), torch.randn(4, dtype=torch.float64, generator=g),
+                  torch.randn(8, generator=g)[::2], torch.randn(4, generator=g).requires_grad_(True)]
+    cameras = []
+    for i, q in enumerate(rotations):
+        t = torch.randn(3, dtype=torch.float64 if i % 3 == 0 else torch.float32, generator=g)
+        if i % 5 == 0:
+            t = t.requires_grad_(True) * 1e30
+        cameras.append(PinholeCamera(rotation=q, translation=t, focal_length=(500.5 + i, 1 / 3),
+                                     principal_point=(i * 0.1, 2)))
+    v = len(cameras)
+    floats = np.ctypeslib.as_array(camera_floats(cameras)).copy()
+    for i, cam in enumerate(cameras):
+        with np.errstate(all="ignore"):
+            r, t = host_extrinsics(cam)
+        want = torch.cat((r.flatten(), t, torch.tensor([*cam.focal_length, *cam.principal_point])))
+        got = np.concatenate((floats[9 * i:9 * i + 9], floats[9 * v + 3 * i:][:3],
+                              floats[12 * v + 4 * i:][:4]))
+        assert np.array_equal(got, want.numpy().astype(np.float32), equal_nan=True), i
+    one = np.ctypeslib.as_array(camera_floats(cameras[:1]))
+    assert np.array_equal(one[:9], floats[:9], equal_nan=True)
