@@ -1,11 +1,14 @@
 // Tile lists of a small scene without a sort of its intersections, without
-// sizes read back by the host, in two launches:
+// sizes read back by the host, in three launches:
 //
-//  1. rank: every Gaussian counts the depth keys before its own (ties by
-//     index), so the packed rectangles are written in depth order.  n^2 / 64
-//     wave comparisons of two VALU instructions: 17 us for 10k Gaussians, 45 us
-//     for 20k, where the four passes of the depth sort take 33 and 40 and five
-//     launches.
+//  1. order: chunks of 256 depth keys are sorted (each key counts those of its
+//     chunk before it), then every Gaussian's rank is its place in its chunk
+//     plus a binary search in each other chunk (ties by index), and the packed
+//     rectangles are written in depth order.  Two launches whose chains are a
+//     few LDS reads long: 4.4 + 4.5 us for 10k Gaussians, 4.4 + 8.3 for 20k.
+//     Counting all n keys for each Gaussian took 17.4 and 46.9 us (n^2 / 64
+//     wave comparisons of two VALU instructions), the four passes of the depth
+//     sort take 33 and 40 us and five launches.
 //  2. lists: a workgroup takes four neighbouring tiles of one tile row, tests
 //     every rectangle in depth order against them (a ballot per 64 Gaussians
 //     and tile) and writes each tile's hits at the tile's own n slots.
@@ -15,8 +18,8 @@
 // its totals in between; it reads every rectangle a few times where this one
 // reads it once per four tiles, so this one is for few Gaussians on few tiles
 // (small_fits).  Lists kernel: 12 us for 10k Gaussians on 256 or 1200 tiles.
-// Frames of 10k Gaussians at 256 x 256 and 640 x 480: 178 -> 69 and 179 -> 79
-// us; a step of 20k at 403 x 307: 510 -> 365 us.
+// Frames of 10k Gaussians at 256 x 256 and 640 x 480: 178 -> 54 and 179 -> 64
+// us.
 //
 // List t is gaussian_ids[ranges[t]) in [t n, (t + 1) n): lists do not touch one
 // another, and follow one another in tile order as the compositing kernels'
@@ -29,7 +32,13 @@ namespace gs {
 namespace {
 
 constexpr int kStrip = 4;          // tiles per workgroup of the lists kernel
+constexpr int kChunk = 256;        // keys sorted by one workgroup
+constexpr int kBlocks = kChunk / 64;
 constexpr int kRankWaves = 16;
+static_assert(kRankWaves == kBlocks * kBlocks, "chunk_kernel: a wave per pair of blocks");
+// Chunks searched from LDS at a time (48 KB, so that two workgroups share a CU).
+constexpr int kRoundChunks = 48;
+constexpr int kWaveChunks = kRoundChunks / kRankWaves;
 constexpr int kListWaves = 16;
 // 16-bit ids and the strip's masks of this many Gaussians fill 63 KB of LDS.
 constexpr int64_t kSmallMax = 24576;
@@ -40,62 +49,128 @@ bool small_fits(int64_t n, int64_t tiles) {
   return n > 0 && n <= kSmallMax && tiles > 0 && n * tiles <= kSmallSlots;
 }
 
-// Workgroup b ranks Gaussians [64 b, 64 b + 64), one per lane; its waves share
-// the keys to compare with, 64 at a time, read as scalars.
+// Workgroup c sorts keys [256 c, 256 c + 256) by (key, index), past the end of
+// the array by ~0u, which come after all others of the last chunk.  Wave (i, j)
+// counts for the 64 keys of block i those of block j before them.
+__global__ __launch_bounds__(kRankWaves * 64) void chunk_kernel(
+    const uint32_t* __restrict__ keys, int n, uint32_t* __restrict__ chunk_keys,
+    uint16_t* __restrict__ chunk_ids) {
+  __shared__ __align__(16) uint32_t own[kChunk];
+  __shared__ uint32_t part[kBlocks][kChunk];
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  const int first = blockIdx.x * kChunk;
+  if (threadIdx.x < kChunk) {
+    const int g = first + int(threadIdx.x);
+    own[threadIdx.x] = g < n ? keys[g] : 0xFFFFFFFFu;
+  }
+  __syncthreads();
+  const int i = wid & (kBlocks - 1), j = wid / kBlocks;
+  const uint32_t mine = own[i * 64 + lane];
+  const uint4* block = reinterpret_cast<const uint4*>(own + j * 64);
+  uint32_t before = 0;
+  if (j < i) {
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      const uint4 k = block[q];
+      before += (k.x <= mine) + (k.y <= mine) + (k.z <= mine) + (k.w <= mine);
+    }
+  } else if (j > i) {
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      const uint4 k = block[q];
+      before += (k.x < mine) + (k.y < mine) + (k.z < mine) + (k.w < mine);
+    }
+  } else {
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      const uint4 k = block[q];
+      before += (k.x < mine || (k.x == mine && 4 * q + 0 < lane)) +
+                (k.y < mine || (k.y == mine && 4 * q + 1 < lane)) +
+                (k.z < mine || (k.z == mine && 4 * q + 2 < lane)) +
+                (k.w < mine || (k.w == mine && 4 * q + 3 < lane));
+    }
+  }
+  part[j][i * 64 + lane] = before;
+  __syncthreads();
+  if (threadIdx.x >= kChunk) return;
+  uint32_t place = 0;
+#pragma unroll
+  for (int b = 0; b < kBlocks; ++b) place += part[b][threadIdx.x];
+  if (place < uint32_t(kChunk)) {  // always: the places are a permutation
+    chunk_keys[first + place] = own[threadIdx.x];
+    chunk_ids[first + place] = uint16_t(first + int(threadIdx.x));
+  }
+}
+
+// Workgroup b ranks the 64 sorted keys [64 b, 64 b + 64) of chunk b / 4, one
+// per lane: neighbours in value, so a wave's searches read few different LDS
+// words.  Its waves share the chunks to search.
 __global__ __launch_bounds__(kRankWaves * 64) void rank_kernel(
-    const uint32_t* __restrict__ keys, const uint32_t* __restrict__ rects, int n,
-    uint32_t* __restrict__ sorted_rects, uint16_t* __restrict__ sorted_ids,
-    float* __restrict__ clear, int clear_per_gaussian) {
+    const uint32_t* __restrict__ chunk_keys, const uint16_t* __restrict__ chunk_ids, int chunks,
+    const uint32_t* __restrict__ rects, int n, uint32_t* __restrict__ sorted_rects,
+    uint16_t* __restrict__ sorted_ids, float* __restrict__ clear, int clear_per_gaussian) {
+  __shared__ __align__(16) uint32_t staged[kRoundChunks * kChunk];
   __shared__ uint32_t part[kRankWaves][64];
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
   const int b = blockIdx.x;
-  const int i = b * 64 + lane;
-  const int blocks = (n + 63) >> 6;
-  const uint32_t mine = i < n ? keys[i] : 0xFFFFFFFFu;
+  const int own = b / kBlocks;
+  const uint32_t mine = chunk_keys[b * 64 + lane];
+  const int id = chunk_ids[b * 64 + lane];
   if (clear) {
-    const int first = b * 64 * clear_per_gaussian;
-    const int last = min(first + 64 * clear_per_gaussian, n * clear_per_gaussian);
+    const int first = min(b * 64, n) * clear_per_gaussian;
+    const int last = min(b * 64 + 64, n) * clear_per_gaussian;
     for (int k = first + int(threadIdx.x); k < last; k += kRankWaves * 64) clear[k] = 0.0f;
   }
-  const int share = (blocks + kRankWaves - 1) / kRankWaves;
-  const int j0 = wid * share, j1 = min(j0 + share, blocks);
   uint32_t before = 0;
-  for (int jb = j0; jb < j1; ++jb) {  // wave-uniform
-    if (jb == b || jb * 64 + 64 > n) {
-      // The workgroup's own Gaussians (a tie comes before the lanes after it)
-      // or the last, partial block: the lanes' keys in turn, past the end one
-      // that is never before another.
-      const int j = jb * 64 + lane;
-      const uint32_t theirs = j < n ? keys[j] : 0xFFFFFFFFu;
-#pragma unroll 8
-      for (int k = 0; k < 64; ++k) {
-        const uint32_t key = uint32_t(__builtin_amdgcn_readlane(int(theirs), k));
-        const uint64_t ties = jb < b ? ~uint64_t(0) : jb > b ? 0 : ~uint64_t(1) << k;
-        const uint64_t m = __builtin_amdgcn_ballot_w64(key < mine) |
-                           (__builtin_amdgcn_ballot_w64(key == mine) & ties);
-        before += __builtin_amdgcn_inverse_ballot_w64(m) ? 1u : 0u;
-      }
-      continue;
+  for (int c0 = 0; c0 < chunks; c0 += kRoundChunks) {  // workgroup-uniform
+    if (c0) __syncthreads();  // the previous round's searches are done
+    const int quads = min(chunks - c0, kRoundChunks) * (kChunk / 4);
+    const uint4* from = reinterpret_cast<const uint4*>(chunk_keys + c0 * kChunk);
+    uint4* to = reinterpret_cast<uint4*>(staged);
+#pragma unroll
+    for (int i = 0; i < kRoundChunks * kChunk / 4 / (kRankWaves * 64); ++i) {
+      const int q = int(threadIdx.x) + i * kRankWaves * 64;
+      if (q < quads) to[q] = from[q];
     }
-    const uint32_t* __restrict__ block = keys + jb * 64;
-    if (jb < b) {
+    __syncthreads();
+    // Keys of chunk c before mine: those of a chunk with lower indices also
+    // where they are equal.  The chunks' searches run side by side; one that
+    // is not there searches the first chunk, for nothing.
+    int at[kWaveChunks];
+    uint32_t place[kWaveChunks], below[kWaveChunks];
 #pragma unroll
-      for (int k = 0; k < 64; ++k) before += block[k] <= mine ? 1u : 0u;
-    } else {
+    for (int t = 0; t < kWaveChunks; ++t) {
+      const int c = c0 + wid + t * kRankWaves;
+      at[t] = c < chunks ? (c - c0) * kChunk : 0;
+      place[t] = 0;
+      // Counted: keys < below.  ~0u + 1 stays ~0u; see the end.
+      below[t] = c < own && mine != 0xFFFFFFFFu ? mine + 1 : mine;
+    }
 #pragma unroll
-      for (int k = 0; k < 64; ++k) before += block[k] < mine ? 1u : 0u;
+    for (int step = kChunk / 2; step > 0; step >>= 1) {
+#pragma unroll
+      for (int t = 0; t < kWaveChunks; ++t)
+        place[t] += staged[at[t] + place[t] + step - 1] < below[t] ? step : 0;
+    }
+#pragma unroll
+    for (int t = 0; t < kWaveChunks; ++t) {
+      const int c = c0 + wid + t * kRankWaves;
+      place[t] += staged[at[t] + place[t]] < below[t] ? 1 : 0;  // place <= 255 before
+      if (c < own && mine == 0xFFFFFFFFu) place[t] = kChunk;     // <= ~0u: all of them
+      if (c < chunks && c != own) before += place[t];
     }
   }
   part[wid][lane] = before;
   __syncthreads();
-  if (wid != 0 || i >= n) return;
-  uint32_t rank = 0;
+  if (wid != 0 || id >= n) return;
+  uint32_t rank = uint32_t(b % kBlocks * 64 + lane);
 #pragma unroll
   for (int w = 0; w < kRankWaves; ++w) rank += part[w][lane];
   if (rank < uint32_t(n)) {  // always: the ranks are a permutation
-    sorted_rects[rank] = rects[i];
-    sorted_ids[rank] = uint16_t(i);
+    sorted_rects[rank] = rects[id];
+    sorted_ids[rank] = uint16_t(id);
   }
 }
 
@@ -204,7 +279,9 @@ extern "C" {
 GS_API size_t gs_small_lists_bytes(int64_t n, int32_t tiles_w, int32_t tiles_h) {
   if (tiles_w <= 0 || tiles_h <= 0 || tiles_w > kMaxAxisTiles || tiles_h > kMaxAxisTiles) return 0;
   if (!small_fits(n, int64_t(tiles_w) * tiles_h)) return 0;
-  return align_up(size_t(n) * 4) + align_up(size_t(n) * 2);
+  const size_t padded = size_t(ceil_div(n, kChunk)) * kChunk;
+  return align_up(size_t(n) * 4) + align_up(size_t(n) * 2) + align_up(padded * 4) +
+         align_up(padded * 2);
 }
 
 GS_API int gs_small_lists(const uint32_t* depth_keys, const uint32_t* tile_rects, int64_t n,
@@ -231,11 +308,20 @@ GS_API int gs_small_lists(const uint32_t* depth_keys, const uint32_t* tile_rects
   GS_REQUIRE(clear_per_gaussian >= 0 && clear_per_gaussian <= 64, GS_ERR_INVALID_ARGUMENT,
              "invalid clear size %d", clear_per_gaussian);
   hipStream_t s = as_stream(stream);
-  uint32_t* rects = static_cast<uint32_t*>(workspace);
-  uint16_t* ids =
-      reinterpret_cast<uint16_t*>(static_cast<char*>(workspace) + align_up(size_t(n) * 4));
-  rank_kernel<<<unsigned(ceil_div(n, 64)), kRankWaves * 64, 0, s>>>(
-      depth_keys, tile_rects, int(n), rects, ids, clear, clear_per_gaussian);
+  const int chunks = int(ceil_div(n, kChunk));
+  char* at = static_cast<char*>(workspace);
+  uint32_t* rects = reinterpret_cast<uint32_t*>(at);
+  at += align_up(size_t(n) * 4);
+  uint16_t* ids = reinterpret_cast<uint16_t*>(at);
+  at += align_up(size_t(n) * 2);
+  uint32_t* chunk_keys = reinterpret_cast<uint32_t*>(at);
+  at += align_up(size_t(chunks) * kChunk * 4);
+  uint16_t* chunk_ids = reinterpret_cast<uint16_t*>(at);
+  chunk_kernel<<<unsigned(chunks), kRankWaves * 64, 0, s>>>(depth_keys, int(n), chunk_keys,
+                                                            chunk_ids);
+  GS_TRY(check_launch("small_lists chunks"));
+  rank_kernel<<<unsigned(chunks * kBlocks), kRankWaves * 64, 0, s>>>(
+      chunk_keys, chunk_ids, chunks, tile_rects, int(n), rects, ids, clear, clear_per_gaussian);
   GS_TRY(check_launch("small_lists rank"));
   const dim3 grid(unsigned(ceil_div(tiles_w, kStrip)), unsigned(tiles_h));
   lists_kernel<<<grid, kListWaves * 64, unsigned(lists_lds(n)), s>>>(rects, ids, int(n), tiles_w,

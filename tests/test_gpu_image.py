@@ -211,7 +211,9 @@ def test_image_tile_rule():
 
 
 @pytest.mark.parametrize("n,tw,th", [(1, 1, 1), (63, 5, 3), (64, 4, 1), (65, 3, 7), (1000, 256, 2),
-                                     (1025, 17, 256), (5000, 30, 41), (24576, 26, 26)])
+                                     (1025, 17, 256), (5000, 30, 41), (24576, 26, 26),
+                                     (255, 3, 2), (256, 3, 2), (257, 3, 2), (12288, 9, 11),
+                                     (12289, 9, 11)])
 def test_small_lists_equal_bucketing(n, tw, th, device):
     """gs_small_lists against the row/column bucketing: the same lists (ties
     by index, Gaussians without a rectangle nowhere), and the clear buffer."""
