@@ -9,16 +9,16 @@
 //     Counting all n keys for each Gaussian took 17.4 and 46.9 us (n^2 / 64
 //     wave comparisons of two VALU instructions), the four passes of the depth
 //     sort take 33 and 40 us and five launches.
-//  2. lists: a workgroup takes four neighbouring tiles of one tile row, tests
-//     every rectangle in depth order against them (a ballot per 64 Gaussians
+//  2. lists: a workgroup takes up to four neighbouring tiles of one tile row,
+//     tests every rectangle in depth order against them (a ballot per 64 Gaussians
 //     and tile) and writes each tile's hits at the tile's own n slots.
 //
 // The row/column bucketing of tile_bin.hip does the same in 15 launches of 2 to
 // 17 us, each a short dependent chain at this size, and has the host wait for
 // its totals in between; it reads every rectangle a few times where this one
-// reads it once per four tiles, so this one is for few Gaussians on few tiles
-// (small_fits).  Lists kernel: 12 us for 10k Gaussians on 256 or 1200 tiles.
-// Frames of 10k Gaussians at 256 x 256 and 640 x 480: 178 -> 54 and 179 -> 64
+// reads it once per one to four tiles, so this one is for few Gaussians on few
+// tiles (small_fits).
+// Frames of 10k Gaussians at 256 x 256 and 640 x 480: 178 -> 46 and 179 -> 61
 // us.
 //
 // List t is gaussian_ids[ranges[t]) in [t n, (t + 1) n): lists do not touch one
@@ -31,7 +31,13 @@
 namespace gs {
 namespace {
 
-constexpr int kStrip = 4;          // tiles per workgroup of the lists kernel
+// Tiles per workgroup of the lists kernel (its strip): 1, 2 or 4, the least whose
+// workgroups are all resident at once, two per CU.  More of them share the
+// chip's loads and each tile's list is written by more waves; past that they
+// wait for one another and read the rectangles again.  10k Gaussians on 256
+// tiles 12.4 us with strips of 4, 6.7 of 1; 20k on 520 tiles 15.5 of 4, 12.0 of
+// 2; 10k on 1200 tiles 12.0 of 4.
+constexpr int64_t kListGroups = 512;
 constexpr int kChunk = 256;        // keys sorted by one workgroup
 constexpr int kBlocks = kChunk / 64;
 constexpr int kRankWaves = 16;
@@ -174,20 +180,21 @@ __global__ __launch_bounds__(kRankWaves * 64) void rank_kernel(
   }
 }
 
-// Workgroup (x, y): tiles x kStrip .. x kStrip + kStrip - 1 of tile row y.
-// Dynamic LDS: the strip's masks [kStrip][blocks], then their prefixes
-// [kStrip][blocks] (16 bits: below n), then the ids in depth order [n].
+// Workgroup (x, y): tiles x STRIP .. x STRIP + STRIP - 1 of tile row y.
+// Dynamic LDS: the strip's masks [STRIP][blocks], then their prefixes
+// [STRIP][blocks] (16 bits: below n), then the ids in depth order [n].
+template <int STRIP>
 __global__ __launch_bounds__(kListWaves * 64) void lists_kernel(
     const uint32_t* __restrict__ sorted_rects, const uint16_t* __restrict__ sorted_ids, int n,
     int tw, int64_t* __restrict__ ranges, int32_t* __restrict__ gaussian_ids) {
   extern __shared__ uint64_t lds[];
   const int blocks = (n + 63) >> 6;
   uint64_t* masks = lds;
-  uint16_t* prefix = reinterpret_cast<uint16_t*>(masks + kStrip * blocks);
-  uint16_t* ids = prefix + kStrip * blocks;
+  uint16_t* prefix = reinterpret_cast<uint16_t*>(masks + STRIP * blocks);
+  uint16_t* ids = prefix + STRIP * blocks;
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
-  const uint32_t tx0 = blockIdx.x * kStrip, ty = blockIdx.y;
+  const uint32_t tx0 = blockIdx.x * STRIP, ty = blockIdx.y;
 
   // 1. Hits of the strip's tiles, 64 Gaussians per wave and step; the loads of
   // four steps are in flight together.
@@ -210,18 +217,18 @@ __global__ __launch_bounds__(kListWaves * 64) void lists_kernel(
       const uint32_t x0 = r & 0xFFu, w1 = (r >> 8) & 0xFFu;
       uint64_t mine = 0;
 #pragma unroll
-      for (int s = 0; s < kStrip; ++s) {
+      for (int s = 0; s < STRIP; ++s) {
         const uint64_t m = __builtin_amdgcn_ballot_w64(row && tx0 + s - x0 <= w1);
         mine = lane == s ? m : mine;
       }
-      if (lane < kStrip) masks[lane * blocks + b] = mine;
+      if (lane < STRIP) masks[lane * blocks + b] = mine;
       if (b * 64 + lane < n) ids[b * 64 + lane] = id[i];
     }
   }
   __syncthreads();
 
   // 2. One wave per tile: the hits before each block, and the tile's range.
-  if (wid < kStrip) {
+  if (wid < STRIP) {
     uint32_t carry = 0;
     for (int b0 = 0; b0 < blocks; b0 += 64) {
       const int b = b0 + lane;
@@ -238,16 +245,17 @@ __global__ __launch_bounds__(kListWaves * 64) void lists_kernel(
   }
   __syncthreads();
 
-  // 3. The lists: each tile's waves take chunks of 64 blocks, one block's mask
-  // and prefix per lane, and visit the blocks with hits.
-  constexpr int kTileWaves = kListWaves / kStrip;
-  const int s = wid & (kStrip - 1);
+  // 3. The lists: each tile's waves take equal chunks of up to 64 blocks,
+  // one block's mask and prefix per lane, and visit the blocks with hits.
+  constexpr int kTileWaves = kListWaves / STRIP;
+  const int s = wid & (STRIP - 1);
   const int tx = int(tx0) + s;
   if (tx >= tw) return;  // wave-uniform, after the last barrier
   const int64_t t = int64_t(ty) * tw + tx;
   int32_t* list = gaussian_ids + t * n;
-  for (int b0 = wid / kStrip * 64; b0 < blocks; b0 += kTileWaves * 64) {
-    const int b = b0 + lane;
+  const int share = min(64, (blocks + kTileWaves - 1) / kTileWaves);
+  for (int b0 = wid / STRIP * share; b0 < blocks; b0 += kTileWaves * share) {
+    const int b = lane < share ? b0 + lane : blocks;
     const uint64_t m = b < blocks ? masks[s * blocks + b] : 0;
     const uint32_t first = b < blocks ? prefix[s * blocks + b] : 0u;
     uint64_t hits = __builtin_amdgcn_ballot_w64(m != 0);
@@ -264,9 +272,13 @@ __global__ __launch_bounds__(kListWaves * 64) void lists_kernel(
   }
 }
 
-size_t lists_lds(int64_t n) {
-  const int64_t blocks = (n + 63) / 64;
-  return size_t(kStrip * blocks * 10 + blocks * 64 * 2);
+template <int STRIP>
+void launch_lists(const uint32_t* rects, const uint16_t* ids, int n, int tw, int th,
+                  int64_t* ranges, int32_t* gaussian_ids, hipStream_t s) {
+  const int64_t blocks = ceil_div(n, 64);
+  const size_t lds = size_t(STRIP * blocks * 10 + blocks * 64 * 2);
+  lists_kernel<STRIP><<<dim3(unsigned(ceil_div(tw, STRIP)), unsigned(th)), kListWaves * 64, lds,
+                        s>>>(rects, ids, n, tw, ranges, gaussian_ids);
 }
 
 }  // namespace
@@ -323,9 +335,11 @@ GS_API int gs_small_lists(const uint32_t* depth_keys, const uint32_t* tile_rects
   rank_kernel<<<unsigned(chunks * kBlocks), kRankWaves * 64, 0, s>>>(
       chunk_keys, chunk_ids, chunks, tile_rects, int(n), rects, ids, clear, clear_per_gaussian);
   GS_TRY(check_launch("small_lists rank"));
-  const dim3 grid(unsigned(ceil_div(tiles_w, kStrip)), unsigned(tiles_h));
-  lists_kernel<<<grid, kListWaves * 64, unsigned(lists_lds(n)), s>>>(rects, ids, int(n), tiles_w,
-                                                                     ranges, gaussian_ids);
+  auto groups = [&](int strip) { return ceil_div(tiles_w, strip) * tiles_h; };
+  auto lists = groups(1) <= kListGroups   ? launch_lists<1>
+               : groups(2) <= kListGroups ? launch_lists<2>
+                                          : launch_lists<4>;
+  lists(rects, ids, int(n), tiles_w, tiles_h, ranges, gaussian_ids, s);
   return check_launch("small_lists");
 }
 
