@@ -325,13 +325,43 @@ __device__ __forceinline__ void composite_tile(const CompositeArgs& a, float4 (*
         composite_batch(mask1, chunk2, base + 64);
       }
     }
+  } else if constexpr (kRecords) {
+    // A tile's quarters with a backward to follow, in images of few tiles or of
+    // long lists: too few waves to hide a gather per batch, and one band per
+    // lane leaves registers for the next batch's records, requested a batch
+    // ahead (ids two ahead; lanes past the list read a record they do not use).
+    // 4M Gaussians in a small cube 334 -> 297 us, 10k at 640 x 480 43.7 -> 41.7;
+    // with more tiles the same (300k at 1237 x 822: 99).  For an image alone,
+    // with fewer registers and more waves, it gave nothing (27.4 -> 28.1 us, 10k
+    // at 256 x 256).  Reading an entry's row from LDS while the one before
+    // blends cost 3 to 9% everywhere.
+    GsRecord next;
+    if (running) next = load_record(a.records, min(id, a.max_id));
+    id = start + 64 + lane < end ? uint32_t(a.ids[start + 64 + lane]) : 0u;
+    for (int64_t base = start; running && base < end; base += 64) {
+      record_at(int(base - start));
+      float rx0, rx1, ry0, ry1;
+      active_rect(rx0, rx1, ry0, ry1);
+      const int64_t e = base + lane;
+      LaneSplat mine;
+      bool keep = false;
+      if (e < end) {
+        keep = touches_rect(next, rx0, rx1, ry0, ry1);
+        mine = lane_splat(next);
+      }
+      stage(chunk, mine);
+      next = load_record(a.records, min(id, a.max_id));
+      id = e + 128 < end ? uint32_t(a.ids[e + 128]) : 0u;
+      const uint64_t mask = __ballot(keep);
+      store_hits(mask, base);
+      composite_batch(mask, chunk, base);
+    }
   } else {
     // The ids of each batch are requested one batch ahead, once the current
     // batch's records are in LDS, so they arrive while the current batch is
     // walked and each batch waits on one dependent load (the record gather).
     for (int64_t base = start; running && base < end; base += 64) {
       checkpoint_at(int(base - start));
-      record_at(int(base - start));
       float rx0, rx1, ry0, ry1;
       active_rect(rx0, rx1, ry0, ry1);
       const int64_t e = base + lane;
