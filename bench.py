@@ -1014,10 +1014,12 @@ def main():
     }
 
     # The HBM-bound kernels, timed per launch the same way: algorithmic bytes
-    # of the projection (parameters in, 104 B of outputs per Gaussian out)
-    # and of its backward (parameters and dL/d projected in, gradients out).
+    # of the step's projection (parameters in; record, depth key and packed
+    # rectangle, 56 B per Gaussian, out) and of its backward (parameters and
+    # dL/d projected in, gradients out).
     kernels = {}
-    for name, t, nbytes in (("project_fwd_kernel", project_timer, bytes_model["project"]),
+    project_bytes = scene.num_points * (44 + 12 * scene.color.shape[1] + 56)
+    for name, t, nbytes in (("project_fwd_kernel", project_timer, project_bytes),
                             ("project_bwd_kernel", project_bwd_timer, bytes_model["project_bwd"])):
         ms = t.mean_ms()
         if ms > 0:
