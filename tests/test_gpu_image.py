@@ -107,9 +107,9 @@ def test_image_equals_op(kind, size, tile, mode, device):
 
 
 def test_image_long_lists(device):
-    """Lists above 8192 entries: checkpointed walk with a backward, the same
-    walk without checkpoints for the image alone; a second backward through
-    one graph re-zeroes its accumulator."""
+    """Lists above 8192 entries: four waves per tile and a backward in segments,
+    against the op's checkpointed walk; a second backward through one graph
+    re-zeroes its accumulator."""
     scene = scenes.config4(n=60000)
     scene = scene.to(device)
     cam = scene.cameras[0]
@@ -117,8 +117,8 @@ def test_image_long_lists(device):
     leaves = [p.detach().clone().requires_grad_(True) for p in scene.params()]
     image = rasterize(splats, cam, 16)
     expected = _op(scene, leaves, cam, 16, "gaussian")
-    # Checkpoints cut a pixel's colour into partial sums at list positions, and
-    # the lists differ: up to 64 roundings of a sum below 4.
+    # The op's checkpoints cut a pixel's colour into partial sums at list
+    # positions: up to 64 roundings of a sum below 4.
     assert (image - expected).abs().max() < 64 * 4 * 2.0 ** -24
     with torch.no_grad():
         assert (image - rasterize(splats, cam, 16)).abs().max() < 64 * 4 * 2.0 ** -24
