@@ -201,7 +201,7 @@ def forward_image(params, request: ImageRequest, keep: bool, timer=None):
     # With long lists the longest walk sets the time of a launch: tiles are
     # split over four waves however many there are (4M Gaussians in a small cube,
     # 4264 tiles with work: 355 + 646 us forward and backward with a wave per
-    # tile and checkpoints, 297 + 385 with four).
+    # tile and checkpoints, 295 + 390 with four).
     view.active_tiles = min(active, SPLIT_TILES - 1) if longest > LONG_LIST else active
     num_tiles, total = tiles_w * tiles_h * subs, ids.numel()
     image = torch.empty((views, height, width, 3), dtype=torch.float32, device=device)
