@@ -78,7 +78,10 @@ def image_tile(asked: int, width: int, height: int, n: int, views: int = 1) -> i
 class ImageRequest:
     """Everything but the Gaussians of an image call on ``n`` of them: the
     ``cameras`` (``camera_floats`` of ``views`` of them), the views and the
-    scalars.
+    scalars.  ``stacked``: the images keep their view axis (``rasterize_views``);
+    one camera's image without it is written as such, since a select of the stack
+    would make the caller's image a view and its gradient a filled and copied
+    stack (1080p, a step: 16 us of GPU time and three launches).
 
     The lists are those of ``tiles`` = (width, height) list tiles, laid out by
     ``list_view``; the compositing tiles by ``view``.  ``small``: the bytes of a
@@ -95,12 +98,13 @@ class ImageRequest:
     and 16 views of 2500 tiles, which walk a quarter of their lists, gained
     nothing."""
 
-    __slots__ = ("floats", "view", "list_view", "views", "tiles", "near", "far", "gaussian",
-                 "small")
+    __slots__ = ("floats", "view", "list_view", "views", "shape", "tiles", "near", "far",
+                 "gaussian", "small")
 
     def __init__(self, n, cameras, views, width, height, tile, threshold, near, far,
-                 rendering_mode, confidence):
+                 rendering_mode, confidence, stacked):
         self.views, self.floats = views, cameras
+        self.shape = (views, height, width, 3) if stacked else (height, width, 3)
         tw, th = nat.tiles(width, height, tile)
         shift = int(tile == 16 and self.views == 1 and tw * th >= SPLIT_TILES)
         tw, th = nat.tiles(width, height, tile << shift)
@@ -151,8 +155,8 @@ def small_lists(depth_keys, tile_rects, tiles_w, tiles_h, nbytes, clear=None):
 
 
 def forward_image(params, request: ImageRequest, keep: bool, timer=None):
-    """Projects, bins and composites; returns ``(image [V, H, W, 3], saved,
-    walk)``, the last two None unless ``keep`` (a backward will follow)."""
+    """Projects, bins and composites; returns ``(image, saved, walk)``, the last
+    two None unless ``keep`` (a backward will follow)."""
     mark = timer or (lambda name: None)
     device = nat.require_gpu(*params)
     mean, rotation, scale, opacity, color = (nat.prepare(t) for t in params)
@@ -204,7 +208,7 @@ def forward_image(params, request: ImageRequest, keep: bool, timer=None):
     # tile and checkpoints, 295 + 390 with four).
     view.active_tiles = min(active, SPLIT_TILES - 1) if longest > LONG_LIST else active
     num_tiles, total = tiles_w * tiles_h * subs, ids.numel()
-    image = torch.empty((views, height, width, 3), dtype=torch.float32, device=device)
+    image = torch.empty(request.shape, dtype=torch.float32, device=device)
     if not backward:
         nat.check(
             nat.launch("composite", lambda: lib.gs_composite_image(
@@ -322,8 +326,8 @@ class _RenderImage(torch.autograd.Function):
 
 
 def render_image(params, request: ImageRequest, timer=None) -> torch.Tensor:
-    """The [V, H, W, 3] images of ``request``'s cameras, differentiable with
-    respect to the five parameter tensors in Gaussian mode."""
+    """The image or stack of images (``request.shape``) of ``request``'s cameras,
+    differentiable with respect to the five parameter tensors in Gaussian mode."""
     if torch.is_grad_enabled() and any(t.requires_grad for t in params):
         return _RenderImage.apply(*params, request, timer)
     return forward_image(params, request, False, timer)[0]

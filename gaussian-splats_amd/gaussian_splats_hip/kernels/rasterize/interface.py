@@ -416,10 +416,9 @@ def rasterize(
             request = ImageRequest(
                 mean.shape[0], camera_floats((camera,)), 1, int(image_width), int(image_height),
                 tile, float(opacity_threshold), float(near), float(far), rendering_mode,
-                float(confidence),
+                float(confidence), stacked=False,
             )
-            return render_image((mean, rotation, scale, opacity, color), request,
-                                stage_timer())[0]
+            return render_image((mean, rotation, scale, opacity, color), request, stage_timer())
     camera_rotation, camera_translation = host_extrinsics(camera)
     return rasterize_outputs(
         mean,

@@ -511,7 +511,7 @@ def rasterize_views(
             request = ImageRequest(
                 params[0].shape[0], camera_floats(cameras), len(cameras), width, height, tile,
                 float(opacity_threshold), float(near), float(far), rendering_mode,
-                float(confidence),
+                float(confidence), stacked=True,
             )
             return render_image(params, request, stage_timer())
     rotations, translations, intrinsics, width, height = camera_tensors(cameras)

@@ -173,6 +173,23 @@ def test_views_image_equals_op(device):
     _same_gradients([getattr(splats, n).grad for n in PARAMS], [p.grad for p in leaves])
 
 
+def test_image_is_no_view(device):
+    """One camera's image is a tensor of its own, as the op's output is: it can
+    be detached in place, and its gradient reaches the backward as it is."""
+    scene = scenes.edge_case_scene(n=200, image_size=(48, 32)).to(device)
+    cam = scene.cameras[0]
+    splats = GaussianSplat.from_tensors(*scene.params())
+    image = rasterize(splats, cam, near=scene.near, far=scene.far)
+    assert image.shape == (32, 48, 3) and not image._is_view()
+    assert image.grad_fn.name() == "_RenderImageBackward"
+    image.detach_()
+    with torch.no_grad():
+        image = rasterize(splats, cam, near=scene.near, far=scene.far)
+    assert image.shape == (32, 48, 3) and not image._is_view()
+    image.detach_()
+    assert rasterize_views(splats, [cam]).shape == (1, 32, 48, 3)
+
+
 def test_no_gaussians_and_nothing_visible(device):
     scene = scenes.edge_case_scene(n=40, image_size=(50, 30)).to(device)
     cam = scene.cameras[0]
