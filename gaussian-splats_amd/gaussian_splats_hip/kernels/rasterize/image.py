@@ -130,9 +130,11 @@ class ImageRequest:
 
 
 class _Walk:
-    """What the forward keeps for its backward beside the saved tensors."""
+    """What the forward keeps for its backward beside the saved tensors, which
+    hold everything of size but the accumulator (the backward takes that), so
+    that a backward which does not retain the graph frees it."""
 
-    __slots__ = ("view", "accumulator", "hits", "order", "records", "longest")
+    __slots__ = ("view", "accumulator", "longest")
 
 
 def small_lists(depth_keys, tile_rects, tiles_w, tiles_h, nbytes, clear=None):
@@ -221,19 +223,17 @@ def forward_image(params, request: ImageRequest, keep: bool, timer=None):
     final_transmittance = torch.empty((views, height, width), dtype=torch.float32, device=device)
     n_contributors = torch.empty((views, height, width), dtype=torch.int32, device=device)
     hits = nat.hit_mask_buffer(view, total, device)
-    walk = _Walk()
-    walk.order = walk.records = None
-    walk.longest = longest
+    order = walk_records = None
     walk_bytes = lib.gs_composite_walk_bytes(view)
     if walk_bytes:
         # Few tiles: the walk's state at fixed positions, for a backward in
         # segments (no plan: the segments are dealt in tile order).
-        walk.records = nat.workspace(walk_bytes, device)
+        walk_records = nat.workspace(walk_bytes, device)
         nat.check(
             nat.launch("composite", lambda: lib.gs_composite_walk(
                 ptr(records), vn, ptr(ids), total, longest, ptr(ranges), view, ptr(image),
                 ptr(final_transmittance), ptr(n_contributors), ptr(hits), nat.buffer_bytes(hits),
-                ptr(walk.records), walk_bytes, stream,
+                ptr(walk_records), walk_bytes, stream,
             )),
             "composite_walk",
         )
@@ -250,28 +250,31 @@ def forward_image(params, request: ImageRequest, keep: bool, timer=None):
         )
         mark("composite")
         # The backward's dispatch plan, behind the forward on the stream.
-        walk.order = torch.empty(lib.gs_tile_order_items(view, 1), dtype=torch.int32,
-                                 device=device)
+        order = torch.empty(lib.gs_tile_order_items(view, 1), dtype=torch.int32, device=device)
         nat.check(
-            lib.gs_tile_order(ptr(ranges), ptr(n_contributors), view, ptr(walk.order), ptr(keys),
+            lib.gs_tile_order(ptr(ranges), ptr(n_contributors), view, ptr(order), ptr(keys),
                               keys.numel(), 1, stream),
             "tile_order",
         )
-    walk.view, walk.accumulator, walk.hits = view, accumulator, hits
-    return image, (records, tile_rects, ids, ranges, final_transmittance, n_contributors), walk
+    walk = _Walk()
+    walk.view, walk.accumulator, walk.longest = view, accumulator, longest
+    saved = (records, tile_rects, ids, ranges, final_transmittance, n_contributors, hits, order,
+             walk_records)
+    return image, saved, walk
 
 
-def _aligned(t: torch.Tensor) -> torch.Tensor:
-    return t if t.is_contiguous() and t.data_ptr() % 16 == 0 else t.clone(
-        memory_format=torch.contiguous_format)
+def _aligned(t: torch.Tensor | None) -> torch.Tensor | None:
+    if t is None or (t.is_contiguous() and t.data_ptr() % 16 == 0):
+        return t
+    return t.clone(memory_format=torch.contiguous_format)
 
 
 def backward_image(params, saved, walk: _Walk, request: ImageRequest, grad_image):
     """Gradients of the five parameter tensors for the image gradient."""
     params = tuple(_aligned(t) for t in params)
     mean, color = params[0], params[4]
-    records, tile_rects, ids, ranges, final_transmittance, n_contributors = (
-        _aligned(t) for t in saved)
+    (records, tile_rects, ids, ranges, final_transmittance, n_contributors, hits, order,
+     walk_records) = (_aligned(t) for t in saved)
     n, device = mean.shape[0], mean.device
     if grad_image is None:
         return tuple(torch.zeros_like(t) for t in params)
@@ -286,9 +289,9 @@ def backward_image(params, saved, walk: _Walk, request: ImageRequest, grad_image
     nat.check(
         nat.launch("composite_bwd", lambda: lib.gs_composite_bwd_image(
             ptr(records), records.shape[0], ptr(ids), ptr(ranges), ptr(grad_image),
-            ptr(final_transmittance), ptr(n_contributors), ptr(walk.order), walk.view,
-            ptr(accumulator), ids.numel(), ptr(walk.hits), nat.buffer_bytes(walk.hits), ptr(walk.records),
-            nat.buffer_bytes(walk.records), walk.longest, stream,
+            ptr(final_transmittance), ptr(n_contributors), ptr(order), walk.view,
+            ptr(accumulator), ids.numel(), ptr(hits), nat.buffer_bytes(hits), ptr(walk_records),
+            nat.buffer_bytes(walk_records), walk.longest, stream,
         )),
         "composite_bwd_image",
     )
