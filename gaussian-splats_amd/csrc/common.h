@@ -242,6 +242,13 @@ constexpr int kWalkPixels = 256;  // per record
 inline size_t walk_record_bytes(int num_tiles) {
   return size_t(num_tiles) * (kWalkSegments - 1) * kWalkPixels * 16;
 }
+// Every tile has room for all of its records (28 KB), also one without a list,
+// so that a slot needs no counter and no pass before the walk.  Images whose
+// records would take more than this (18724 tiles: 2189 x 2189 pixels) keep none
+// and walk back in quarters, which costs less there than the memory is worth: 8
+// views of 200k Gaussians in a small cube, 22500 tiles and 616 MB of records,
+// 1658 us a step, 1701 without.
+constexpr size_t kWalkRecordBytes = size_t(512) << 20;
 // The forward's waves also leave each quarter's largest contributor count:
 // keys[4 tile + quarter].
 

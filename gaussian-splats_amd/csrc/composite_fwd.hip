@@ -702,6 +702,7 @@ extern "C" GS_API size_t gs_composite_walk_bytes(gs_view view) {
   if (check_view(view, true) != GS_OK || view.tile_size != 16) return 0;
   const Mosaic m = mosaic_of(view);
   if (!dispatch_plan(m.num_tiles(), 16, view.active_tiles, false).split_all) return 0;
+  if (walk_record_bytes(m.num_tiles()) > kWalkRecordBytes) return 0;
   return walk_record_bytes(m.num_tiles()) + align_up(size_t(m.num_tiles()) * 16);
 }
 
@@ -713,7 +714,8 @@ extern "C" GS_API int gs_composite_walk(
   clear_error();
   const size_t need = gs_composite_walk_bytes(view);
   GS_REQUIRE(need > 0 && view.rendering_mode == GS_MODE_GAUSSIAN, GS_ERR_UNSUPPORTED,
-             "walk records are for Gaussian rendering on few tiles of 16 pixels");
+             "walk records are for Gaussian rendering on few tiles of 16 pixels, up to %zu bytes",
+             kWalkRecordBytes);
   GS_REQUIRE(final_transmittance && n_contributors && hit_masks && walk, GS_ERR_INVALID_ARGUMENT,
              "null pointer argument");
   GS_REQUIRE(walk_bytes >= need, GS_ERR_WORKSPACE,

@@ -226,8 +226,8 @@ def forward_image(params, request: ImageRequest, keep: bool, timer=None):
     order = walk_records = None
     walk_bytes = lib.gs_composite_walk_bytes(view)
     if walk_bytes:
-        # Few tiles: the walk's state at fixed positions, for a backward in
-        # segments (no plan: the segments are dealt in tile order).
+        # Few tiles with work: the walk's state at fixed positions, for a backward
+        # in segments (no plan: the segments are dealt in tile order).
         walk_records = nat.workspace(walk_bytes, device)
         nat.check(
             nat.launch("composite", lambda: lib.gs_composite_walk(

@@ -439,8 +439,9 @@ GS_API int gs_composite_image(
  * gs_composite_bwd_image walks each tile back in segments of all of its
  * pixels.  longest_list (totals[3] of gs_bin_tiles_plan, 0: unknown) sets how
  * far apart the positions are and must be the same in both calls.
- * gs_composite_walk_bytes: the size of `walk`, or 0 when the view is not of
- * that kind (GS_ERR_UNSUPPORTED). */
+ * gs_composite_walk_bytes: the size of `walk`, at most 512 MiB and 16 bytes per
+ * tile, or 0 when the view is not of that kind or has too many tiles for it
+ * (GS_ERR_UNSUPPORTED). */
 GS_API size_t gs_composite_walk_bytes(gs_view view);
 GS_API int gs_composite_walk(
     const void* records, int64_t num_records, const int32_t* gaussian_ids,

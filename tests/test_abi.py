@@ -231,6 +231,21 @@ def test_hit_masks_host_checks():
     assert status == nat.GS_ERR_WORKSPACE
 
 
+def test_walk_records_are_bounded():
+    """gs_composite_walk_bytes: 7 records of 4 KiB and 16 bytes of keys per tile,
+    never above 512 MiB of records; other views keep none."""
+    lib = nat.library()
+    size = lambda w, h, **kw: lib.gs_composite_walk_bytes(
+        _view(image_width=w, image_height=h, active_tiles=100, **kw))
+    assert size(100, 100) == 49 * 7 * 4096 + 1024
+    most = size(151 * 16, 124 * 16)
+    assert most == 18724 * 7 * 4096 + 18724 * 16 + 192
+    assert most - 18724 * 16 - 192 <= 512 << 20
+    assert size(175 * 16, 107 * 16) == 0  # 18725 tiles
+    assert size(4096, 4096) == 0 and size(800, 800, views=16, mosaic_cols=4) == 0
+    assert size(100, 100, tile_size=32) == 0 and size(1920, 1080, list_shift=1) > 0
+
+
 def test_misaligned_buffers_rejected():
     lib = nat.library()
     fake = ctypes.c_void_p(16)

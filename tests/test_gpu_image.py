@@ -159,6 +159,33 @@ def test_image_walk_segments(size, n, device):
     _same_gradients(second, [p.grad for p in leaves])
 
 
+def _cluster(n, size, spread=0.1):
+    """Gaussians in the middle of a large image: few of its tiles have work."""
+    scene = scenes.edge_case_scene(n=n, sh_degree=0, image_size=size, seed=8)
+    g = torch.Generator().manual_seed(n)
+    scene.mean[:, :2] = torch.randn(n, 2, generator=g) * spread
+    scene.mean[:, 2] = -(torch.rand(n, generator=g) + 4)
+    scene.scale[:] = torch.rand(n, 3, generator=g) - 5
+    return scene
+
+
+def test_image_few_tiles_of_too_many(device):
+    """More tiles than the walk records' bound, few with work: every tile split
+    into quarters in both directions, without records."""
+    scene = _cluster(9000, (4096, 1200)).to(device)
+    splats = GaussianSplat.from_tensors(*scene.params())
+    leaves = [p.detach().clone().requires_grad_(True) for p in scene.params()]
+    image = rasterize(splats, scene.cameras[0], near=scene.near, far=scene.far)
+    order, walk_records = image.grad_fn.saved_tensors[-2:]
+    assert walk_records is None and (order[order >= 0] & 0x20).all()
+    expected = _op(scene, leaves, scene.cameras[0], 16, "gaussian")
+    assert torch.equal(image, expected)
+    weight = torch.linspace(-1, 1, image.numel(), device=device).reshape(image.shape)
+    (image * weight).sum().backward()
+    (expected * weight).sum().backward()
+    _same_gradients([getattr(splats, n).grad for n in PARAMS], [p.grad for p in leaves])
+
+
 def test_views_image_equals_op(device):
     scene = scenes.config5(seed=2, n=4000, views=5, size=90, focal=110).to(device)
     splats = GaussianSplat.from_tensors(*scene.params())
