@@ -287,9 +287,10 @@ __host__ __device__ inline int region_max_tiles(int num_tiles) {
   const int chunks = (num_tiles + k - 1) / k;
   return (chunks + 7) / 8 * k;
 }
-inline DispatchPlan dispatch_plan(int num_tiles, int tile_size, int active, bool backward) {
+inline DispatchPlan dispatch_plan(int num_tiles, const gs_view& v, bool backward) {
   DispatchPlan p;
-  p.split_all = tile_size >= 16 && composite_split(num_tiles, active);
+  p.split_all =
+      v.tile_size >= 16 && (v.split_tiles || composite_split(num_tiles, v.active_tiles));
   p.segments = backward && !p.split_all;
   const int t_max = region_max_tiles(num_tiles);
   const int cap = p.split_all ? 4 * t_max : p.segments ? (1 + kSegmentSpare) * t_max : t_max;

@@ -554,7 +554,7 @@ int composite_bwd(const float* projected_mean, const float* inverse_covariance,
   a.views = m.views;
   a.grad = grad_projected;
   a.grad_abs = grad_absolute;
-  const DispatchPlan plan = dispatch_plan(a.num_tiles, view.tile_size, view.active_tiles, true);
+  const DispatchPlan plan = dispatch_plan(a.num_tiles, view, true);
   a.items = tile_order;
   a.num_items = plan.items();
   a.split_all = plan.split_all;

@@ -552,7 +552,7 @@ extern "C" GS_API size_t gs_composite_checkpoint_bytes(gs_view view, int64_t num
   if (longest_list <= kCheckpointMinList) return 0;  // no walk would record one
   if (view.tile_size > 16) return 0;  // 16 pixels per lane leave no registers for them
   const Mosaic m = mosaic_of(view);
-  if (dispatch_plan(m.num_tiles(), view.tile_size, view.active_tiles, false).split_all) return 0;
+  if (dispatch_plan(m.num_tiles(), view, false).split_all) return 0;
   return checkpoint_layout(nullptr, view.tile_size, num_intersections, m.subs()).bytes;
 }
 
@@ -600,7 +600,7 @@ int composite(const void* records, int64_t num_records, const int32_t* gaussian_
   a.image = image;
   a.final_t = final_transmittance;
   a.n_contrib = n_contributors;
-  const DispatchPlan plan = dispatch_plan(a.num_tiles, view.tile_size, view.active_tiles, false);
+  const DispatchPlan plan = dispatch_plan(a.num_tiles, view, false);
   a.items = tile_order;
   a.num_items = plan.items();
   a.split_all = plan.split_all;
@@ -701,7 +701,7 @@ extern "C" GS_API int gs_composite_image(const void* records, int64_t num_record
 extern "C" GS_API size_t gs_composite_walk_bytes(gs_view view) {
   if (check_view(view, true) != GS_OK || view.tile_size != 16) return 0;
   const Mosaic m = mosaic_of(view);
-  if (!dispatch_plan(m.num_tiles(), 16, view.active_tiles, false).split_all) return 0;
+  if (!dispatch_plan(m.num_tiles(), view, false).split_all) return 0;
   if (walk_record_bytes(m.num_tiles()) > kWalkRecordBytes) return 0;
   return walk_record_bytes(m.num_tiles()) + align_up(size_t(m.num_tiles()) * 16);
 }

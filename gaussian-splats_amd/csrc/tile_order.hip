@@ -319,13 +319,11 @@ int tile_order_launch(const int64_t* ranges, const int32_t* n_contributors, cons
                       hipStream_t s) {
   const int num_tiles = m.num_tiles();
   GS_REQUIRE(num_tiles < (1 << 24), GS_ERR_OVERFLOW, "too many tiles (%d)", num_tiles);
-  const DispatchPlan plan =
-      dispatch_plan(num_tiles, view.tile_size, view.active_tiles, n_contributors != nullptr);
+  const DispatchPlan plan = dispatch_plan(num_tiles, view, n_contributors != nullptr);
   uint32_t* crossings = key + num_tiles;
   // The forward writes keys only when it walked whole tiles.
-  const bool forward_keys = keys_ready && n_contributors &&
-                            !dispatch_plan(num_tiles, view.tile_size, view.active_tiles, false)
-                                 .split_all;
+  const bool forward_keys =
+      keys_ready && n_contributors && !dispatch_plan(num_tiles, view, false).split_all;
   if (!forward_keys) {
     tile_key_kernel<<<unsigned(ceil_div(num_tiles, 4)), 256, 0, s>>>(
         ranges, n_contributors, m.tiles_w(), num_tiles, view.tile_size, view.image_width,
@@ -350,8 +348,7 @@ GS_API int64_t gs_tile_order_items(gs_view view, int32_t by_contributors) {
   clear_error();
   if (check_view(view, true) != GS_OK) return -1;
   const Mosaic m = mosaic_of(view);
-  return dispatch_plan(m.num_tiles(), view.tile_size, view.active_tiles, by_contributors != 0)
-      .items();
+  return dispatch_plan(m.num_tiles(), view, by_contributors != 0).items();
 }
 
 GS_API int gs_tile_order(const int64_t* ranges, const int32_t* n_contributors, gs_view view,

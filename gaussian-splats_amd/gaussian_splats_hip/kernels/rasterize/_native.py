@@ -15,7 +15,7 @@ from pathlib import Path
 import torch
 
 LIB_PATH = Path(__file__).resolve().parents[2] / "_lib" / "libgs_raster.so"
-ABI_VERSION = 19
+ABI_VERSION = 20
 
 GS_OK = 0
 GS_ERR_INVALID_ARGUMENT = 1
@@ -61,6 +61,7 @@ class GsView(ctypes.Structure):
         ("mosaic_cols", c_int32),
         ("active_tiles", c_int32),
         ("list_shift", c_int32),
+        ("split_tiles", c_int32),
     ]
 
 
@@ -82,6 +83,7 @@ def make_view(
     mosaic_cols: int = 1,
     active_tiles: int = 0,
     list_shift: int = 0,
+    split_tiles: int = 0,
 ) -> GsView:
     if rendering_mode not in MODES:
         raise ValueError(f"Invalid rendering mode: {rendering_mode}")
@@ -89,7 +91,7 @@ def make_view(
         float(fx), float(fy), float(cx), float(cy), int(image_width), int(image_height),
         int(tile_size), float(near), float(far), MODES[rendering_mode], float(confidence),
         float(opacity_threshold), float(covariance_epsilon), int(views), int(mosaic_cols),
-        int(active_tiles), int(list_shift),
+        int(active_tiles), int(list_shift), int(split_tiles),
     )
 
 

@@ -75,6 +75,21 @@ def image_tile(asked: int, width: int, height: int, n: int, views: int = 1) -> i
     return None
 
 
+def split_long_lists(longest: int, entries: int, lists: int, tiles: int) -> bool:
+    """Whether an image call's tiles are split over four waves each although
+    ``tiles`` of them (SPLIT_TILES or more) have work: the lists are long (the
+    ``longest`` one, and the mean of ``entries`` in ``lists`` non-empty ones
+    above a third of the tiles), so the longest walk sets the time of a launch,
+    not the number of waves.  A step with a wave per tile and with four: 80k
+    Gaussians in a small cube on 4704 tiles (mean list half of them) 963 and 792
+    us, 2M on 7272 tiles 1988 and 1863, a shell of 2M in four views on 10824
+    tiles (mean 0.75 of them) 5359 and 4820.  A few long lists are no reason: 1M
+    at 1080p with one dense spot (mean 0.29) 682 and 762, 1M at 3840 x 2160 with
+    one (0.05) 1274 and 1628.  Nor are long ones on many tiles: 2M in a small
+    cube on 13300 tiles 2399 and 2580."""
+    return longest > LONG_LIST and tiles < 3 * SPLIT_TILES and 3 * entries > lists * tiles
+
+
 class ImageRequest:
     """Everything but the Gaussians of an image call on ``n`` of them: the
     ``cameras`` (``camera_floats`` of ``views`` of them), the views and the
@@ -169,7 +184,7 @@ def forward_image(params, request: ImageRequest, keep: bool, timer=None):
     lib, stream, ptr = nat.library(), nat.stream(device), nat.ptr
     n, views = mean.shape[0], request.views
     vn = views * n
-    view = nat.GsView.from_buffer_copy(request.view)  # active_tiles is set below
+    view = nat.GsView.from_buffer_copy(request.view)  # active_, split_tiles are set below
     width, height = view.image_width, view.image_height
     tiles_w, tiles_h = request.tiles
 
@@ -203,12 +218,9 @@ def forward_image(params, request: ImageRequest, keep: bool, timer=None):
         longest = nat.longest_list(ranges)
     mark("sort")
     subs = 1 << (2 * view.list_shift)  # compositing tiles per list
-    active = nat.active_tiles(ranges) * subs
-    # With long lists the longest walk sets the time of a launch: tiles are
-    # split over four waves however many there are (4M Gaussians in a small cube,
-    # 4264 tiles with work: 355 + 646 us forward and backward with a wave per
-    # tile and checkpoints, 295 + 390 with four).
-    view.active_tiles = min(active, SPLIT_TILES - 1) if longest > LONG_LIST else active
+    lists = nat.active_tiles(ranges)
+    view.active_tiles = lists * subs
+    view.split_tiles = split_long_lists(longest, ids.numel(), lists, lists * subs)
     num_tiles, total = tiles_w * tiles_h * subs, ids.numel()
     image = torch.empty(request.shape, dtype=torch.float32, device=device)
     if not backward:

@@ -42,7 +42,7 @@ extern "C" {
 
 #define GS_API __attribute__((visibility("default")))
 
-#define GS_ABI_VERSION 19
+#define GS_ABI_VERSION 20
 
 typedef enum gs_status {
   GS_OK = 0,
@@ -87,6 +87,10 @@ typedef struct gs_view {
    * pixels): `ranges` covers the grid of doubled tiles, and each view's tile
    * grid is rounded up to whole ones.  0: one list per tile. */
   int32_t list_shift;
+  /* 1: the compositing calls split every tile of 16 or 32 pixels over four
+   * waves whatever active_tiles says (a caller whose lists are long throughout,
+   * whose longest walk sets a launch's time).  0: by active_tiles. */
+  int32_t split_tiles;
 } gs_view;
 
 /* ABI version of the loaded library (GS_ABI_VERSION). No counterpart in the
@@ -433,9 +437,9 @@ GS_API int gs_composite_image(
     const void* records, int64_t num_records, const int32_t* gaussian_ids,
     int64_t num_intersections, const int64_t* ranges, gs_view view, float* image, void* stream);
 
-/* gs_composite for a Gaussian image call on few tiles (fewer than 4096 tiles
- * of 16 pixels with work, whose pixel bands are split over four waves each),
- * which also records the walk's state at fixed positions, so that
+/* gs_composite for a Gaussian image call on tiles of 16 pixels whose bands are
+ * split over four waves each (fewer than 4096 tiles with work, or
+ * view.split_tiles), which also records the walk's state at fixed positions, so that
  * gs_composite_bwd_image walks each tile back in segments of all of its
  * pixels.  longest_list (totals[3] of gs_bin_tiles_plan, 0: unknown) sets how
  * far apart the positions are and must be the same in both calls.

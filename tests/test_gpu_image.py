@@ -106,16 +106,22 @@ def test_image_equals_op(kind, size, tile, mode, device):
         assert (x - y).norm() <= 8 * spread + 1e-6 * y.norm(), name
 
 
-def test_image_long_lists(device):
-    """Lists above 8192 entries: four waves per tile and a backward in segments,
-    against the op's checkpointed walk; a second backward through one graph
-    re-zeroes its accumulator."""
-    scene = scenes.config4(n=60000)
+@pytest.mark.parametrize("n,focal", [(60_000, 1600.0), (120_000, 2400.0)])
+def test_image_long_lists(n, focal, device):
+    """Lists above 8192 entries: four waves per tile and a backward in segments
+    (at the longer focal length on more than 4096 tiles with work), against the
+    op's checkpointed walk; a second backward through one graph re-zeroes its
+    accumulator."""
+    scene = scenes.config4(n=n, focal=focal)
     scene = scene.to(device)
     cam = scene.cameras[0]
     splats = GaussianSplat.from_tensors(*scene.params())
     leaves = [p.detach().clone().requires_grad_(True) for p in scene.params()]
     image = rasterize(splats, cam, 16)
+    ranges, walk_records = (image.grad_fn.saved_tensors[i] for i in (8, -1))
+    lengths = ranges[:, 1] - ranges[:, 0]
+    assert lengths.max() > 8192 and walk_records is not None
+    assert (4 * (lengths > 0).sum() >= 4096) == (focal == 2400.0)
     expected = _op(scene, leaves, cam, 16, "gaussian")
     # The op's checkpoints cut a pixel's colour into partial sums at list
     # positions: up to 64 roundings of a sum below 4.
@@ -262,6 +268,39 @@ def test_backward_frees_the_walk(device):
         held.append(torch.cuda.memory_allocated() - before)
     assert kept > 30 << 20
     assert held[1] <= image.numel() * 4 + (1 << 20)
+
+
+def test_split_long_lists_rule():
+    from gaussian_splats_hip.kernels.rasterize.image import split_long_lists
+
+    assert split_long_lists(8193, 8_000_000, 1500, 6000)
+    assert not split_long_lists(8192, 8_000_000, 1500, 6000)
+    # One long list among many short ones, and long lists on many tiles.
+    assert not split_long_lists(26_170, 4_796_677, 2040, 8160)
+    assert not split_long_lists(470_000, 53_000_000, 3325, 13_300)
+
+
+def test_image_one_long_list(device):
+    """One list above 8192 entries among many short ones: a wave per tile
+    without records, against the op's checkpointed walk."""
+    scene = scenes.edge_case_scene(n=40_000, sh_degree=0, image_size=(1920, 1080), seed=6)
+    g = torch.Generator().manual_seed(4)
+    scene.mean[20_000:] = torch.tensor([0.3, 0.2, -5.0]) + torch.randn(20_000, 3, generator=g) * 0.01
+    scene.scale[20_000:], scene.opacity[20_000:] = -5.0, -4.0
+    scene = scene.to(device)
+    splats = GaussianSplat.from_tensors(*scene.params())
+    leaves = [p.detach().clone().requires_grad_(True) for p in scene.params()]
+    image = rasterize(splats, scene.cameras[0], near=scene.near, far=scene.far)
+    ranges, order, walk_records = (image.grad_fn.saved_tensors[i] for i in (8, -2, -1))
+    assert (ranges[:, 1] - ranges[:, 0]).max() > 8192
+    assert walk_records is None and order is not None
+    expected = _op(scene, leaves, scene.cameras[0], 16, "gaussian")
+    # The op's checkpoints cut a pixel's colour into partial sums (see below).
+    assert (image - expected).abs().max() < 64 * 4 * 2.0 ** -24
+    weight = torch.linspace(-1, 1, image.numel(), device=device).reshape(image.shape)
+    (image * weight).sum().backward()
+    (expected * weight).sum().backward()
+    _same_gradients([getattr(splats, n).grad for n in PARAMS], [p.grad for p in leaves])
 
 
 def test_image_tile_rule():
