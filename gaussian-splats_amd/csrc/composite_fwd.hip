@@ -95,7 +95,7 @@ __device__ __forceinline__ void composite_tile(const CompositeArgs& a, float4 (*
   if (view >= a.views) {  // an empty slot of the mosaic's last row
     if (write_key && lane == 0) {
       a.tile_keys[tile] = 0u;
-      a.tile_keys[a.num_tiles + tile] = uint32_t(checkpoint_count(start, 0, list_len));
+      a.tile_keys[a.num_tiles + tile] = 0u;
     }
     return;
   }
@@ -434,7 +434,9 @@ __device__ __forceinline__ void composite_tile(const CompositeArgs& a, float4 (*
     for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o, 64));
     if (lane == 0) {
       a.tile_keys[tile] = uint32_t(min(m, 0xFFFF));
-      a.tile_keys[a.num_tiles + tile] = uint32_t(checkpoint_count(start, m, list_len));
+      // Without checkpoints the backward has no record to start a segment from.
+      a.tile_keys[a.num_tiles + tile] =
+          a.ckpt_counter ? uint32_t(checkpoint_count(start, m, list_len)) : 0u;
     }
   }
 }

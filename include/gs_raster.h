@@ -421,7 +421,8 @@ GS_API size_t gs_composite_checkpoint_bytes(gs_view view, int64_t num_intersecti
  * counterpart in the reference): a workspace for the backward's
  * gs_tile_order, filled as each tile's walk ends with its key (the largest
  * contributor count of its pixels, capped at 2^16 - 1) and its checkpoint
- * crossings, so that plan (keys_ready) does not read n_contributors again.
+ * crossings (none without `checkpoints`), so that plan (keys_ready) does not
+ * read n_contributors again.
  * Not written when every tile is split into quarters. */
 GS_API size_t gs_composite_hit_mask_bytes(gs_view view, int64_t num_intersections);
 GS_API int gs_composite(

@@ -281,19 +281,22 @@ def test_split_long_lists_rule():
 
 
 def test_image_one_long_list(device):
-    """One list above 8192 entries among many short ones: a wave per tile
-    without records, against the op's checkpointed walk."""
+    """One list above 8192 entries among many short ones (faint Gaussians in
+    front of the others): a wave per tile without records, against the op's
+    checkpointed walk."""
     scene = scenes.edge_case_scene(n=40_000, sh_degree=0, image_size=(1920, 1080), seed=6)
     g = torch.Generator().manual_seed(4)
-    scene.mean[20_000:] = torch.tensor([0.3, 0.2, -5.0]) + torch.randn(20_000, 3, generator=g) * 0.01
-    scene.scale[20_000:], scene.opacity[20_000:] = -5.0, -4.0
+    scene.mean[20_000:] = torch.tensor([0.05, 0.03, -0.8]) + torch.randn(20_000, 3, generator=g) * 0.002
+    scene.scale[20_000:], scene.opacity[20_000:] = -6.0, -5.3
     scene = scene.to(device)
     splats = GaussianSplat.from_tensors(*scene.params())
     leaves = [p.detach().clone().requires_grad_(True) for p in scene.params()]
     image = rasterize(splats, scene.cameras[0], near=scene.near, far=scene.far)
     ranges, order, walk_records = (image.grad_fn.saved_tensors[i] for i in (8, -2, -1))
     assert (ranges[:, 1] - ranges[:, 0]).max() > 8192
-    assert walk_records is None and order is not None
+    assert walk_records is None
+    # Whole tiles: without checkpoints no walk is cut into segments.
+    assert torch.equal(order[order >= 0] & 0x7F, torch.zeros_like(order[order >= 0]))
     expected = _op(scene, leaves, scene.cameras[0], 16, "gaussian")
     # The op's checkpoints cut a pixel's colour into partial sums (see below).
     assert (image - expected).abs().max() < 64 * 4 * 2.0 ** -24
