@@ -218,39 +218,65 @@ inline CheckpointLayout checkpoint_layout(void* base, int tile_size, int64_t tot
 }
 
 // Walk records (image calls whose forward splits every tile into quarters):
-// the walk back of a 16-pixel tile is cut at fixed walk positions, so that a
-// tile runs on up to kWalkSegments waves that each take all of its pixels.
-// Whenever a quarter's forward wave starts the batch at walk_bound(j), it
-// records per pixel (T, colour since its previous record), and at the end of
-// the walk turns the colours into the colour composited after the record (a
-// suffix sum, as with the checkpoints above).  Record j of a tile exists for the pixels still
-// active there, the only ones a backward segment starts from it.  Short bounds
-// first: segments are waves that take as long as they are, and twice as many
-// waves of half the length leave less of the chip idle at the end (300k
-// Gaussians at 1237 x 822, backward: 158 us, 190 with bounds twice as far).
-constexpr int kWalkSegments = 8;
-// A list shared by 2 x 2 tiles (shift) holds about twice the entries a tile
-// keeps: the bounds double.  Long lists (above kCheckpointMinList) are those of
-// faint or dense scenes, which walk thousands of entries at places: bounds that
-// reach further.
-__host__ __device__ inline int walk_bound(int j, int shift, bool long_lists) {
-  const int b[2][kWalkSegments] = {{0, 64, 128, 192, 256, 384, 640, 1280},
-                                   {0, 128, 384, 768, 1280, 2048, 3072, 4608}};
-  return long_lists ? b[1][j] : b[0][j] << shift;  // 0 <= j < kWalkSegments
-}
+// the walk back of a 16-pixel tile is cut at recorded walk positions, so that a
+// tile runs on up to kWalkSegments waves that each take all of its pixels.  A
+// quarter's forward wave records per pixel (T, colour since its previous
+// record) as it starts the batch at a cut, and at the end of the walk turns the
+// colours into the colour composited after the record (a suffix sum, as with the
+// checkpoints above).  A record exists for the pixels still active at its cut,
+// the only ones a backward segment starts from it.
+//
+// The first `fixed` cuts stand where the tile's pixels mostly are active still.
+// The `spread` cuts behind them are the multiples of a spacing, `unit` entries at
+// first: with `spread` of them and the next one reached, every other one goes and
+// the spacing doubles, so they spread over a walk of any length.  The record at
+// the multiple t of the unit is in slot fixed + t mod spread: spread is a power
+// of two less one, so the kept multiples 2^e .. spread 2^e have different slots,
+// and a multiple's slot is the same in all quarters.  A tile is cut at the
+// multiples of its quarters' largest spacing, which each of them still has.
+//
+// Seven cuts at fixed positions, up to 1280 or 4608 entries, left the rest of a
+// long walk to one wave.  A step of 1M Gaussians far away at 1080p 3993 us with
+// them, 2951 with these; with a faint dense spot in front 6384, 4501; 100k of
+// them in front at 640 x 480 38.5 ms, 19.0.  With all cuts spread, the entries
+// that most pixels take fall into few segments (1M far away at 640 x 480 1018 us,
+// 1032 with these, 1403 with four fixed cuts of eleven).
+constexpr int kWalkSegments = 12;
+constexpr uint32_t kWalkMostDoubled = 17;  // lists hold less than 2^26 entries
 constexpr int kWalkPixels = 256;  // per record
-inline size_t walk_record_bytes(int num_tiles) {
-  return size_t(num_tiles) * (kWalkSegments - 1) * kWalkPixels * 16;
+constexpr size_t kWalkRecordBytes = size_t(1152) << 20;
+struct WalkCuts {
+  int fixed, spread, unit;
+  int shift;  // positions are twice these for a list shared by 2 x 2 tiles
+  __host__ __device__ int records() const { return fixed + spread; }
+  // Position of cut i (0 <= i <= records()), and the slot of its record.
+  __host__ __device__ int position(int i, int doubled) const {
+    const int cuts[8] = {64, 128, 256, 384, 768, 1280, 2048, 3072};
+    if (i < fixed) return cuts[i] << shift;
+    return ((i - fixed + 1) * unit << shift) << doubled;
+  }
+  __host__ __device__ int slot(int i, int doubled) const {
+    return i < fixed ? i
+                     : fixed + int((uint32_t(i - fixed + 1) << doubled) % uint32_t(spread));
+  }
+};
+// Every tile has room for all of its records, also one without a list, so that a
+// slot needs no counter and no pass before the walk; larger images, whose tiles
+// fill the chip in fewer segments, have fewer: 11 up to 26810 tiles (44 KB each),
+// 7 up to 42130 (16 views of 800 x 800 have 40000), 3 up to 98304, none beyond.
+inline WalkCuts walk_cuts(int num_tiles, int shift) {
+  const size_t most = kWalkRecordBytes / (size_t(kWalkPixels) * 16 * size_t(num_tiles));
+  return most >= 11  ? WalkCuts{8, 3, 4096, shift}
+         : most >= 7 ? WalkCuts{4, 3, 640, shift}
+         : most >= 3 ? WalkCuts{2, 1, 384, shift}
+                     : WalkCuts{0, 0, 0, shift};
 }
-// Every tile has room for all of its records (28 KB), also one without a list,
-// so that a slot needs no counter and no pass before the walk.  Images whose
-// records would take more than this (18724 tiles: 2189 x 2189 pixels) keep none
-// and walk back in quarters, which costs less there than the memory is worth: 8
-// views of 200k Gaussians in a small cube, 22500 tiles and 616 MB of records,
-// 1658 us a step, 1701 without.
-constexpr size_t kWalkRecordBytes = size_t(512) << 20;
-// The forward's waves also leave each quarter's largest contributor count:
-// keys[4 tile + quarter].
+inline size_t walk_record_bytes(int num_tiles) {
+  return size_t(num_tiles) * walk_cuts(num_tiles, 0).records() * kWalkPixels * 16;
+}
+// The forward's waves also leave each quarter's largest contributor count and
+// how often it doubled its spacing: keys[4 tile + quarter].
+inline size_t walk_key_bytes(int num_tiles) { return size_t(num_tiles) * 4 * 8; }
 
 // Dispatch plan of the compositing kernels (gs_tile_order).  Each of the 8
 // XCD regions of tiles (a contiguous range of tile indices) owns the same

@@ -22,8 +22,6 @@
 // them in one register, written by one nine-lane fp32 atomic add per (tile,
 // Gaussian).  Replaces composite_bwd.py:47-204 and the index_add_ scatter of
 // composite_bwd.py:268-273.
-#include <climits>
-
 #include "common.h"
 #include "raster_math.h"
 
@@ -61,10 +59,10 @@ struct CompositeBwdArgs {
   // The forward's hit masks (hit_mask_slot), read by the MASKS kernels.
   const uint64_t* hit_masks;
   int64_t hit_capacity;  // words
-  // WALK kernels: the forward's walk records and quarters' contributor counts.
+  // WALK kernels: the forward's walk records (WalkCuts) and quarters' keys.
   const float4* walk_records;
-  const int32_t* quarter_keys;
-  bool long_lists;  // walk_bound's
+  const int4* quarter_keys;  // two per tile
+  WalkCuts cuts;
 };
 
 // One wave takes PIX pixels per lane of `tile`: the 64-pixel bands band0 ..
@@ -86,9 +84,9 @@ struct CompositeBwdArgs {
 // RECORDS: the projection's 48-byte records are gathered (three 16-byte loads
 // of one or two lines, as the forward does) instead of the op's four projected
 // outputs.
-// WALK: segment `seg` between the forward's walk bounds instead, started from
-// its walk records (a pixel no longer active at the segment's end starts from
-// its final T, with nothing composited after it).  On few tiles a wave per tile
+// WALK: segment `seg` between the cuts of the forward's walk records instead,
+// started from the record at its end (a pixel no longer active there
+// starts from its final T, with nothing composited after it).  On few tiles a wave per tile
 // leaves SIMDs idle behind the longest walk, and a wave per quarter of the
 // tile's bands repeats each entry's fold, reduction and atomic up to four times:
 // quarters -> segments 218 -> 158 us (300k Gaussians, 1237 x 822), 112 -> 81
@@ -106,14 +104,17 @@ __device__ __forceinline__ void composite_bwd_tile(const CompositeBwdArgs& a, fl
   const int vx = tx / a.view_tw, vy = ty / a.view_th;
   const int view = vy * a.cols + vx;
   if (view >= a.views) return;  // an empty slot of the mosaic's last row
-  // WALK: nothing to do for a segment past the tile's largest contributor count.
-  const int walk_lo = WALK ? walk_bound(seg, a.list_shift, a.long_lists) : 0;
-  const int walk_hi = WALK && seg + 1 < kWalkSegments
-                          ? walk_bound(seg + 1, a.list_shift, a.long_lists)
-                          : INT_MAX;
+  // WALK: the tile's cuts are those of its quarters' largest spacing; nothing to
+  // do for a segment past its largest contributor count.
+  int walk_lo = 0, walk_hi = 0, walk_slot = 0;
   if constexpr (WALK) {
-    const int4 n4 = reinterpret_cast<const int4*>(a.quarter_keys)[tile];
-    if (max(max(n4.x, n4.y), max(n4.z, n4.w)) <= walk_lo) return;
+    const int4 k0 = a.quarter_keys[2 * tile], k1 = a.quarter_keys[2 * tile + 1];
+    const int doubled =
+        int(min(uint32_t(max(max(k0.y, k0.w), max(k1.y, k1.w))), kWalkMostDoubled));
+    if (seg > 0) walk_lo = a.cuts.position(seg - 1, doubled);
+    walk_hi = a.cuts.position(seg, doubled);
+    if (max(max(k0.x, k0.z), max(k1.x, k1.z)) <= walk_lo) return;
+    walk_slot = a.cuts.slot(seg, doubled);
   }
   const int ox = (tx - vx * a.view_tw) * TILE, oy = (ty - vy * a.view_th) * TILE;
   const int64_t view_base = int64_t(view) * a.width * a.height;  // first pixel of the view
@@ -169,7 +170,7 @@ __device__ __forceinline__ void composite_bwd_tile(const CompositeBwdArgs& a, fl
     hi = min(max_n, walk_hi);
     if (hi == walk_hi) {  // the walk goes on past this segment
       const float4* rec = a.walk_records +
-                          (int64_t(tile) * (kWalkSegments - 1) + seg) * kWalkPixels + lane;
+                          (int64_t(tile) * a.cuts.records() + walk_slot) * kWalkPixels + lane;
 #pragma unroll
       for (int p = 0; p < PIX; ++p) {
         if (ncon[p] > hi) {
@@ -397,7 +398,7 @@ __device__ __forceinline__ void composite_bwd_tile(const CompositeBwdArgs& a, fl
 
 // Tiles of the WALK kernel dealt to an XCD at a time (2^shift).
 constexpr int kWalkDealShift = 3;
-static_assert(kWalkSegments == 2 * kCompositeWaves, "two workgroups per tile");
+static_assert(kWalkSegments % kCompositeWaves == 0, "whole workgroups per tile");
 
 // kCompositeWaves waves per workgroup, one work item each (composite_item);
 // workgroups are mapped onto XCDs so that each XCD takes one region of the
@@ -420,15 +421,17 @@ __global__ __launch_bounds__(kCompositeWaves * 64) void composite_bwd_kernel(Com
   // broadcasts per entry instead of twelve v_readlane.
   __shared__ float4 chunk[kCompositeWaves][64][3];
   if constexpr (WALK) {
-    // A workgroup takes half of a tile's segments: all tiles' later halves
-    // first (few exist, but they are the long ones), then the earlier ones.
+    // A workgroup takes four of a tile's segments: all tiles' last ones first
+    // (few exist, but they are the long ones), the first ones at the end.
     // Interleaved, every second workgroup would have no work, and those with
     // work go to the same half of the shader engines (300k Gaussians at 1237 x
     // 822: 303 us).
-    const int half_grid = gridDim.x >> 1;
-    const bool later = int(blockIdx.x) < half_grid;
-    const int tile = xcd_deal(later ? blockIdx.x : blockIdx.x - half_grid, kWalkDealShift);
-    const int seg = (later ? kCompositeWaves : 0) + ((wid + tile) & (kCompositeWaves - 1));
+    const int groups = (a.cuts.records() + 1) / kCompositeWaves;  // per tile
+    const int grid = gridDim.x / groups;
+    const int group = blockIdx.x / grid;
+    const int tile = xcd_deal(blockIdx.x - group * grid, kWalkDealShift);
+    const int seg =
+        (groups - 1 - group) * kCompositeWaves + ((wid + tile) & (kCompositeWaves - 1));
     if (tile < a.num_tiles)
       composite_bwd_tile<TILE, ABS, PIX_TILE, MASKS, RECORDS, true>(a, chunk[wid], lane, tile, 0,
                                                                     seg);
@@ -459,9 +462,10 @@ void launch_masks(const CompositeBwdArgs& a, unsigned blocks, hipStream_t s) {
   if constexpr (MASKS && TILE >= 16) {  // image calls (gs_composite_bwd_image)
     if constexpr (TILE == 16 && QUARTERS) {
       if (a.walk_records) {
+        const int groups = (a.cuts.records() + 1) / kCompositeWaves;  // per tile
         launch_timed(composite_bwd_kernel<16, false, false, true, true, true>,
-                     unsigned(2 * deal_grid(a.num_tiles, kWalkDealShift)), kCompositeWaves * 64, 0,
-                     s, a);
+                     unsigned(groups * deal_grid(a.num_tiles, kWalkDealShift)),
+                     kCompositeWaves * 64, 0, s, a);
         return;
       }
     }
@@ -515,7 +519,7 @@ int composite_bwd(const float* projected_mean, const float* inverse_covariance,
                   const int32_t* tile_order, gs_view view, float* grad_projected,
                   float* grad_absolute, const void* checkpoints, size_t checkpoint_bytes,
                   int64_t num_intersections, const uint64_t* hit_masks, size_t hit_mask_bytes,
-                  const void* walk, size_t walk_bytes, int64_t longest_list, void* stream) {
+                  const void* walk, size_t walk_bytes, void* stream) {
   GS_TRY(check_view(view, true));
   GS_REQUIRE(view.rendering_mode == GS_MODE_GAUSSIAN, GS_ERR_UNSUPPORTED,
              "Backward gradients are only supported for Gaussian rendering.");
@@ -576,14 +580,15 @@ int composite_bwd(const float* projected_mean, const float* inverse_covariance,
   }
   a.walk_records = nullptr;
   a.quarter_keys = nullptr;
-  a.long_lists = longest_list > kCheckpointMinList;
+  a.cuts = WalkCuts{};
   if (walk) {
     const size_t need = gs_composite_walk_bytes(view);
     GS_REQUIRE(need > 0 && walk_bytes >= need, GS_ERR_WORKSPACE,
                "walk buffer too small (%zu bytes, need %zu)", walk_bytes, need);
     a.walk_records = static_cast<const float4*>(walk);
-    a.quarter_keys = reinterpret_cast<const int32_t*>(static_cast<const char*>(walk) +
-                                                      walk_record_bytes(a.num_tiles));
+    a.quarter_keys = reinterpret_cast<const int4*>(static_cast<const char*>(walk) +
+                                                   walk_record_bytes(a.num_tiles));
+    a.cuts = walk_cuts(a.num_tiles, m.shift);
   }
   a.ckpt_stamp = nullptr;
   a.ckpt_table_len = 0;
@@ -632,7 +637,7 @@ extern "C" GS_API int gs_composite_bwd(const float* projected_mean,
                        nullptr, n, gaussian_ids, ranges, grad_image, final_transmittance,
                        n_contributors, tile_order, view, grad_projected, grad_absolute,
                        checkpoints, checkpoint_bytes, num_intersections, hit_masks,
-                       hit_mask_bytes, nullptr, 0, 0, stream);
+                       hit_mask_bytes, nullptr, 0, stream);
 }
 
 extern "C" GS_API int gs_composite_bwd_image(
@@ -640,7 +645,7 @@ extern "C" GS_API int gs_composite_bwd_image(
     const float* grad_image, const float* final_transmittance, const int32_t* n_contributors,
     const int32_t* tile_order, gs_view view, float* grad_projected, int64_t num_intersections,
     const uint64_t* hit_masks, size_t hit_mask_bytes, const void* walk, size_t walk_bytes,
-    int64_t longest_list, void* stream) {
+    void* stream) {
   clear_error();
   GS_REQUIRE(view.tile_size >= 16, GS_ERR_UNSUPPORTED,
              "image calls composite tiles of 16 or 32 pixels (got %d)", view.tile_size);
@@ -649,5 +654,5 @@ extern "C" GS_API int gs_composite_bwd_image(
                        static_cast<const GsRecord*>(records), n, gaussian_ids, ranges, grad_image,
                        final_transmittance, n_contributors, tile_order, view, grad_projected,
                        nullptr, nullptr, 0, num_intersections, hit_masks, hit_mask_bytes, walk,
-                       walk_bytes, longest_list, stream);
+                       walk_bytes, stream);
 }

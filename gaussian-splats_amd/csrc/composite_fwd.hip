@@ -57,11 +57,10 @@ struct CompositeArgs {
   // checkpoints a backward walk crosses), written by whole-tile walks; or
   // null: none.
   uint32_t* tile_keys;
-  // Walk records of quarter waves (walk_bound) and, per quarter, the largest
-  // contributor count; or null: none.
+  // Walk records of quarter waves (WalkCuts) and their keys; or null: none.
   float4* walk_records;
-  int32_t* quarter_keys;
-  bool long_lists;  // walk_bound's
+  int2* quarter_keys;
+  WalkCuts cuts;
   int deal_shift;  // without a plan: chunk of workgroups dealt to an XCD (negative: contiguous)
 };
 
@@ -166,29 +165,46 @@ __device__ __forceinline__ void composite_tile(const CompositeArgs& a, float4 (*
     ++ck_count;
     ck_next = ck_count < kMaxCheckpoints ? checkpoint_batch(start, ck_count + 1) : -1;
   };
-  // Quarter waves with walk records: at each bound of the walk (a batch start)
-  // the pixels' T and the colour since the previous record, summed beside the
-  // image's own sum (pr, pg, pb; the first record's is the image's), so that
-  // the image does not depend on the records.
+  // Quarter waves with walk records: at each cut (a batch start) the pixels' T
+  // and the colour since the previous record, summed beside the image's own sum
+  // (pr, pg, pb; the first record's is the image's), so that the image does not
+  // depend on the records.
   constexpr bool kRecords = HITS && TILE == 16 && PIX == 1;
-  int walk_count = 0, walk_next = -1;
+  int walk_count = 0, walk_doubled = 0, walk_next = -1;
   float pr = 0.0f, pg = 0.0f, pb = 0.0f;
-  if constexpr (kRecords)
-    walk_next = a.walk_records ? walk_bound(1, a.list_shift, a.long_lists) : -1;
-  float4* const walk =
-      kRecords ? a.walk_records + int64_t(tile) * (kWalkSegments - 1) * kWalkPixels + 64 * band0 +
-                     lane
-               : nullptr;
+  if constexpr (kRecords) walk_next = a.walk_records ? a.cuts.position(0, 0) : -1;
+  auto walk_record = [&](int i) {
+    return a.walk_records + 64 * band0 + lane +
+           (int64_t(tile) * a.cuts.records() + a.cuts.slot(i, walk_doubled)) * kWalkPixels;
+  };
   auto record_at = [&](int bpos) {
     if constexpr (kRecords) {
       if (bpos != walk_next) return;
-      walk[walk_count * kWalkPixels] =
-          walk_count == 0 ? make_float4(T[0], cr[0], cg[0], cb[0]) : make_float4(T[0], pr, pg, pb);
+      float4 now = walk_count == 0 ? make_float4(T[0], cr[0], cg[0], cb[0])
+                                   : make_float4(T[0], pr, pg, pb);
+      if (walk_count == a.cuts.records()) {
+        // Odd multiples of the spacing go, their colours to the next record
+        // (the last one's to the record written below, in the first one's slot).
+        for (int i = a.cuts.fixed; i + 1 < walk_count; i += 2) {
+          const float4 gone = *walk_record(i);
+          float4 kept = *walk_record(i + 1);
+          kept.y += gone.y;
+          kept.z += gone.z;
+          kept.w += gone.w;
+          *walk_record(i + 1) = kept;
+        }
+        const float4 last = *walk_record(walk_count - 1);
+        now.y += last.y;
+        now.z += last.z;
+        now.w += last.w;
+        walk_count = a.cuts.fixed + (a.cuts.spread >> 1);
+        ++walk_doubled;
+      }
+      *walk_record(walk_count) = now;
       pr = pg = pb = 0.0f;
       ++walk_count;
-      walk_next = walk_count + 1 < kWalkSegments
-                      ? walk_bound(walk_count + 1, a.list_shift, a.long_lists)
-                      : -1;
+      // The next cut of this spacing; past the last one, the one that doubles it.
+      walk_next = a.cuts.position(walk_count, walk_doubled);
     }
   };
   // The overlap test's rectangle: the columns and rows of the pixels still
@@ -395,9 +411,9 @@ __device__ __forceinline__ void composite_tile(const CompositeArgs& a, float4 (*
   }
 
   if constexpr (kRecords) {
-    for (int j = walk_count - 1; j >= 0; --j) {
-      const float4 v = walk[j * kWalkPixels];
-      walk[j * kWalkPixels] = make_float4(v.x, pr, pg, pb);
+    for (int i = walk_count - 1; i >= 0; --i) {
+      const float4 v = *walk_record(i);
+      *walk_record(i) = make_float4(v.x, pr, pg, pb);
       pr += v.y;
       pg += v.z;
       pb += v.w;
@@ -406,7 +422,7 @@ __device__ __forceinline__ void composite_tile(const CompositeArgs& a, float4 (*
       int m = ncon[0];
 #pragma unroll
       for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o, 64));
-      if (lane == 0) a.quarter_keys[tile * 4 + band0] = m;
+      if (lane == 0) a.quarter_keys[tile * 4 + band0] = make_int2(m, walk_doubled);
     }
   }
 
@@ -566,14 +582,13 @@ extern "C" GS_API size_t gs_composite_hit_mask_bytes(gs_view view, int64_t num_i
 
 namespace {
 
-// `longest_list` (0: unknown) selects the bounds of the walk records.
 int composite(const void* records, int64_t num_records, const int32_t* gaussian_ids,
-              int64_t num_intersections, int64_t longest_list, const int64_t* ranges,
-              const int32_t* tile_order, gs_view view, float* image,
+              int64_t num_intersections, const int64_t* ranges, const int32_t* tile_order,
+              gs_view view, float* image,
               float* final_transmittance, int32_t* n_contributors,
               void* checkpoints, size_t checkpoint_bytes, uint64_t* hit_masks,
               size_t hit_mask_bytes, uint32_t* tile_keys, size_t tile_keys_bytes,
-              void* walk_records, int32_t* quarter_keys, void* stream) {
+              void* walk_records, void* quarter_keys, void* stream) {
   GS_TRY(check_view(view, true));
   GS_REQUIRE(ranges && image, GS_ERR_INVALID_ARGUMENT, "null pointer argument");
   GS_REQUIRE(num_records >= 0 && num_records <= (int64_t(1) << 31), GS_ERR_INVALID_ARGUMENT,
@@ -620,8 +635,8 @@ int composite(const void* records, int64_t num_records, const int32_t* gaussian_
   // backward's plan computes them itself.
   a.tile_keys = plan.split_all ? nullptr : tile_keys;
   a.walk_records = plan.split_all ? static_cast<float4*>(walk_records) : nullptr;
-  a.quarter_keys = quarter_keys;
-  a.long_lists = longest_list > kCheckpointMinList;
+  a.quarter_keys = static_cast<int2*>(quarter_keys);
+  a.cuts = walk_cuts(a.num_tiles, m.shift);
   a.deal_shift = a.num_tiles <= kDealTiles ? kDealShift : -1;
   if (hit_masks) {
     GS_REQUIRE(view.rendering_mode == GS_MODE_GAUSSIAN, GS_ERR_UNSUPPORTED,
@@ -684,7 +699,7 @@ extern "C" GS_API int gs_composite(const void* records, int64_t num_records,
   GS_TRY(check_view(view, true));
   GS_REQUIRE(final_transmittance && n_contributors, GS_ERR_INVALID_ARGUMENT,
              "null pointer argument");
-  return composite(records, num_records, gaussian_ids, num_intersections, 0, ranges, tile_order,
+  return composite(records, num_records, gaussian_ids, num_intersections, ranges, tile_order,
                    view, image, final_transmittance, n_contributors, checkpoints,
                    checkpoint_bytes, hit_masks, hit_mask_bytes, tile_keys, tile_keys_bytes,
                    nullptr, nullptr, stream);
@@ -695,7 +710,7 @@ extern "C" GS_API int gs_composite_image(const void* records, int64_t num_record
                                          const int64_t* ranges, gs_view view, float* image,
                                          void* stream) {
   clear_error();
-  return composite(records, num_records, gaussian_ids, num_intersections, 0, ranges, nullptr, view,
+  return composite(records, num_records, gaussian_ids, num_intersections, ranges, nullptr, view,
                    image, nullptr, nullptr, nullptr, 0, nullptr, 0, nullptr, 0,
                    nullptr, nullptr, stream);
 }
@@ -704,29 +719,27 @@ extern "C" GS_API size_t gs_composite_walk_bytes(gs_view view) {
   if (check_view(view, true) != GS_OK || view.tile_size != 16) return 0;
   const Mosaic m = mosaic_of(view);
   if (!dispatch_plan(m.num_tiles(), view, false).split_all) return 0;
-  if (walk_record_bytes(m.num_tiles()) > kWalkRecordBytes) return 0;
-  return walk_record_bytes(m.num_tiles()) + align_up(size_t(m.num_tiles()) * 16);
+  if (walk_cuts(m.num_tiles(), 0).records() == 0) return 0;
+  return walk_record_bytes(m.num_tiles()) + walk_key_bytes(m.num_tiles());
 }
 
 extern "C" GS_API int gs_composite_walk(
     const void* records, int64_t num_records, const int32_t* gaussian_ids,
-    int64_t num_intersections, int64_t longest_list, const int64_t* ranges, gs_view view,
-    float* image, float* final_transmittance, int32_t* n_contributors, uint64_t* hit_masks,
+    int64_t num_intersections, const int64_t* ranges, gs_view view, float* image,
+    float* final_transmittance, int32_t* n_contributors, uint64_t* hit_masks,
     size_t hit_mask_bytes, void* walk, size_t walk_bytes, void* stream) {
   clear_error();
   const size_t need = gs_composite_walk_bytes(view);
   GS_REQUIRE(need > 0 && view.rendering_mode == GS_MODE_GAUSSIAN, GS_ERR_UNSUPPORTED,
-             "walk records are for Gaussian rendering on few tiles of 16 pixels, up to %zu bytes",
-             kWalkRecordBytes);
+             "walk records are for Gaussian rendering on few tiles of 16 pixels");
   GS_REQUIRE(final_transmittance && n_contributors && hit_masks && walk, GS_ERR_INVALID_ARGUMENT,
              "null pointer argument");
   GS_REQUIRE(walk_bytes >= need, GS_ERR_WORKSPACE,
              "walk buffer too small (%zu bytes, need %zu)", walk_bytes, need);
   GS_REQUIRE((reinterpret_cast<uintptr_t>(walk) & 15u) == 0, GS_ERR_INVALID_ARGUMENT,
              "the walk buffer must be 16-byte aligned");
-  int32_t* keys = reinterpret_cast<int32_t*>(static_cast<char*>(walk) +
-                                             walk_record_bytes(mosaic_of(view).num_tiles()));
-  return composite(records, num_records, gaussian_ids, num_intersections, longest_list, ranges,
-                   nullptr, view, image, final_transmittance, n_contributors, nullptr, 0, hit_masks,
+  void* keys = static_cast<char*>(walk) + walk_record_bytes(mosaic_of(view).num_tiles());
+  return composite(records, num_records, gaussian_ids, num_intersections, ranges, nullptr, view,
+                   image, final_transmittance, n_contributors, nullptr, 0, hit_masks,
                    hit_mask_bytes, nullptr, 0, walk, keys, stream);
 }

@@ -15,7 +15,7 @@ from pathlib import Path
 import torch
 
 LIB_PATH = Path(__file__).resolve().parents[2] / "_lib" / "libgs_raster.so"
-ABI_VERSION = 20
+ABI_VERSION = 21
 
 GS_OK = 0
 GS_ERR_INVALID_ARGUMENT = 1
@@ -311,12 +311,12 @@ _SIGNATURES = {
     "gs_composite_bwd_image": (
         c_int,
         [c_void_p, c_int64] + [c_void_p] * 6
-        + [GsView, c_void_p, c_int64, c_void_p, c_size_t, c_void_p, c_size_t, c_int64, c_void_p],
+        + [GsView, c_void_p, c_int64, c_void_p, c_size_t, c_void_p, c_size_t, c_void_p],
     ),
     "gs_composite_walk_bytes": (c_size_t, [GsView]),
     "gs_composite_walk": (
         c_int,
-        [c_void_p, c_int64, c_void_p, c_int64, c_int64, c_void_p, GsView] + [c_void_p] * 4
+        [c_void_p, c_int64, c_void_p, c_int64, c_void_p, GsView] + [c_void_p] * 4
         + [c_size_t, c_void_p, c_size_t, c_void_p],
     ),
     "gs_device_errors": (c_int, [c_void_p, c_int32, c_void_p]),

@@ -149,7 +149,7 @@ class _Walk:
     hold everything of size but the accumulator (the backward takes that), so
     that a backward which does not retain the graph frees it."""
 
-    __slots__ = ("view", "accumulator", "longest")
+    __slots__ = ("view", "accumulator")
 
 
 def small_lists(depth_keys, tile_rects, tiles_w, tiles_h, nbytes, clear=None):
@@ -238,12 +238,12 @@ def forward_image(params, request: ImageRequest, keep: bool, timer=None):
     order = walk_records = None
     walk_bytes = lib.gs_composite_walk_bytes(view)
     if walk_bytes:
-        # Few tiles with work: the walk's state at fixed positions, for a backward
-        # in segments (no plan: the segments are dealt in tile order).
+        # Every tile split: the walk's state at some positions, for a backward in
+        # segments (no plan: the segments are dealt in tile order).
         walk_records = nat.workspace(walk_bytes, device)
         nat.check(
             nat.launch("composite", lambda: lib.gs_composite_walk(
-                ptr(records), vn, ptr(ids), total, longest, ptr(ranges), view, ptr(image),
+                ptr(records), vn, ptr(ids), total, ptr(ranges), view, ptr(image),
                 ptr(final_transmittance), ptr(n_contributors), ptr(hits), nat.buffer_bytes(hits),
                 ptr(walk_records), walk_bytes, stream,
             )),
@@ -269,7 +269,7 @@ def forward_image(params, request: ImageRequest, keep: bool, timer=None):
             "tile_order",
         )
     walk = _Walk()
-    walk.view, walk.accumulator, walk.longest = view, accumulator, longest
+    walk.view, walk.accumulator = view, accumulator
     saved = (records, tile_rects, ids, ranges, final_transmittance, n_contributors, hits, order,
              walk_records)
     return image, saved, walk
@@ -303,7 +303,7 @@ def backward_image(params, saved, walk: _Walk, request: ImageRequest, grad_image
             ptr(records), records.shape[0], ptr(ids), ptr(ranges), ptr(grad_image),
             ptr(final_transmittance), ptr(n_contributors), ptr(order), walk.view,
             ptr(accumulator), ids.numel(), ptr(hits), nat.buffer_bytes(hits), ptr(walk_records),
-            nat.buffer_bytes(walk_records), walk.longest, stream,
+            nat.buffer_bytes(walk_records), stream,
         )),
         "composite_bwd_image",
     )

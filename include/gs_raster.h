@@ -42,7 +42,7 @@ extern "C" {
 
 #define GS_API __attribute__((visibility("default")))
 
-#define GS_ABI_VERSION 20
+#define GS_ABI_VERSION 21
 
 typedef enum gs_status {
   GS_OK = 0,
@@ -440,18 +440,16 @@ GS_API int gs_composite_image(
 
 /* gs_composite for a Gaussian image call on tiles of 16 pixels whose bands are
  * split over four waves each (fewer than 4096 tiles with work, or
- * view.split_tiles), which also records the walk's state at fixed positions, so that
- * gs_composite_bwd_image walks each tile back in segments of all of its
- * pixels.  longest_list (totals[3] of gs_bin_tiles_plan, 0: unknown) sets how
- * far apart the positions are and must be the same in both calls.
- * gs_composite_walk_bytes: the size of `walk`, at most 512 MiB and 16 bytes per
- * tile, or 0 when the view is not of that kind or has too many tiles for it
- * (GS_ERR_UNSUPPORTED). */
+ * view.split_tiles), which also records the walk's state at up to 11 positions
+ * per tile, so that gs_composite_bwd_image walks each tile back in segments of
+ * all of its pixels.  gs_composite_walk_bytes: the size of `walk`, at most 1152
+ * MiB of records and 32 bytes per tile (larger images keep fewer records per
+ * tile), or 0 when the view is not of that kind (GS_ERR_UNSUPPORTED). */
 GS_API size_t gs_composite_walk_bytes(gs_view view);
 GS_API int gs_composite_walk(
     const void* records, int64_t num_records, const int32_t* gaussian_ids,
-    int64_t num_intersections, int64_t longest_list, const int64_t* ranges, gs_view view,
-    float* image, float* final_transmittance, int32_t* n_contributors, uint64_t* hit_masks,
+    int64_t num_intersections, const int64_t* ranges, gs_view view, float* image,
+    float* final_transmittance, int32_t* n_contributors, uint64_t* hit_masks,
     size_t hit_mask_bytes, void* walk, size_t walk_bytes, void* stream);
 
 /* Back-to-front compositing gradient, accumulated with atomics into
@@ -493,7 +491,7 @@ GS_API int gs_composite_bwd_image(
     const float* grad_image, const float* final_transmittance, const int32_t* n_contributors,
     const int32_t* tile_order, gs_view view, float* grad_projected, int64_t num_intersections,
     const uint64_t* hit_masks, size_t hit_mask_bytes, const void* walk, size_t walk_bytes,
-    int64_t longest_list, void* stream);
+    void* stream);
 
 /* Chain rule from grad_projected to the parameters.  Replaces project_bwd
  * (src/gaussian_splats/kernels/rasterize/project_bwd.py:8-381); gradients are

@@ -232,18 +232,25 @@ def test_hit_masks_host_checks():
 
 
 def test_walk_records_are_bounded():
-    """gs_composite_walk_bytes: 7 records of 4 KiB and 16 bytes of keys per tile,
-    never above 512 MiB of records; other views keep none."""
+    """gs_composite_walk_bytes: 11 records of 4 KiB and 32 bytes of keys per tile,
+    fewer records in larger images, never above 1152 MiB of records; views that
+    are not split keep none."""
     lib = nat.library()
-    size = lambda w, h, **kw: lib.gs_composite_walk_bytes(
-        _view(image_width=w, image_height=h, active_tiles=100, **kw))
-    assert size(100, 100) == 49 * 7 * 4096 + 1024
-    most = size(151 * 16, 124 * 16)
-    assert most == 18724 * 7 * 4096 + 18724 * 16 + 192
-    assert most - 18724 * 16 - 192 <= 512 << 20
-    assert size(175 * 16, 107 * 16) == 0  # 18725 tiles
-    assert size(4096, 4096) == 0 and size(800, 800, views=16, mosaic_cols=4) == 0
-    assert size(100, 100, tile_size=32) == 0 and size(1920, 1080, list_shift=1) > 0
+
+    def size(tw, th, active_tiles=100, **kw):
+        return lib.gs_composite_walk_bytes(_view(
+            image_width=tw * 16, image_height=th * 16, active_tiles=active_tiles, **kw))
+
+    for tw, th, records in ((7, 7, 11), (7 * 5, 2 * 383, 11), (197, 137, 7), (110, 383, 7),
+                            (253, 167, 3), (256, 256, 3), (1024, 96, 3), (1024, 97, 0)):
+        want = tw * th * (records * 4096 + 32) if records else 0
+        assert size(tw, th) == want
+        assert records * 4096 * tw * th <= 1152 << 20
+    assert size(50, 50, views=16, mosaic_cols=4) == 40000 * (7 * 4096 + 32)
+    assert size(100, 100, active_tiles=0) == 0
+    assert size(100, 100, active_tiles=0, split_tiles=1) == 10000 * (11 * 4096 + 32)
+    assert size(120, 68, list_shift=1) == 8160 * (11 * 4096 + 32)
+    assert lib.gs_composite_walk_bytes(_view(tile_size=32, active_tiles=100)) == 0
 
 
 def test_misaligned_buffers_rejected():

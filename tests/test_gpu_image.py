@@ -4,6 +4,8 @@ gradients equal up to the order of their sums."""
 
 from __future__ import annotations
 
+import math
+
 import pytest
 import torch
 
@@ -165,31 +167,54 @@ def test_image_walk_segments(size, n, device):
     _same_gradients(second, [p.grad for p in leaves])
 
 
-def _cluster(n, size, spread=0.1):
-    """Gaussians in the middle of a large image: few of its tiles have work."""
-    scene = scenes.edge_case_scene(n=n, sh_degree=0, image_size=size, seed=8)
+def _points(n, size, spread):
+    """Faint Gaussians of half a pixel in ``spread`` pixels around the middle: each
+    pixel takes few entries of its tile's long list.  Ten wide opaque ones lie
+    across them halfway into the list, a little below the middle, so the tiles'
+    quarters walk to different depths."""
+    scene = scenes.edge_case_scene(n=n, sh_degree=1, image_size=size, seed=8)
     g = torch.Generator().manual_seed(n)
-    scene.mean[:, :2] = torch.randn(n, 2, generator=g) * spread
-    scene.mean[:, 2] = -(torch.rand(n, generator=g) + 4)
-    scene.scale[:] = torch.rand(n, 3, generator=g) - 5
+    pixel = 5 / (0.75 * size[0])
+    scene.mean[:, :2] = torch.randn(n, 2, generator=g) * spread * pixel
+    scene.mean[:, 2] = -(torch.rand(n, generator=g) * 0.1 + 5)
+    scene.scale[:] = math.log(0.5 * pixel) + torch.tensor([-0.5, 0.5, 0.0])
+    scene.opacity[:] = torch.randn(n, 1, generator=g) * 0.3 - 4.5
+    scene.mean[-10:] = torch.tensor([0.0, -2 * pixel, -5.05])
+    scene.rotation[-10:] = torch.tensor([1.0, 0.0, 0.0, 0.0])
+    scene.scale[-10:] = torch.log(torch.tensor([60.0, 6.0, 1.0]) * pixel)
+    scene.opacity[-10:] = 6.0
     return scene
 
 
-def test_image_few_tiles_of_too_many(device):
-    """More tiles than the walk records' bound, few with work: every tile split
-    into quarters in both directions, without records."""
-    scene = _cluster(9000, (4096, 1200)).to(device)
+@pytest.mark.parametrize("size,n,spread", [((24, 24), 24_000, 2.0), ((40, 24), 90_000, 3.0),
+                                           ((1111, 1043), 60_000, 8.0),
+                                           ((4096, 1712), 20_000, 8.0),
+                                           ((4096, 2816), 20_000, 8.0)])
+def test_image_long_walks(size, n, spread, device):
+    """Walks that drop records and double their spacing, in images of 11, 7 and 3
+    records per tile, with and without shared lists."""
+    scene = _points(n, size, spread).to(device)
+    cam = scene.cameras[0]
     splats = GaussianSplat.from_tensors(*scene.params())
     leaves = [p.detach().clone().requires_grad_(True) for p in scene.params()]
-    image = rasterize(splats, scene.cameras[0], near=scene.near, far=scene.far)
-    order, walk_records = image.grad_fn.saved_tensors[-2:]
-    assert walk_records is None and (order[order >= 0] & 0x20).all()
-    expected = _op(scene, leaves, scene.cameras[0], 16, "gaussian")
+    image = rasterize(splats, cam, near=scene.near, far=scene.far)
+    walk_records = image.grad_fn.saved_tensors[-1]
+    tiles = -(-size[0] // 16) * -(-size[1] // 16)
+    records = {True: 11, False: 7 if tiles < 42_130 else 3}[tiles < 26_810]
+    padded = walk_records.numel() // (records * 4096 + 32)
+    assert walk_records.numel() == padded * (records * 4096 + 32) and padded >= tiles
+    keys = walk_records[padded * records * 4096:].view(torch.int32).reshape(padded, 4, 2)
+    expected = _op(scene, leaves, cam, 16, "gaussian")
     assert torch.equal(image, expected)
-    weight = torch.linspace(-1, 1, image.numel(), device=device).reshape(image.shape)
+    # Without a symmetry that the wide Gaussians' rotation gradients, odd moments
+    # over their pixels, would cancel by.
+    weight = torch.randn(image.shape, device=device, generator=torch.Generator(device).manual_seed(n))
     (image * weight).sum().backward()
     (expected * weight).sum().backward()
     _same_gradients([getattr(splats, n).grad for n in PARAMS], [p.grad for p in leaves])
+    # The spacing has doubled, and not equally often in a tile's quarters.
+    doubled = keys[..., 1]
+    assert doubled.max() >= 1 and (doubled.amax(1) != doubled.amin(1)).any()
 
 
 def test_views_image_equals_op(device):
@@ -255,7 +280,7 @@ def test_saved_tensor_hooks(device):
 
 def test_backward_frees_the_walk(device):
     """A backward that does not retain the graph frees what the forward kept for
-    it (here 34 MB of walk records), also while the image is held."""
+    it (here 54 MB of walk records), also while the image is held."""
     scene = scenes.edge_case_scene(n=500, image_size=(640, 480)).to(device)
     splats = GaussianSplat.from_tensors(*scene.params())
     held = []
@@ -266,7 +291,7 @@ def test_backward_frees_the_walk(device):
         kept = torch.cuda.memory_allocated() - before
         image.sum().backward()
         held.append(torch.cuda.memory_allocated() - before)
-    assert kept > 30 << 20
+    assert kept > 50 << 20
     assert held[1] <= image.numel() * 4 + (1 << 20)
 
 
