@@ -75,21 +75,6 @@ def image_tile(asked: int, width: int, height: int, n: int, views: int = 1) -> i
     return None
 
 
-def split_long_lists(longest: int, entries: int, lists: int, tiles: int) -> bool:
-    """Whether an image call's tiles are split over four waves each although
-    ``tiles`` of them (SPLIT_TILES or more) have work: the lists are long (the
-    ``longest`` one, and the mean of ``entries`` in ``lists`` non-empty ones
-    above a third of the tiles), so the longest walk sets the time of a launch,
-    not the number of waves.  A step with a wave per tile and with four: 80k
-    Gaussians in a small cube on 4704 tiles (mean list half of them) 963 and 792
-    us, 2M on 7272 tiles 1988 and 1863, a shell of 2M in four views on 10824
-    tiles (mean 0.75 of them) 5359 and 4820.  A few long lists are no reason: 1M
-    at 1080p with one dense spot (mean 0.29) 682 and 762, 1M at 3840 x 2160 with
-    one (0.05) 1274 and 1628.  Nor are long ones on many tiles: 2M in a small
-    cube on 13300 tiles 2399 and 2580."""
-    return longest > LONG_LIST and tiles < 3 * SPLIT_TILES and 3 * entries > lists * tiles
-
-
 class ImageRequest:
     """Everything but the Gaussians of an image call on ``n`` of them: the
     ``cameras`` (``camera_floats`` of ``views`` of them), the views and the
@@ -207,7 +192,10 @@ def forward_image(params, request: ImageRequest, keep: bool, timer=None):
     if request.small:
         ids, ranges = small_lists(depth_keys, tile_rects, tiles_w, tiles_h, request.small,
                                   accumulator)
-        longest = 0  # unknown to the host; too few Gaussians or tiles for checkpoints
+        # Unknown to the host; a list may hold them all.  An image alone is not
+        # split for that (14k Gaussians at 1111 x 1043: 109 us, 117 split; with a
+        # backward 324 and 308, and 5043 and 1656 where a list does hold 10k).
+        longest = n if backward else 0
         mark("bin")
         mark("emit")
     else:
@@ -218,9 +206,14 @@ def forward_image(params, request: ImageRequest, keep: bool, timer=None):
         longest = nat.longest_list(ranges)
     mark("sort")
     subs = 1 << (2 * view.list_shift)  # compositing tiles per list
-    lists = nat.active_tiles(ranges)
-    view.active_tiles = lists * subs
-    view.split_tiles = split_long_lists(longest, ids.numel(), lists, lists * subs)
+    view.active_tiles = nat.active_tiles(ranges) * subs
+    # With a long list the longest walk may set the time of a launch: its tiles
+    # are split over four waves however many have work.  Whether it does is not
+    # known before the walk.  1M Gaussians at 1080p with a dense spot, a step with
+    # a wave per tile and with four: 652 and 743 us where the spot's pixels
+    # saturate after some hundred entries, 10.9 and 4.5 ms where they do not; 80k
+    # in a small cube on 4704 tiles 963 and 804.
+    view.split_tiles = longest > LONG_LIST
     num_tiles, total = tiles_w * tiles_h * subs, ids.numel()
     image = torch.empty(request.shape, dtype=torch.float32, device=device)
     if not backward:

@@ -295,33 +295,22 @@ def test_backward_frees_the_walk(device):
     assert held[1] <= image.numel() * 4 + (1 << 20)
 
 
-def test_split_long_lists_rule():
-    from gaussian_splats_hip.kernels.rasterize.image import split_long_lists
-
-    assert split_long_lists(8193, 8_000_000, 1500, 6000)
-    assert not split_long_lists(8192, 8_000_000, 1500, 6000)
-    # One long list among many short ones, and long lists on many tiles.
-    assert not split_long_lists(26_170, 4_796_677, 2040, 8160)
-    assert not split_long_lists(470_000, 53_000_000, 3325, 13_300)
-
-
-def test_image_one_long_list(device):
+@pytest.mark.parametrize("n", [40_000, 14_000])
+def test_image_one_long_list(n, device):
     """One list above 8192 entries among many short ones (faint Gaussians in
-    front of the others): a wave per tile without records, against the op's
-    checkpointed walk."""
-    scene = scenes.edge_case_scene(n=40_000, sh_degree=0, image_size=(1920, 1080), seed=6)
+    front of the others) on more than 4096 tiles, its length known to the host
+    (bucketing) or not (small scenes): four waves per tile and walk records."""
+    scene = scenes.edge_case_scene(n=n, sh_degree=0, image_size=(1111, 1043), seed=6)
     g = torch.Generator().manual_seed(4)
-    scene.mean[20_000:] = torch.tensor([0.05, 0.03, -0.8]) + torch.randn(20_000, 3, generator=g) * 0.002
-    scene.scale[20_000:], scene.opacity[20_000:] = -6.0, -5.3
+    m = n - 10_000
+    scene.mean[m:] = torch.tensor([0.05, 0.03, -0.8]) + torch.randn(10_000, 3, generator=g) * 0.002
+    scene.scale[m:], scene.opacity[m:] = -6.0, -5.3
     scene = scene.to(device)
     splats = GaussianSplat.from_tensors(*scene.params())
     leaves = [p.detach().clone().requires_grad_(True) for p in scene.params()]
     image = rasterize(splats, scene.cameras[0], near=scene.near, far=scene.far)
-    ranges, order, walk_records = (image.grad_fn.saved_tensors[i] for i in (8, -2, -1))
-    assert (ranges[:, 1] - ranges[:, 0]).max() > 8192
-    assert walk_records is None
-    # Whole tiles: without checkpoints no walk is cut into segments.
-    assert torch.equal(order[order >= 0] & 0x7F, torch.zeros_like(order[order >= 0]))
+    ranges, walk_records = (image.grad_fn.saved_tensors[i] for i in (8, -1))
+    assert (ranges[:, 1] - ranges[:, 0]).max() > 8192 and walk_records is not None
     expected = _op(scene, leaves, scene.cameras[0], 16, "gaussian")
     # The op's checkpoints cut a pixel's colour into partial sums (see below).
     assert (image - expected).abs().max() < 64 * 4 * 2.0 ** -24
@@ -329,6 +318,33 @@ def test_image_one_long_list(device):
     (image * weight).sum().backward()
     (expected * weight).sum().backward()
     _same_gradients([getattr(splats, n).grad for n in PARAMS], [p.grad for p in leaves])
+
+
+def test_plan_without_checkpoints(device):
+    """A whole-tile forward without a checkpoint buffer leaves keys of a plan
+    without segments, also for lists above 8192 entries."""
+    from gaussian_splats_hip.kernels.rasterize import _native as nat
+
+    w, h = 1111, 1043
+    scene = _points(60_000, (w, h), 8.0).to(device)
+    splats = GaussianSplat.from_tensors(*scene.params())
+    image = rasterize(splats, scene.cameras[0], near=scene.near, far=scene.far)
+    records, _, ids, ranges = image.grad_fn.saved_tensors[5:9]
+    assert (ranges[:, 1] - ranges[:, 0]).max() > 8192
+    view = nat.make_view(1.0, 1.0, 0.0, 0.0, w, h, 16, opacity_threshold=0.999, list_shift=1)
+    out = [torch.empty((h, w, 3), device=device), torch.empty((h, w), device=device)]
+    ncon = torch.empty((h, w), dtype=torch.int32, device=device)
+    keys = nat.workspace(nat.library().gs_tile_order_workspace_bytes(4 * ranges.shape[0]), device)
+    lib, ptr, stream = nat.library(), nat.ptr, nat.stream(device)
+    nat.check(lib.gs_composite(
+        ptr(records), records.shape[0], ptr(ids), ids.numel(), ptr(ranges), None, view,
+        *map(ptr, out), ptr(ncon), None, 0, None, 0, ptr(keys), keys.numel(), stream), "composite")
+    order = torch.empty(lib.gs_tile_order_items(view, 1), dtype=torch.int32, device=device)
+    nat.check(lib.gs_tile_order(ptr(ranges), ptr(ncon), view, ptr(order), ptr(keys), keys.numel(),
+                                1, stream), "tile_order")
+    assert torch.equal(out[0], image)
+    tiles = order[order >= 0]
+    assert len(tiles) == 4 * ranges.shape[0] and not (tiles & 0x7F).any()
 
 
 def test_image_tile_rule():
