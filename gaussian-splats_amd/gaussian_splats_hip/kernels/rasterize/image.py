@@ -75,6 +75,19 @@ def image_tile(asked: int, width: int, height: int, n: int, views: int = 1) -> i
     return None
 
 
+def far_away(longest: int, entries: int, lists: int, n: int) -> bool:
+    """Whether ``lists`` shared lists of a single view of ``n`` Gaussians are to be
+    made again, one per tile: Gaussians smaller than a list tile (``entries`` below
+    two each) on few tiles, the ``longest`` list with more than an eighth of them,
+    as a scene seen from far away.  Each tile walks up to four times its own
+    entries there, and nothing was saved in placing them.  1M of them far away at
+    1080p, a frame 1392 us with shared lists, 786 with lists made again (620 before
+    lists were shared), a step 2910 and 1376 (1735); 200k a step 1693 and 1099
+    (1450)."""
+    return (lists * 4 < SPLIT_TILES and longest > LONG_LIST and 8 * longest > n
+            and entries < 2 * n)
+
+
 class ImageRequest:
     """Everything but the Gaussians of an image call on ``n`` of them: the
     ``cameras`` (``camera_floats`` of ``views`` of them), the views and the
@@ -98,15 +111,17 @@ class ImageRequest:
     and 16 views of 2500 tiles, which walk a quarter of their lists, gained
     nothing."""
 
-    __slots__ = ("floats", "view", "list_view", "views", "shape", "tiles", "near", "far",
-                 "gaussian", "small")
+    __slots__ = ("arguments", "floats", "view", "list_view", "views", "shape", "tiles", "near",
+                 "far", "gaussian", "small")
 
     def __init__(self, n, cameras, views, width, height, tile, threshold, near, far,
-                 rendering_mode, confidence, stacked):
+                 rendering_mode, confidence, stacked, share=True):
+        self.arguments = (n, cameras, views, width, height, tile, threshold, near, far,
+                          rendering_mode, confidence, stacked)
         self.views, self.floats = views, cameras
         self.shape = (views, height, width, 3) if stacked else (height, width, 3)
         tw, th = nat.tiles(width, height, tile)
-        shift = int(tile == 16 and self.views == 1 and tw * th >= SPLIT_TILES)
+        shift = int(share and tile == 16 and self.views == 1 and tw * th >= SPLIT_TILES)
         tw, th = nat.tiles(width, height, tile << shift)
         cols = mosaic_columns(self.views, tw, th)
         self.tiles = (cols * tw, -(-self.views // cols) * th)
@@ -122,6 +137,10 @@ class ImageRequest:
 
         self.view = view(tile, shift)
         self.list_view = view(tile << shift, 0) if shift else self.view
+
+    def unshared(self) -> ImageRequest:
+        """The same request with a list per tile."""
+        return ImageRequest(*self.arguments, share=False)
 
     def cameras(self):
         """The three arrays of ``floats``: rotations, translations, intrinsics."""
@@ -156,9 +175,10 @@ def small_lists(depth_keys, tile_rects, tiles_w, tiles_h, nbytes, clear=None):
     return ids, ranges
 
 
-def forward_image(params, request: ImageRequest, keep: bool, timer=None):
+def forward_image(params, request: ImageRequest, keep: bool, timer=None, again=False):
     """Projects, bins and composites; returns ``(image, saved, walk)``, the last
-    two None unless ``keep`` (a backward will follow)."""
+    two None unless ``keep`` (a backward will follow).  ``again``: the call's
+    timer has been started."""
     mark = timer or (lambda name: None)
     device = nat.require_gpu(*params)
     mean, rotation, scale, opacity, color = (nat.prepare(t) for t in params)
@@ -176,7 +196,8 @@ def forward_image(params, request: ImageRequest, keep: bool, timer=None):
     records = torch.empty((vn, 12), dtype=torch.float32, device=device)
     depth_keys = torch.empty(vn, dtype=torch.int32, device=device)
     tile_rects = torch.empty(vn, dtype=torch.int32, device=device)
-    mark("start")
+    if not again:
+        mark("start")
     nat.check(
         nat.launch("project", lambda: lib.gs_project_image(
             ptr(mean), ptr(rotation), ptr(scale), ptr(opacity), ptr(color), n, color.shape[1],
@@ -206,7 +227,11 @@ def forward_image(params, request: ImageRequest, keep: bool, timer=None):
         longest = nat.longest_list(ranges)
     mark("sort")
     subs = 1 << (2 * view.list_shift)  # compositing tiles per list
-    view.active_tiles = nat.active_tiles(ranges) * subs
+    lists = nat.active_tiles(ranges)
+    if view.list_shift and far_away(longest, ids.numel(), lists, n):
+        del records, depth_keys, tile_rects, accumulator, ids, ranges
+        return forward_image(params, request.unshared(), keep, timer, again=True)
+    view.active_tiles = lists * subs
     # With a long list the longest walk may set the time of a launch: its tiles
     # are split over four waves however many have work.  Whether it does is not
     # known before the walk.  1M Gaussians at 1080p with a dense spot, a step with

@@ -167,18 +167,22 @@ def test_image_walk_segments(size, n, device):
     _same_gradients(second, [p.grad for p in leaves])
 
 
-def _points(n, size, spread):
+def _points(n, size, spread, background=0):
     """Faint Gaussians of half a pixel in ``spread`` pixels around the middle: each
     pixel takes few entries of its tile's long list.  Ten wide opaque ones lie
     across them halfway into the list, a little below the middle, so the tiles'
-    quarters walk to different depths."""
+    quarters walk to different depths.  ``background``: of the Gaussians, those
+    that lie all over the image instead, faint too."""
     scene = scenes.edge_case_scene(n=n, sh_degree=1, image_size=size, seed=8)
+    m = n - background
+    mean, scale = scene.mean[m:].clone(), scene.scale[m:].clone()
     g = torch.Generator().manual_seed(n)
     pixel = 5 / (0.75 * size[0])
     scene.mean[:, :2] = torch.randn(n, 2, generator=g) * spread * pixel
     scene.mean[:, 2] = -(torch.rand(n, generator=g) * 0.1 + 5)
     scene.scale[:] = math.log(0.5 * pixel) + torch.tensor([-0.5, 0.5, 0.0])
     scene.opacity[:] = torch.randn(n, 1, generator=g) * 0.3 - 4.5
+    scene.mean[m:], scene.scale[m:] = mean, scale
     scene.mean[-10:] = torch.tensor([0.0, -2 * pixel, -5.05])
     scene.rotation[-10:] = torch.tensor([1.0, 0.0, 0.0, 0.0])
     scene.scale[-10:] = torch.log(torch.tensor([60.0, 6.0, 1.0]) * pixel)
@@ -186,14 +190,14 @@ def _points(n, size, spread):
     return scene
 
 
-@pytest.mark.parametrize("size,n,spread", [((24, 24), 24_000, 2.0), ((40, 24), 90_000, 3.0),
-                                           ((1111, 1043), 60_000, 8.0),
-                                           ((4096, 1712), 20_000, 8.0),
-                                           ((4096, 2816), 20_000, 8.0)])
-def test_image_long_walks(size, n, spread, device):
+@pytest.mark.parametrize("size,n,spread,background,shared", [
+    ((24, 24), 24_000, 2.0, 0, False), ((40, 24), 90_000, 3.0, 0, False),
+    ((1111, 1043), 70_000, 8.0, 4000, True), ((4096, 1712), 20_000, 8.0, 0, False),
+    ((4096, 2816), 20_000, 8.0, 0, True)])
+def test_image_long_walks(size, n, spread, background, shared, device):
     """Walks that drop records and double their spacing, in images of 11, 7 and 3
-    records per tile, with and without shared lists."""
-    scene = _points(n, size, spread).to(device)
+    records per tile, with a list per tile and with lists shared by 2 x 2."""
+    scene = _points(n, size, spread, background).to(device)
     cam = scene.cameras[0]
     splats = GaussianSplat.from_tensors(*scene.params())
     leaves = [p.detach().clone().requires_grad_(True) for p in scene.params()]
@@ -203,9 +207,13 @@ def test_image_long_walks(size, n, spread, device):
     records = {True: 11, False: 7 if tiles < 42_130 else 3}[tiles < 26_810]
     padded = walk_records.numel() // (records * 4096 + 32)
     assert walk_records.numel() == padded * (records * 4096 + 32) and padded >= tiles
+    assert (image.grad_fn.saved_tensors[8].shape[0] < tiles) == shared
     keys = walk_records[padded * records * 4096:].view(torch.int32).reshape(padded, 4, 2)
     expected = _op(scene, leaves, cam, 16, "gaussian")
-    assert torch.equal(image, expected)
+    if background:  # the op's checkpoints cut a pixel's colour into partial sums (see below)
+        assert (image - expected).abs().max() < 64 * 4 * 2.0 ** -24
+    else:
+        assert torch.equal(image, expected)
     # Without a symmetry that the wide Gaussians' rotation gradients, odd moments
     # over their pixels, would cancel by.
     weight = torch.randn(image.shape, device=device, generator=torch.Generator(device).manual_seed(n))
@@ -295,6 +303,37 @@ def test_backward_frees_the_walk(device):
     assert held[1] <= image.numel() * 4 + (1 << 20)
 
 
+def test_image_far_away(device):
+    """Small Gaussians on few tiles of a large image: a list per tile after all,
+    in a frame and in a step, and the stages' times of both attempts under the
+    usual names."""
+    from gaussian_splats_hip.kernels.rasterize.image import far_away
+    from gaussian_splats_hip.timing import record_timings
+
+    assert far_away(211_177, 1_185_219, 56, 1_000_000)
+    assert not far_away(94_490, 1_337_256, 162, 1_000_000)  # not an eighth in one list
+    assert not far_away(577_233, 41_233_268, 968, 2_000_000)  # larger than a list tile
+    assert not far_away(211_177, 1_185_219, 1024, 1_000_000)  # many tiles
+    assert not far_away(8192, 24_000, 4, 20_000)  # short lists
+    scene = _points(30_000, (1111, 1043), 20.0).to(device)
+    cam = scene.cameras[0]
+    splats = GaussianSplat.from_tensors(*scene.params())
+    leaves = [p.detach().clone().requires_grad_(True) for p in scene.params()]
+    with record_timings(device) as times:
+        image = rasterize(splats, cam, near=scene.near, far=scene.far)
+    assert set(times["default"]) == {"Project", "Bin", "Emit", "Sort", "Composite"}
+    ranges = image.grad_fn.saved_tensors[8]
+    assert ranges.shape[0] == 70 * 66
+    expected = _op(scene, leaves, cam, 16, "gaussian")
+    assert torch.equal(image, expected)
+    with torch.no_grad():
+        assert torch.equal(image, rasterize(splats, cam, near=scene.near, far=scene.far))
+    weight = torch.randn(image.shape, device=device, generator=torch.Generator(device).manual_seed(1))
+    (image * weight).sum().backward()
+    (expected * weight).sum().backward()
+    _same_gradients([getattr(splats, n).grad for n in PARAMS], [p.grad for p in leaves])
+
+
 @pytest.mark.parametrize("n", [40_000, 14_000])
 def test_image_one_long_list(n, device):
     """One list above 8192 entries among many short ones (faint Gaussians in
@@ -326,7 +365,7 @@ def test_plan_without_checkpoints(device):
     from gaussian_splats_hip.kernels.rasterize import _native as nat
 
     w, h = 1111, 1043
-    scene = _points(60_000, (w, h), 8.0).to(device)
+    scene = _points(60_000, (w, h), 8.0, 4000).to(device)
     splats = GaussianSplat.from_tensors(*scene.params())
     image = rasterize(splats, scene.cameras[0], near=scene.near, far=scene.far)
     records, _, ids, ranges = image.grad_fn.saved_tensors[5:9]
