@@ -189,14 +189,13 @@ struct CheckpointLayout {
 // buffer must come from the forward over the same lists.
 constexpr uint32_t kCheckpointMagic = 0x70636773u;  // "sgcp"
 constexpr int kCheckpointStampWords = 4;  // magic, tile size, tiles, table length
-inline CheckpointLayout checkpoint_layout(void* base, int tile_size, int64_t total, int subs,
+inline CheckpointLayout checkpoint_layout(void* base, int tile_size, int64_t total,
                                           size_t available = ~size_t(0)) {
   CheckpointLayout c;
   const size_t record = size_t(checkpoint_pixels(tile_size)) * 16;
   // A crossing's position lies below the list end + 64 (its batch starts
   // inside the list): table slots up to (total + 63) / kCheckpointEntries.
-  // With one list for several tiles each tile has slots of its own.
-  c.table_len = (total / kCheckpointEntries + 2) * subs;
+  c.table_len = total / kCheckpointEntries + 2;
   char* p = static_cast<char*>(base);
   size_t off = 0;
   auto take = [&](size_t n) {

@@ -190,8 +190,7 @@ __device__ __forceinline__ void composite_bwd_tile(const CompositeBwdArgs& a, fl
         a.ckpt_stamp[2] == uint32_t(a.num_tiles) && a.ckpt_stamp[3] == a.ckpt_table_len;
     const int m = table ? checkpoint_count(start, max_n, a.ranges[2 * list + 1] - start) : 0;
     const int64_t first = checkpoint_first(start);
-    const int slot = lane < m ? a.ckpt_table[(first / kCheckpointEntries + lane) * subs + sub]
-                              : -1;
+    const int slot = lane < m ? a.ckpt_table[first / kCheckpointEntries + lane] : -1;
     // A slot outside the pool (never written by this forward) counts as missing.
     const uint64_t missing = __ballot(lane < m && (slot < 0 || int64_t(slot) >= a.ckpt_capacity));
     const int w = missing ? __builtin_ctzll(missing) : m;
@@ -592,12 +591,14 @@ int composite_bwd(const float* projected_mean, const float* inverse_covariance,
   }
   a.ckpt_stamp = nullptr;
   a.ckpt_table_len = 0;
+  GS_REQUIRE(!checkpoints || view.list_shift == 0, GS_ERR_UNSUPPORTED,
+             "checkpoints are recorded for one list per tile only");
   // The forward records checkpoints under these conditions only
   // (composite_fwd.hip); its stamp is checked on the device as well.
   if (checkpoints && !plan.split_all && view.tile_size <= 16 && n > 0) {
     GS_REQUIRE(num_intersections >= 0, GS_ERR_INVALID_ARGUMENT, "negative intersection count");
     const CheckpointLayout c = checkpoint_layout(const_cast<void*>(checkpoints), view.tile_size,
-                                                 num_intersections, m.subs(), checkpoint_bytes);
+                                                 num_intersections, checkpoint_bytes);
     GS_REQUIRE(checkpoint_bytes >= c.header_bytes, GS_ERR_WORKSPACE,
                "checkpoint buffer too small (%zu bytes, need at least %zu)", checkpoint_bytes,
                c.header_bytes);

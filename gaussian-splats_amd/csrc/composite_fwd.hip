@@ -151,7 +151,7 @@ __device__ __forceinline__ void composite_tile(const CompositeArgs& a, float4 (*
     slot = uint32_t(__builtin_amdgcn_readfirstlane(int(slot)));
     const bool ok = ck_written == ck_count && int64_t(slot) < a.ckpt_capacity;
     const int64_t pos = checkpoint_first(start) + int64_t(ck_count) * kCheckpointEntries;
-    if (lane == 0) a.ckpt_table[pos / kCheckpointEntries * subs + sub] = ok ? int32_t(slot) : -1;
+    if (lane == 0) a.ckpt_table[pos / kCheckpointEntries] = ok ? int32_t(slot) : -1;
     if (ok) {
       float4* rec = a.ckpt_records + int64_t(slot) * kRecord;
 #pragma unroll
@@ -569,9 +569,9 @@ extern "C" GS_API size_t gs_composite_checkpoint_bytes(gs_view view, int64_t num
   if (check_view(view, true) != GS_OK || num_intersections < 0) return 0;
   if (longest_list <= kCheckpointMinList) return 0;  // no walk would record one
   if (view.tile_size > 16) return 0;  // 16 pixels per lane leave no registers for them
-  const Mosaic m = mosaic_of(view);
-  if (dispatch_plan(m.num_tiles(), view, false).split_all) return 0;
-  return checkpoint_layout(nullptr, view.tile_size, num_intersections, m.subs()).bytes;
+  if (view.list_shift) return 0;
+  if (dispatch_plan(mosaic_of(view).num_tiles(), view, false).split_all) return 0;
+  return checkpoint_layout(nullptr, view.tile_size, num_intersections).bytes;
 }
 
 extern "C" GS_API size_t gs_composite_hit_mask_bytes(gs_view view, int64_t num_intersections) {
@@ -652,9 +652,10 @@ int composite(const void* records, int64_t num_records, const int32_t* gaussian_
   }
   hipStream_t s = as_stream(stream);
   if (checkpoints) {
+    GS_REQUIRE(view.list_shift == 0, GS_ERR_UNSUPPORTED,
+               "checkpoints are recorded for one list per tile only");
     const CheckpointLayout c =
-        checkpoint_layout(checkpoints, view.tile_size, num_intersections, m.subs(),
-                          checkpoint_bytes);
+        checkpoint_layout(checkpoints, view.tile_size, num_intersections, checkpoint_bytes);
     GS_REQUIRE(checkpoint_bytes >= c.header_bytes, GS_ERR_WORKSPACE,
                "checkpoint buffer too small (%zu bytes, need at least %zu)", checkpoint_bytes,
                c.header_bytes);

@@ -41,18 +41,16 @@ __global__ __launch_bounds__(256) void tile_key_kernel(const int64_t* __restrict
                                                        const int32_t* __restrict__ ncon,
                                                        int tiles_w, int num_tiles, int tile,
                                                        int width, int height, int view_tw,
-                                                       int view_th, int cols, int views, int shift,
+                                                       int view_th, int cols, int views,
                                                        uint32_t* __restrict__ key,
                                                        uint32_t* __restrict__ crossings) {
   const int lane = threadIdx.x & 63;
   const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (t >= num_tiles) return;
-  const int tx = t % tiles_w, ty = t / tiles_w;
-  int sub;
-  const int list = list_of_tile(tx, ty, tiles_w, shift, sub);
   int64_t work;
   if (ncon) {
     // Mosaic tile -> view and pixel origin inside it (see gs_view).
+    const int tx = t % tiles_w, ty = t / tiles_w;
     const int vx = tx / view_tw, vy = ty / view_th;
     const int view = vy * cols + vx;
     const int ox = (tx - vx * view_tw) * tile, oy = (ty - vy * view_th) * tile;
@@ -66,14 +64,13 @@ __global__ __launch_bounds__(256) void tile_key_kernel(const int64_t* __restrict
     for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o, 64));
     work = m;
   } else {
-    work = ranges[2 * list + 1] - ranges[2 * list];
+    work = ranges[2 * t + 1] - ranges[2 * t];
   }
   if (lane == 0) {
     key[t] = uint32_t(min(max(work, int64_t(0)), int64_t(0xFFFF)));
-    crossings[t] =
-        ncon && ranges ? uint32_t(checkpoint_count(ranges[2 * list], int(work),
-                                                   ranges[2 * list + 1] - ranges[2 * list]))
-                       : 0u;
+    crossings[t] = ncon && ranges ? uint32_t(checkpoint_count(ranges[2 * t], int(work),
+                                                              ranges[2 * t + 1] - ranges[2 * t]))
+                                  : 0u;
   }
 }
 
@@ -325,9 +322,11 @@ int tile_order_launch(const int64_t* ranges, const int32_t* n_contributors, cons
   const bool forward_keys =
       keys_ready && n_contributors && !dispatch_plan(num_tiles, view, false).split_all;
   if (!forward_keys) {
+    GS_REQUIRE(m.shift == 0, GS_ERR_UNSUPPORTED,
+               "with a list for 2 x 2 tiles the plan needs the forward's keys");
     tile_key_kernel<<<unsigned(ceil_div(num_tiles, 4)), 256, 0, s>>>(
         ranges, n_contributors, m.tiles_w(), num_tiles, view.tile_size, view.image_width,
-        view.image_height, m.tw, m.th, m.cols, m.views, m.shift, key, crossings);
+        view.image_height, m.tw, m.th, m.cols, m.views, key, crossings);
     GS_TRY(check_launch("tile_order keys"));
   }
   tile_plan_kernel<<<8, kOrderThreads, 0, s>>>(key, crossings, num_tiles,

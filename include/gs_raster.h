@@ -85,7 +85,9 @@ typedef struct gs_view {
   int32_t active_tiles;
   /* 1: the lists are those of 2 x 2 tiles (compositing calls with tiles of 16
    * pixels): `ranges` covers the grid of doubled tiles, and each view's tile
-   * grid is rounded up to whole ones.  0: one list per tile. */
+   * grid is rounded up to whole ones.  Checkpoints, and plans other than from
+   * the forward's keys, are refused with it (GS_ERR_UNSUPPORTED).  0: one list
+   * per tile. */
   int32_t list_shift;
   /* 1: the compositing calls split every tile of 16 or 32 pixels over four
    * waves whatever active_tiles says (a caller whose lists are long throughout,

@@ -253,6 +253,31 @@ def test_walk_records_are_bounded():
     assert lib.gs_composite_walk_bytes(_view(tile_size=32, active_tiles=100)) == 0
 
 
+def test_shared_lists_host_checks():
+    """Lists shared by 2 x 2 tiles go with walk records or the forward's keys:
+    checkpoints and plans from the lists are refused before any launch."""
+    lib = nat.library()
+    fake = ctypes.c_void_p(256)
+    view = _view(image_width=1920, image_height=1080, list_shift=1)
+    assert lib.gs_composite_checkpoint_bytes(view, 1 << 20, 9000) == 0
+    assert lib.gs_composite_checkpoint_bytes(_view(image_width=1920, image_height=1080), 1 << 20,
+                                             9000) > 0
+    status = lib.gs_composite(fake, 10, fake, 10, fake, None, view, fake, fake, fake, fake, 1 << 20,
+                              None, 0, None, 0, None)
+    assert status == nat.GS_ERR_UNSUPPORTED and b"one list per tile" in lib.gs_last_error()
+    status = lib.gs_composite_bwd(*([fake] * 4), 10, *([fake] * 5), None, view, fake, None, fake,
+                                  1 << 20, 10, None, 0, None)
+    assert status == nat.GS_ERR_UNSUPPORTED and b"one list per tile" in lib.gs_last_error()
+    for ncon, ready in ((None, 0), (fake, 0)):
+        status = lib.gs_tile_order(fake, ncon, view, fake, fake, 1 << 20, ready, None)
+        assert status == nat.GS_ERR_UNSUPPORTED and b"forward's keys" in lib.gs_last_error()
+    assert lib.gs_tile_order_noalloc(fake, fake, view, fake, None) != nat.GS_OK
+    for bad in (dict(list_shift=2), dict(list_shift=1, tile_size=32), dict(split_tiles=2)):
+        status = lib.gs_composite(fake, 10, fake, 10, fake, None, _view(**bad), fake, fake, fake,
+                                  None, 0, None, 0, None, 0, None)
+        assert status == nat.GS_ERR_INVALID_ARGUMENT
+
+
 def test_misaligned_buffers_rejected():
     lib = nat.library()
     fake = ctypes.c_void_p(16)
