@@ -50,12 +50,18 @@ def _same_gradients(a, b):
 @pytest.mark.parametrize("mode", ["gaussian", "ellipsoid"])
 @pytest.mark.parametrize("tile", [4, 8, 16, 32])
 @pytest.mark.parametrize("kind,size", [("edge", (96, 80)), ("edge", (17, 1)), ("needle", (333, 207)),
-                                       ("cloud", (1111, 1043)), ("cloud", (1100, 1030))])
+                                       ("cloud", (1111, 1043)), ("cloud", (1100, 1030)),
+                                       ("small", (1111, 1043)), ("wide", (4097, 17))])
 def test_image_equals_op(kind, size, tile, mode, device):
     if kind == "needle":
         scene = _needles(3000, size)
     elif kind == "cloud":  # above 4096 tiles of 16 pixels: whole tiles per wave
         scene = scenes.edge_case_scene(n=20000, sh_degree=0, image_size=size, seed=6)
+    elif kind == "small":  # lists of a small scene, shared by 2 x 2 tiles
+        scene = scenes.edge_case_scene(n=2000, image_size=size, seed=7)
+    elif kind == "wide":  # above 4096 pixels: tiles of 32
+        scene = scenes.edge_case_scene(n=3000, image_size=size, seed=7)
+        scene.mean[:, 1] *= 0.01
     else:
         scene = scenes.edge_case_scene(n=1000, image_size=size)
     scene = scene.to(device)
@@ -63,6 +69,9 @@ def test_image_equals_op(kind, size, tile, mode, device):
     splats = GaussianSplat.from_tensors(*scene.params())
     leaves = [p.detach().clone().requires_grad_(True) for p in scene.params()]
     image = rasterize(splats, cam, tile, near=scene.near, far=scene.far, rendering_mode=mode)
+    if kind in ("small", "wide") and mode == "gaussian":
+        lists = image.grad_fn.saved_tensors[8].shape[0]
+        assert lists == {"small": 35 * 33, "wide": 129}[kind]
     expected = _op(scene, leaves, cam, tile, mode)
     if mode == "ellipsoid":
         # A pixel within rounding of the ellipse's edge may lie outside the
@@ -254,6 +263,25 @@ def test_image_is_no_view(device):
     assert image.shape == (32, 48, 3) and not image._is_view()
     image.detach_()
     assert rasterize_views(splats, [cam]).shape == (1, 32, 48, 3)
+
+
+def test_views_of_32_pixel_tiles(device):
+    """A mosaic above 256 tiles of 16 pixels per axis: tiles of 32, each walked
+    whole by one wave (the wide image's, above, in quarters)."""
+    scene = scenes.config5(seed=2, n=2000, views=36, size=704, focal=880).to(device)
+    splats = GaussianSplat.from_tensors(*scene.params())
+    leaves = [p.detach().clone().requires_grad_(True) for p in scene.params()]
+    images = rasterize_views(splats, scene.cameras)
+    ranges, order = (images.grad_fn.saved_tensors[i] for i in (8, -2))
+    assert ranges.shape[0] == (6 * 22) ** 2 and not (order[order >= 0] & 0x7F).any()
+    r, t, k, w, h = camera_tensors(scene.cameras)
+    expected = rasterize_views_outputs(*leaves, r, t, k, w, h, 32, 0.999, 0.2, 100.0, "gaussian",
+                                       0.95)[0]
+    assert torch.equal(images, expected)
+    weight = torch.linspace(-1, 1, images[0].numel(), device=device).reshape(images[0].shape)
+    (images * weight).mean().backward()
+    (expected * weight).mean().backward()
+    _same_gradients([getattr(splats, n).grad for n in PARAMS], [p.grad for p in leaves])
 
 
 def test_no_gaussians_and_nothing_visible(device):
