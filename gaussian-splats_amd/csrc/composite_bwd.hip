@@ -315,9 +315,10 @@ __device__ __forceinline__ void composite_bwd_tile(const CompositeBwdArgs& a, fl
       float ax = -0.0f, ay = -0.0f;  // ABS: sums of |mean gradient terms| / |kNegHalfLog2e|
       const float padx = s.pa * c.dx, hbdx = half_pb * c.dx;
       uint64_t touched = 0;
-      // Branch-free: an entry a pixel did not process while active, or whose
-      // alpha is cut to 0, runs with alpha = 0, which leaves T, g.S and every
-      // sum unchanged.  29 VALU instructions per band.
+      // Only the lanes whose pixel took the entry (processed it while active, alpha
+      // not cut) run the rest: with alpha = 0 in the others instead, a gradient or
+      // colour that is not finite would reach entries its pixel did not take (times
+      // the weight 0).  The same time either way.  29 VALU instructions per band.
 #pragma unroll
       for (int k = 0; k < PIX; ++k) {
         // A band of 64 pixels that the Gaussian cannot reach, or none of which
@@ -326,34 +327,33 @@ __device__ __forceinline__ void composite_bwd_tile(const CompositeBwdArgs& a, fl
         if (!((band_mask >> k) & 1u) || active == 0) continue;
         const float dy = pyf[k] - s.v;
         float raw;
-        const float a0 = entry_alpha<false>(s, c, dy, raw);
-        const uint64_t hit = ballot_of(a0 >= kMinAlpha) & active;
-        const float alpha = in_mask(hit) ? a0 : 0.0f;
+        const float alpha = entry_alpha<false>(s, c, dy, raw);
+        const uint64_t hit = ballot_of(alpha >= kMinAlpha) & active;
         touched |= hit;
-        // T before the entry = T after it / (1 - alpha) = T + w with
-        // w = T alpha / (1 - alpha): v_rcp_f32's error (up to an ulp, of one
-        // sign) then enters scaled by alpha, so walking back through thousands
-        // of small-alpha entries does not accumulate it (with the plain
-        // reciprocal: ~2e-4 relative after 1600 entries).  alpha = 0 gives
-        // exactly T.
-        const float w = T[k] * (alpha * __builtin_amdgcn_rcpf(1.0f - alpha));
-        T[k] += w;
-        sr += gr[k] * w;
-        sg += gg[k] * w;
-        sb += gb[k] * w;
-        const float gc = gr[k] * s.r + gg[k] * s.g + gb[k] * s.bl;
-        const float diff = gc - gs_[k];
-        gs_[k] += alpha * diff;
-        // o times dL/dalpha * G = w diff where alpha is not clamped (a cut
-        // alpha has w = 0).
-        const float q = raw <= kMaxAlpha ? w * diff : 0.0f;
-        const float qy = q * dy;
-        s0 += q;
-        s1 += qy;
-        s2 += qy * dy;
-        if constexpr (ABS) {
-          ax += fabsf(q * fmaf(half_pb, dy, padx));
-          ay += fabsf(q * fmaf(s.pc, dy, hbdx));
+        if (in_mask(hit)) {
+          // T before the entry = T after it / (1 - alpha) = T + w with
+          // w = T alpha / (1 - alpha): v_rcp_f32's error (up to an ulp, of one
+          // sign) then enters scaled by alpha, so walking back through thousands
+          // of small-alpha entries does not accumulate it (with the plain
+          // reciprocal: ~2e-4 relative after 1600 entries).
+          const float w = T[k] * (alpha * __builtin_amdgcn_rcpf(1.0f - alpha));
+          T[k] += w;
+          sr += gr[k] * w;
+          sg += gg[k] * w;
+          sb += gb[k] * w;
+          const float gc = gr[k] * s.r + gg[k] * s.g + gb[k] * s.bl;
+          const float diff = gc - gs_[k];
+          gs_[k] += alpha * diff;
+          // o times dL/dalpha * G = w diff where alpha is not clamped.
+          const float q = raw <= kMaxAlpha ? w * diff : 0.0f;
+          const float qy = q * dy;
+          s0 += q;
+          s1 += qy;
+          s2 += qy * dy;
+          if constexpr (ABS) {
+            ax += fabsf(q * fmaf(half_pb, dy, padx));
+            ay += fabsf(q * fmaf(s.pc, dy, hbdx));
+          }
         }
       }
       if (touched == 0) continue;

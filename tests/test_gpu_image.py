@@ -248,6 +248,41 @@ def test_views_image_equals_op(device):
     _same_gradients([getattr(splats, n).grad for n in PARAMS], [p.grad for p in leaves])
 
 
+@pytest.mark.parametrize("size,n", [((96, 80), 1000), ((1111, 1043), 30_000), ((4097, 17), 3000)])
+@pytest.mark.parametrize("path", ["image", "op4", "op16"])
+def test_gradient_that_is_not_finite(path, size, n, device):
+    """An infinite gradient at one pixel reaches the Gaussians that the pixel took
+    and no others, whose gradients are those without it."""
+    scene = scenes.edge_case_scene(n=n, image_size=size, seed=7)
+    scene.mean[:, 1] *= size[1] / size[0]
+    scene.color[:, 0] += 3  # no channel clamped at 0, which has no gradient
+    scene = scene.to(device)
+    cam = scene.cameras[0]
+    if path == "image":
+        splats = GaussianSplat.from_tensors(*scene.params())
+        params = [getattr(splats, p) for p in PARAMS]
+        image = rasterize(splats, cam, near=scene.near, far=scene.far)
+    else:
+        params = [p.detach().clone().requires_grad_(True) for p in scene.params()]
+        image = _op(scene, params, cam, int(path[2:]), "gaussian")
+
+    def gradients(weight):
+        return torch.autograd.grad(image, params, weight, retain_graph=True)
+
+    weight = torch.randn(image.shape, device=device, generator=torch.Generator(device).manual_seed(2))
+    y, x = size[1] // 2, size[0] // 2
+    weight[y, x] = 0
+    want = gradients(weight)
+    alone = torch.zeros_like(weight)
+    alone[y, x] = 1
+    took = gradients(alone)[4].flatten(1).any(1)
+    assert 0 < took.sum() < n
+    weight[y, x] = torch.tensor([float("inf"), 1.0, -1.0])
+    got = gradients(weight)
+    assert not got[4][took].isfinite().all()
+    _same_gradients([g[~took] for g in got], [w[~took] for w in want])
+
+
 def test_image_is_no_view(device):
     """One camera's image is a tensor of its own, as the op's output is: it can
     be detached in place, and its gradient reaches the backward as it is."""
