@@ -145,6 +145,11 @@ STAGE_KERNELS = {
 }
 
 
+# What the figures by stage and the list entries of a line describe.
+STAGES_OF = ("the op's stages (reference tile lists, asked tile size), run apart from the timed "
+             "steps, whose rasterize calls return images alone and go through fewer, tighter lists")
+
+
 def stage_entries(stages_ms, bytes_model):
     """Per stage: its kernels, time, algorithmic bytes and HBM fraction; and
     the whole binning (bin + emit) against its own bytes."""
@@ -659,6 +664,7 @@ def bench_views(args, scene):
             "intersections": int(gids.numel()),
         },
         **compared,
+        "stages_of": STAGES_OF,
         "stages": stages,
         "roofline": {
             "kernel": "composite_bwd_kernel",
@@ -1054,6 +1060,7 @@ def main():
             "tile_size": args.tile_size,
             "intersections": info["total"],
         },
+        "stages_of": STAGES_OF,
         "stages": stages,
         "kernels": kernels,
         "roofline": roofline,
