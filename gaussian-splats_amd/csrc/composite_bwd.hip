@@ -144,6 +144,18 @@ __device__ __forceinline__ void composite_bwd_tile(const CompositeBwdArgs& a, fl
     gs_[k] = 0.0f;
     max_n = max(max_n, ncon[k]);
   }
+  // Gradients that are not finite count as 0 in the walk, where their product
+  // with the weight 0 of an entry that the pixel did not take would be NaN; the
+  // entries that it took get them after the walk.
+  bool odd_pixel = false;
+#pragma unroll
+  for (int k = 0; k < PIX; ++k) {
+    odd_pixel |= !(is_finite(gr[k]) && is_finite(gg[k]) && is_finite(gb[k]));
+    gr[k] = is_finite(gr[k]) ? gr[k] : 0.0f;
+    gg[k] = is_finite(gg[k]) ? gg[k] : 0.0f;
+    gb[k] = is_finite(gb[k]) ? gb[k] : 0.0f;
+  }
+  const bool any_odd_pixel = ballot_of(odd_pixel) != 0;
   // MASKS: each band's largest contributor count.  The forward's wave of a
   // band wrote the masks of every batch below it and may have stopped after
   // it, so later words of the band are never read.  The wave-wide maxima are
@@ -315,10 +327,9 @@ __device__ __forceinline__ void composite_bwd_tile(const CompositeBwdArgs& a, fl
       float ax = -0.0f, ay = -0.0f;  // ABS: sums of |mean gradient terms| / |kNegHalfLog2e|
       const float padx = s.pa * c.dx, hbdx = half_pb * c.dx;
       uint64_t touched = 0;
-      // Only the lanes whose pixel took the entry (processed it while active, alpha
-      // not cut) run the rest: with alpha = 0 in the others instead, a gradient or
-      // colour that is not finite would reach entries its pixel did not take (times
-      // the weight 0).  The same time either way.  29 VALU instructions per band.
+      // Branch-free: an entry a pixel did not process while active, or whose
+      // alpha is cut to 0, runs with alpha = 0, which leaves T, g.S and every
+      // sum unchanged.  29 VALU instructions per band.
 #pragma unroll
       for (int k = 0; k < PIX; ++k) {
         // A band of 64 pixels that the Gaussian cannot reach, or none of which
@@ -327,33 +338,34 @@ __device__ __forceinline__ void composite_bwd_tile(const CompositeBwdArgs& a, fl
         if (!((band_mask >> k) & 1u) || active == 0) continue;
         const float dy = pyf[k] - s.v;
         float raw;
-        const float alpha = entry_alpha<false>(s, c, dy, raw);
-        const uint64_t hit = ballot_of(alpha >= kMinAlpha) & active;
+        const float a0 = entry_alpha<false>(s, c, dy, raw);
+        const uint64_t hit = ballot_of(a0 >= kMinAlpha) & active;
+        const float alpha = in_mask(hit) ? a0 : 0.0f;
         touched |= hit;
-        if (in_mask(hit)) {
-          // T before the entry = T after it / (1 - alpha) = T + w with
-          // w = T alpha / (1 - alpha): v_rcp_f32's error (up to an ulp, of one
-          // sign) then enters scaled by alpha, so walking back through thousands
-          // of small-alpha entries does not accumulate it (with the plain
-          // reciprocal: ~2e-4 relative after 1600 entries).
-          const float w = T[k] * (alpha * __builtin_amdgcn_rcpf(1.0f - alpha));
-          T[k] += w;
-          sr += gr[k] * w;
-          sg += gg[k] * w;
-          sb += gb[k] * w;
-          const float gc = gr[k] * s.r + gg[k] * s.g + gb[k] * s.bl;
-          const float diff = gc - gs_[k];
-          gs_[k] += alpha * diff;
-          // o times dL/dalpha * G = w diff where alpha is not clamped.
-          const float q = raw <= kMaxAlpha ? w * diff : 0.0f;
-          const float qy = q * dy;
-          s0 += q;
-          s1 += qy;
-          s2 += qy * dy;
-          if constexpr (ABS) {
-            ax += fabsf(q * fmaf(half_pb, dy, padx));
-            ay += fabsf(q * fmaf(s.pc, dy, hbdx));
-          }
+        // T before the entry = T after it / (1 - alpha) = T + w with
+        // w = T alpha / (1 - alpha): v_rcp_f32's error (up to an ulp, of one
+        // sign) then enters scaled by alpha, so walking back through thousands
+        // of small-alpha entries does not accumulate it (with the plain
+        // reciprocal: ~2e-4 relative after 1600 entries).  alpha = 0 gives
+        // exactly T.
+        const float w = T[k] * (alpha * __builtin_amdgcn_rcpf(1.0f - alpha));
+        T[k] += w;
+        sr += gr[k] * w;
+        sg += gg[k] * w;
+        sb += gb[k] * w;
+        const float gc = gr[k] * s.r + gg[k] * s.g + gb[k] * s.bl;
+        const float diff = gc - gs_[k];
+        gs_[k] += alpha * diff;
+        // o times dL/dalpha * G = w diff where alpha is not clamped (a cut
+        // alpha has w = 0).
+        const float q = raw <= kMaxAlpha ? w * diff : 0.0f;
+        const float qy = q * dy;
+        s0 += q;
+        s1 += qy;
+        s2 += qy * dy;
+        if constexpr (ABS) {
+          ax += fabsf(q * fmaf(half_pb, dy, padx));
+          ay += fabsf(q * fmaf(s.pc, dy, hbdx));
         }
       }
       if (touched == 0) continue;
@@ -390,6 +402,37 @@ __device__ __forceinline__ void composite_bwd_tile(const CompositeBwdArgs& a, fl
         if ((lane & 31) == 0)
           unsafeAtomicAdd(a.grad_abs + int64_t(__builtin_amdgcn_readlane(gid, j)) * 2 + (lane >> 5),
                           tabs);
+      }
+    }
+  }
+  if (!any_odd_pixel) return;
+  // Pixels whose gradient is not finite: each entry they took gets that gradient
+  // where it goes by the weight alone (colour), and NaN where an alpha that is
+  // not clamped carries it.  Apart from the walk, which keeps its registers (with the lanes that did not take
+  // an entry masked in it, 10k Gaussians at 640 x 480 took 67 us instead of 64).
+  const float nan = __builtin_nanf("");
+  for (int pos = lo; pos < hi; ++pos) {
+    const int g = int(min(uint32_t(a.ids[start + pos]), a.max_id));
+    const GsRecord rec = RECORDS ? load_record(a.records, g)
+                                 : load_projected(a.pmean, a.pinv, a.pcolor, a.popacity, g);
+    const LaneSplat l = lane_splat(rec);
+    const Splat s = {l.u, l.v, l.o, l.pa, l.pb, l.pc, l.cut, l.r, l.g, l.b};
+    const ColumnTerms c = column_terms(s, pxf);
+#pragma unroll
+    for (int k = 0; k < PIX; ++k) {
+      float raw;
+      if (pos >= ncon[k] || !(entry_alpha<false>(s, c, pyf[k] - s.v, raw) >= kMinAlpha)) continue;
+      const float* grad =
+          a.grad_image + 3 * (view_base + int64_t(pyf[k]) * a.width + int64_t(pxf));
+      if (is_finite(grad[0]) && is_finite(grad[1]) && is_finite(grad[2])) continue;
+      const float carried = raw <= kMaxAlpha ? nan : 0.0f;
+      for (int i = 0; i < 9; ++i) {
+        const float x = i >= 5 && i < 8 ? grad[i - 5] : carried;
+        if (!is_finite(x)) unsafeAtomicAdd(a.grad + int64_t(g) * 9 + i, x);
+      }
+      if constexpr (ABS) {
+        unsafeAtomicAdd(a.grad_abs + int64_t(g) * 2, carried);
+        unsafeAtomicAdd(a.grad_abs + int64_t(g) * 2 + 1, carried);
       }
     }
   }

@@ -42,6 +42,8 @@ __device__ __forceinline__ LaneSplat lane_splat(const GsRecord& r) {
   return s;
 }
 
+__device__ __forceinline__ bool is_finite(float x) { return fabsf(x) < __builtin_huge_valf(); }
+
 // A lane owns one pixel column of its tile (pixel q = lane + 64 k lies in
 // column lane % tile for every tile size up to 64), so the part of the
 // exponent that depends only on dx is computed once per (lane, splat):
