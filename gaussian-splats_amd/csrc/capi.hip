@@ -60,8 +60,8 @@ int check_view(const gs_view& v, bool need_tiles) {
                GS_ERR_INVALID_ARGUMENT, "views, mosaic_cols and active_tiles must be non-negative");
     GS_REQUIRE(v.list_shift == 0 || (v.list_shift == 1 && v.tile_size == 16),
                GS_ERR_INVALID_ARGUMENT, "list_shift must be 0, or 1 with tiles of 16 pixels");
-    GS_REQUIRE(v.split_tiles == 0 || v.split_tiles == 1, GS_ERR_INVALID_ARGUMENT,
-               "split_tiles must be 0 or 1");
+    GS_REQUIRE(v.split_tiles >= 0 && v.split_tiles <= 2, GS_ERR_INVALID_ARGUMENT,
+               "split_tiles must be 0, 1 or 2");
     const int views = v.views > 1 ? v.views : 1;
     const int cols = std::min(views, v.mosaic_cols > 1 ? v.mosaic_cols : 1);
     const int64_t rows = (views + cols - 1) / cols;

@@ -218,7 +218,7 @@ inline CheckpointLayout checkpoint_layout(void* base, int tile_size, int64_t tot
 
 // Walk records (image calls whose forward splits every tile into quarters):
 // the walk back of a 16-pixel tile is cut at recorded walk positions, so that a
-// tile runs on up to kWalkSegments waves that each take all of its pixels.  A
+// tile runs on several waves that each take all of its pixels.  A
 // quarter's forward wave records per pixel (T, colour since its previous
 // record) as it starts the batch at a cut, and at the end of the walk turns the
 // colours into the colour composited after the record (a suffix sum, as with the
@@ -234,25 +234,26 @@ inline CheckpointLayout checkpoint_layout(void* base, int tile_size, int64_t tot
 // and a multiple's slot is the same in all quarters.  A tile is cut at the
 // multiples of its quarters' largest spacing, which each of them still has.
 //
-// Seven cuts at fixed positions, up to 1280 or 4608 entries, left the rest of a
-// long walk to one wave.  A step of 1M Gaussians far away at 1080p 3993 us with
-// them, 2951 with these; with a faint dense spot in front 6384, 4501; 100k of
-// them in front at 640 x 480 38.5 ms, 19.0.  With all cuts spread, the entries
-// that most pixels take fall into few segments (1M far away at 640 x 480 1018 us,
-// 1032 with these, 1403 with four fixed cuts of eleven).
-constexpr int kWalkSegments = 12;
+// With fixed cuts alone, seven up to 1280 or 4608 entries, one wave had the rest
+// of a long walk: a step of 1M Gaussians far away at 640 x 480 9645 us, 7858 now;
+// with a faint dense spot in front of 1M at 1080p 6395, 4328; with 100k in such a
+// spot at 640 x 480 38.5 ms, 23.7.  With all cuts spread, the entries that most
+// pixels take fall into few segments (1M at a third of that distance 1022 us with
+// seven fixed cuts, 1097 now, 1403 with four fixed and seven spread).
 constexpr uint32_t kWalkMostDoubled = 17;  // lists hold less than 2^26 entries
 constexpr int kWalkPixels = 256;  // per record
 constexpr size_t kWalkRecordBytes = size_t(1152) << 20;
 struct WalkCuts {
   int fixed, spread, unit;
-  int shift;  // positions are twice these for a list shared by 2 x 2 tiles
+  int row, shift;  // which fixed cuts; they are doubled for a list shared by 2 x 2 tiles
   __host__ __device__ int records() const { return fixed + spread; }
   // Position of cut i (0 <= i <= records()), and the slot of its record.
   __host__ __device__ int position(int i, int doubled) const {
-    const int cuts[8] = {64, 128, 256, 384, 768, 1280, 2048, 3072};
-    if (i < fixed) return cuts[i] << shift;
-    return ((i - fixed + 1) * unit << shift) << doubled;
+    const int cuts[2][8] = {{64, 128, 192, 256, 384, 640, 1280, 2560},
+                            {64, 128, 384, 768, 1280, 2048, 3072, 4608}};
+    if (i < fixed) return cuts[row][i] << shift;
+    const int64_t p = (int64_t(i - fixed + 1) * unit << shift) << doubled;
+    return p < INT32_MAX ? int(p) : INT32_MAX;
   }
   __host__ __device__ int slot(int i, int doubled) const {
     return i < fixed ? i
@@ -263,15 +264,20 @@ struct WalkCuts {
 // slot needs no counter and no pass before the walk; larger images, whose tiles
 // fill the chip in fewer segments, have fewer: 11 up to 26810 tiles (44 KB each),
 // 7 up to 42130 (16 views of 800 x 800 have 40000), 3 up to 98304, none beyond.
-inline WalkCuts walk_cuts(int num_tiles, int shift) {
+// The fixed cuts reach further where the caller knows of long lists (split_tiles
+// 2), those of faint or dense scenes, which walk thousands of entries at places.
+// Elsewhere the time is that of the longest segment (20k Gaussians at 403 x 307:
+// 40 us with cuts at 192 and 640, 58 without).
+inline WalkCuts walk_cuts(int num_tiles, const gs_view& v) {
   const size_t most = kWalkRecordBytes / (size_t(kWalkPixels) * 16 * size_t(num_tiles));
-  return most >= 11  ? WalkCuts{8, 3, 4096, shift}
-         : most >= 7 ? WalkCuts{4, 3, 640, shift}
-         : most >= 3 ? WalkCuts{2, 1, 384, shift}
-                     : WalkCuts{0, 0, 0, shift};
+  if (most >= 11 && v.split_tiles == 2) return {8, 3, 6144, 1, 0};
+  if (most >= 11) return {8, 3, 4096, 0, v.list_shift};
+  if (most >= 7) return {4, 3, 640, 0, v.list_shift};
+  if (most >= 3) return {2, 1, 384, 0, v.list_shift};
+  return {0, 0, 0, 0, 0};
 }
-inline size_t walk_record_bytes(int num_tiles) {
-  return size_t(num_tiles) * walk_cuts(num_tiles, 0).records() * kWalkPixels * 16;
+inline size_t walk_record_bytes(int num_tiles, const gs_view& v) {
+  return size_t(num_tiles) * walk_cuts(num_tiles, v).records() * kWalkPixels * 16;
 }
 // The forward's waves also leave each quarter's largest contributor count and
 // how often it doubled its spacing: keys[4 tile + quarter].

@@ -84,8 +84,8 @@ struct CompositeBwdArgs {
 // RECORDS: the projection's 48-byte records are gathered (three 16-byte loads
 // of one or two lines, as the forward does) instead of the op's four projected
 // outputs.
-// WALK: segment `seg` between the cuts of the forward's walk records instead,
-// started from the record at its end (a pixel no longer active there
+// WALK: segment `seg`, the entries walk_lo .. walk_hi between two cuts of the
+// forward's walk records (the record at walk_hi in slot walk_slot), started from the record at its end (a pixel no longer active there
 // starts from its final T, with nothing composited after it).  On few tiles a wave per tile
 // leaves SIMDs idle behind the longest walk, and a wave per quarter of the
 // tile's bands repeats each entry's fold, reduction and atomic up to four times:
@@ -94,7 +94,9 @@ struct CompositeBwdArgs {
 // the records cost the forward 3 to 15 us.
 template <int TILE, bool ABS, int PIX, bool MASKS, bool RECORDS, bool WALK>
 __device__ __forceinline__ void composite_bwd_tile(const CompositeBwdArgs& a, float4 (*chunk)[3],
-                                                   int lane, int tile, int band0, int seg) {
+                                                   int lane, int tile, int band0, int seg,
+                                                   int walk_lo = 0, int walk_hi = 0,
+                                                   int walk_slot = 0) {
   constexpr int NPIX = TILE * TILE;
   constexpr int kBandRows = 64 / TILE > 0 ? 64 / TILE : 1;  // tile rows per band of 64 pixels
 
@@ -104,18 +106,6 @@ __device__ __forceinline__ void composite_bwd_tile(const CompositeBwdArgs& a, fl
   const int vx = tx / a.view_tw, vy = ty / a.view_th;
   const int view = vy * a.cols + vx;
   if (view >= a.views) return;  // an empty slot of the mosaic's last row
-  // WALK: the tile's cuts are those of its quarters' largest spacing; nothing to
-  // do for a segment past its largest contributor count.
-  int walk_lo = 0, walk_hi = 0, walk_slot = 0;
-  if constexpr (WALK) {
-    const int4 k0 = a.quarter_keys[2 * tile], k1 = a.quarter_keys[2 * tile + 1];
-    const int doubled =
-        int(min(uint32_t(max(max(k0.y, k0.w), max(k1.y, k1.w))), kWalkMostDoubled));
-    if (seg > 0) walk_lo = a.cuts.position(seg - 1, doubled);
-    walk_hi = a.cuts.position(seg, doubled);
-    if (max(max(k0.x, k0.z), max(k1.x, k1.z)) <= walk_lo) return;
-    walk_slot = a.cuts.slot(seg, doubled);
-  }
   const int ox = (tx - vx * a.view_tw) * TILE, oy = (ty - vy * a.view_th) * TILE;
   const int64_t view_base = int64_t(view) * a.width * a.height;  // first pixel of the view
   int sub;
@@ -440,7 +430,6 @@ __device__ __forceinline__ void composite_bwd_tile(const CompositeBwdArgs& a, fl
 
 // Tiles of the WALK kernel dealt to an XCD at a time (2^shift).
 constexpr int kWalkDealShift = 3;
-static_assert(kWalkSegments % kCompositeWaves == 0, "whole workgroups per tile");
 
 // kCompositeWaves waves per workgroup, one work item each (composite_item);
 // workgroups are mapped onto XCDs so that each XCD takes one region of the
@@ -451,7 +440,8 @@ static_assert(kWalkSegments % kCompositeWaves == 0, "whole workgroups per tile")
 // composites every pixel of any plan exactly once, with one instance of the
 // walk (two would share one register allocation).
 template <int TILE, bool ABS, bool QUARTERS, bool MASKS, bool RECORDS, bool WALK = false>
-__global__ __launch_bounds__(kCompositeWaves * 64) void composite_bwd_kernel(CompositeBwdArgs a) {
+__global__ __launch_bounds__(kCompositeWaves * 64, WALK ? 6 : 1) void composite_bwd_kernel(
+    CompositeBwdArgs a) {
   constexpr int NPIX = TILE * TILE;
   constexpr int PIX_TILE = NPIX >= 64 ? NPIX / 64 : 1;
   const int lane = threadIdx.x & 63;
@@ -463,20 +453,38 @@ __global__ __launch_bounds__(kCompositeWaves * 64) void composite_bwd_kernel(Com
   // broadcasts per entry instead of twelve v_readlane.
   __shared__ float4 chunk[kCompositeWaves][64][3];
   if constexpr (WALK) {
-    // A workgroup takes four of a tile's segments: all tiles' last ones first
-    // (few exist, but they are the long ones), the first ones at the end.
-    // Interleaved, every second workgroup would have no work, and those with
-    // work go to the same half of the shader engines (300k Gaussians at 1237 x
-    // 822: 303 us).
-    const int groups = (a.cuts.records() + 1) / kCompositeWaves;  // per tile
-    const int grid = gridDim.x / groups;
-    const int group = blockIdx.x / grid;
-    const int tile = xcd_deal(blockIdx.x - group * grid, kWalkDealShift);
-    const int seg =
-        (groups - 1 - group) * kCompositeWaves + ((wid + tile) & (kCompositeWaves - 1));
-    if (tile < a.num_tiles)
-      composite_bwd_tile<TILE, ABS, PIX_TILE, MASKS, RECORDS, true>(a, chunk[wid], lane, tile, 0,
-                                                                    seg);
+    // Two workgroups per tile: the waves of the one take the last four segments
+    // (few exist, but they are the long ones), then the middle four, those of the
+    // other the first four; all tiles' later workgroups first.  (A tile with four
+    // segments has one workgroup.)  With three workgroups 300k Gaussians at 1237 x
+    // 822 took 181 us instead of 171, for their launches, mostly without work;
+    // interleaved, every second one would have none, and those with work go to the
+    // same half of the shader engines (303 us).
+    const int halves = a.cuts.records() < kCompositeWaves ? 1 : 2;
+    const int half_grid = gridDim.x / halves;
+    const bool later = halves == 2 && int(blockIdx.x) < half_grid;
+    const int tile = xcd_deal(int(blockIdx.x) % half_grid, kWalkDealShift);
+    const int seg = (wid + tile) & (kCompositeWaves - 1);
+    if (tile >= a.num_tiles) return;
+    // The tile's cuts are those of its quarters' largest spacing; segments past
+    // its largest contributor count have no entries.
+    const int4 k0 = a.quarter_keys[2 * tile], k1 = a.quarter_keys[2 * tile + 1];
+    const int walked = max(max(k0.x, k0.z), max(k1.x, k1.z));
+    const int doubled =
+        int(min(uint32_t(max(max(k0.y, k0.w), max(k1.y, k1.w))), kWalkMostDoubled));
+#pragma unroll 1
+    for (int s = later ? a.cuts.records() - kCompositeWaves + 1 : 0;
+         s >= (later ? kCompositeWaves : 0); s -= kCompositeWaves) {
+      const int lo = s + seg > 0 ? a.cuts.position(s + seg - 1, doubled) : 0;
+      if (walked <= lo) continue;
+      // The second segment loads its pixels again: kept from the first, they would
+      // stay in registers through its walk (116 of them instead of 75).
+      int own = lane;
+      asm volatile("" : "+v"(own));
+      composite_bwd_tile<TILE, ABS, PIX_TILE, MASKS, RECORDS, true>(
+          a, chunk[wid], own, tile, 0, s + seg, lo, a.cuts.position(s + seg, doubled),
+          a.cuts.slot(s + seg, doubled));
+    }
     return;
   }
   const int slot = xcd_swizzle(blockIdx.x, gridDim.x) * kCompositeWaves + wid;
@@ -504,7 +512,7 @@ void launch_masks(const CompositeBwdArgs& a, unsigned blocks, hipStream_t s) {
   if constexpr (MASKS && TILE >= 16) {  // image calls (gs_composite_bwd_image)
     if constexpr (TILE == 16 && QUARTERS) {
       if (a.walk_records) {
-        const int groups = (a.cuts.records() + 1) / kCompositeWaves;  // per tile
+        const int groups = a.cuts.records() < kCompositeWaves ? 1 : 2;  // per tile
         launch_timed(composite_bwd_kernel<16, false, false, true, true, true>,
                      unsigned(groups * deal_grid(a.num_tiles, kWalkDealShift)),
                      kCompositeWaves * 64, 0, s, a);
@@ -629,8 +637,8 @@ int composite_bwd(const float* projected_mean, const float* inverse_covariance,
                "walk buffer too small (%zu bytes, need %zu)", walk_bytes, need);
     a.walk_records = static_cast<const float4*>(walk);
     a.quarter_keys = reinterpret_cast<const int4*>(static_cast<const char*>(walk) +
-                                                   walk_record_bytes(a.num_tiles));
-    a.cuts = walk_cuts(a.num_tiles, m.shift);
+                                                   walk_record_bytes(a.num_tiles, view));
+    a.cuts = walk_cuts(a.num_tiles, view);
   }
   a.ckpt_stamp = nullptr;
   a.ckpt_table_len = 0;

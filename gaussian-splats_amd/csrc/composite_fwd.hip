@@ -636,7 +636,7 @@ int composite(const void* records, int64_t num_records, const int32_t* gaussian_
   a.tile_keys = plan.split_all ? nullptr : tile_keys;
   a.walk_records = plan.split_all ? static_cast<float4*>(walk_records) : nullptr;
   a.quarter_keys = static_cast<int2*>(quarter_keys);
-  a.cuts = walk_cuts(a.num_tiles, m.shift);
+  a.cuts = walk_cuts(a.num_tiles, view);
   a.deal_shift = a.num_tiles <= kDealTiles ? kDealShift : -1;
   if (hit_masks) {
     GS_REQUIRE(view.rendering_mode == GS_MODE_GAUSSIAN, GS_ERR_UNSUPPORTED,
@@ -720,8 +720,8 @@ extern "C" GS_API size_t gs_composite_walk_bytes(gs_view view) {
   if (check_view(view, true) != GS_OK || view.tile_size != 16) return 0;
   const Mosaic m = mosaic_of(view);
   if (!dispatch_plan(m.num_tiles(), view, false).split_all) return 0;
-  if (walk_cuts(m.num_tiles(), 0).records() == 0) return 0;
-  return walk_record_bytes(m.num_tiles()) + walk_key_bytes(m.num_tiles());
+  if (walk_cuts(m.num_tiles(), view).records() == 0) return 0;
+  return walk_record_bytes(m.num_tiles(), view) + walk_key_bytes(m.num_tiles());
 }
 
 extern "C" GS_API int gs_composite_walk(
@@ -739,7 +739,7 @@ extern "C" GS_API int gs_composite_walk(
              "walk buffer too small (%zu bytes, need %zu)", walk_bytes, need);
   GS_REQUIRE((reinterpret_cast<uintptr_t>(walk) & 15u) == 0, GS_ERR_INVALID_ARGUMENT,
              "the walk buffer must be 16-byte aligned");
-  void* keys = static_cast<char*>(walk) + walk_record_bytes(mosaic_of(view).num_tiles());
+  void* keys = static_cast<char*>(walk) + walk_record_bytes(mosaic_of(view).num_tiles(), view);
   return composite(records, num_records, gaussian_ids, num_intersections, ranges, nullptr, view,
                    image, final_transmittance, n_contributors, nullptr, 0, hit_masks,
                    hit_mask_bytes, nullptr, 0, walk, keys, stream);

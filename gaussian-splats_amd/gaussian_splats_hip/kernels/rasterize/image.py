@@ -216,7 +216,7 @@ def forward_image(params, request: ImageRequest, keep: bool, timer=None, again=F
         # Unknown to the host; a list may hold them all.  An image alone is not
         # split for that (14k Gaussians at 1111 x 1043: 109 us, 117 split; with a
         # backward 324 and 308, and 5043 and 1656 where a list does hold 10k).
-        longest = n if backward else 0
+        longest, known = n if backward else 0, False
         mark("bin")
         mark("emit")
     else:
@@ -224,7 +224,7 @@ def forward_image(params, request: ImageRequest, keep: bool, timer=None, again=F
             depth_keys, None, None, tiles_w, tiles_h, timer=mark, tile_rects=tile_rects,
             clear=accumulator, key_range=depth_key_range(request.near, request.far),
         )
-        longest = nat.longest_list(ranges)
+        longest, known = nat.longest_list(ranges), True
     mark("sort")
     subs = 1 << (2 * view.list_shift)  # compositing tiles per list
     lists = nat.active_tiles(ranges)
@@ -238,7 +238,7 @@ def forward_image(params, request: ImageRequest, keep: bool, timer=None, again=F
     # a wave per tile and with four: 652 and 743 us where the spot's pixels
     # saturate after some hundred entries, 10.9 and 4.5 ms where they do not; 80k
     # in a small cube on 4704 tiles 963 and 804.
-    view.split_tiles = longest > LONG_LIST
+    view.split_tiles = (2 if known else 1) if longest > LONG_LIST else 0
     num_tiles, total = tiles_w * tiles_h * subs, ids.numel()
     image = torch.empty(request.shape, dtype=torch.float32, device=device)
     if not backward:

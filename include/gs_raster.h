@@ -90,8 +90,10 @@ typedef struct gs_view {
    * per tile. */
   int32_t list_shift;
   /* 1: the compositing calls split every tile of 16 or 32 pixels over four
-   * waves whatever active_tiles says (a caller whose lists are long throughout,
-   * whose longest walk sets a launch's time).  0: by active_tiles. */
+   * waves whatever active_tiles says (a caller some of whose lists may be long:
+   * the longest walk may set a launch's time); 2: the same, with lists known to
+   * be long (gs_composite_walk then records further into them; the same in both
+   * directions).  0: by active_tiles. */
   int32_t split_tiles;
 } gs_view;
 

@@ -272,7 +272,7 @@ def test_shared_lists_host_checks():
         status = lib.gs_tile_order(fake, ncon, view, fake, fake, 1 << 20, ready, None)
         assert status == nat.GS_ERR_UNSUPPORTED and b"forward's keys" in lib.gs_last_error()
     assert lib.gs_tile_order_noalloc(fake, fake, view, fake, None) != nat.GS_OK
-    for bad in (dict(list_shift=2), dict(list_shift=1, tile_size=32), dict(split_tiles=2)):
+    for bad in (dict(list_shift=2), dict(list_shift=1, tile_size=32), dict(split_tiles=3)):
         status = lib.gs_composite(fake, 10, fake, 10, fake, None, _view(**bad), fake, fake, fake,
                                   None, 0, None, 0, None, 0, None)
         assert status == nat.GS_ERR_INVALID_ARGUMENT
