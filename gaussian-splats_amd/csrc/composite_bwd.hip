@@ -398,8 +398,8 @@ __device__ __forceinline__ void composite_bwd_tile(const CompositeBwdArgs& a, fl
   if (!any_odd_pixel) return;
   // Pixels whose gradient is not finite: each entry they took gets that gradient
   // where it goes by the weight alone (colour), and NaN where an alpha that is
-  // not clamped carries it.  Apart from the walk, which keeps its registers (with the lanes that did not take
-  // an entry masked in it, 10k Gaussians at 640 x 480 took 67 us instead of 64).
+  // not clamped carries it.  Apart from the walk, which keeps its time (masking
+  // the lanes that did not take an entry in it cost 1 to 5%).
   const float nan = __builtin_nanf("");
   for (int pos = lo; pos < hi; ++pos) {
     const int g = int(min(uint32_t(a.ids[start + pos]), a.max_id));
@@ -449,8 +449,8 @@ __global__ __launch_bounds__(kCompositeWaves * 64, WALK ? 6 : 1) void composite_
   // derived from it are scalar too.
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // The wave's current 64 entries, three float4 per entry (u, v, o, pa),
-  // (pb, pc, r, g), (b, oa, ob, oc): written once per lane, then read as LDS
-  // broadcasts per entry instead of twelve v_readlane.
+  // (pb, pc, r, g), (b, pb / 2, 1 / o, -): written once per lane, then read as
+  // LDS broadcasts per entry.
   __shared__ float4 chunk[kCompositeWaves][64][3];
   if constexpr (WALK) {
     // Two workgroups per tile: the waves of the one take the last four segments

@@ -116,7 +116,7 @@ GS_API int gs_camera_rotation(float w, float x, float y, float z, float* rotatio
  * (created beforehand; either may be null) for the calling thread's next
  * timed kernel: the main kernel of gs_project_and_count, gs_project_views,
  * gs_project_bwd, gs_project_bwd_views, gs_composite, gs_composite_bwd, their
- * _image variants, gs_ply_pack or gs_ply_unpack (the first one launched, for calls that
+ * _image variants, gs_composite_walk, gs_ply_pack or gs_ply_unpack (the first one launched, for calls that
  * launch several).
  * That launch carries the events (hipExtLaunchKernel), so they take the
  * kernel's own start and end timestamps; hipEventElapsedTime of the pair is
