@@ -150,7 +150,8 @@ def test_image_long_lists(n, focal, device):
 @pytest.mark.parametrize("size,n", [(48, 4000), (24, 700), (24, 65), (24, 129), (736, 2500)])
 def test_image_walk_segments(size, n, device):
     """Faint Gaussians that each cover the image: every pixel walks the whole
-    list, through every walk bound, and some pixels saturate on the way."""
+    list, through the fixed cuts of its walk records, and some pixels saturate on
+    the way."""
     g = torch.Generator().manual_seed(n)
     scene = scenes.edge_case_scene(n=n, sh_degree=1, image_size=(size, size), seed=3)
     scene.mean[:, :2] = torch.randn(n, 2, generator=g) * 0.3
